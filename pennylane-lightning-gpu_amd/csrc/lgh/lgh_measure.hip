@@ -86,22 +86,23 @@ void launch_reduce(StreamCtx *ctx, const double *partials, int nparts, int nvals
     LGH_LAUNCH_CHECK();
 }
 
-// Reduction workspace layout: [partials (nvals * nparts) | results (nvals)].
+// Reduction workspace: partials (nvals * nparts).
 struct RedBuf {
     double *partials;
-    double *result;
 };
 static RedBuf red_buf(StreamCtx *ctx, int nvals, int nparts, size_t extra_offset = 0) {
-    char *ws = static_cast<char *>(ctx->workspace(extra_offset + sizeof(double) * size_t(nvals) * (nparts + 1) + 256));
+    char *ws = static_cast<char *>(ctx->workspace(extra_offset + sizeof(double) * size_t(nvals) * nparts + 256));
     RedBuf r;
     r.partials = reinterpret_cast<double *>(ws + extra_offset);
-    r.result = r.partials + size_t(nvals) * nparts;
     return r;
 }
 
-static void fetch(StreamCtx *ctx, const double *dev, int nvals, double *out) {
+// Sums each of the nvals rows of partials and returns the values: the
+// reduction writes them into pinned host memory itself, so no copy follows
+// it (a copy of 16 bytes is one more 4 us launch in a chain of three).
+static void reduce_to_host(StreamCtx *ctx, const double *partials, int nparts, int nvals, double *out) {
     double *h = static_cast<double *>(ctx->host_buffer(sizeof(double) * nvals));
-    LGH_HIP(hipMemcpyAsync(h, dev, sizeof(double) * nvals, hipMemcpyDeviceToHost, ctx->stream));
+    launch_reduce(ctx, partials, nparts, nvals, h);
     ctx->sync();
     std::memcpy(out, h, sizeof(double) * nvals);
 }
@@ -461,57 +462,126 @@ __global__ __launch_bounds__(kBlock) void k_csr(const I *__restrict__ indptr, co
 
 // ---------------------------------------------------------------- probabilities
 
-struct WireBits {
-    int k;
-    int b[32]; // state-index bit of wires[j]; output bit j
+// Marginal probabilities.  A wavefront's 64 lanes read the amplitudes of six
+// index bits with the other wires of the output fixed, and add up |a|^2 in
+// registers over the index bits that are summed out; the
+// summed bits among the lanes are added with shuffles at the end, so each
+// output value of the wavefront costs one store and nothing is accumulated
+// in memory.  The summed bits above the lanes are split over `splits`
+// wavefronts where the output alone has too few values to fill the device;
+// up to 16 of them meet in LDS, k_probs_sum adds the rest in a fixed order.
+// Bound by reading the state.  24 qubits, 10 wires, complex128: 118 us as an
+// LDS histogram with one atomic per amplitude (135 us a call), 57 us a call here;
+// 11 wires took 5.3 ms with one thread per output value, 57 us here.
+constexpr int kProbsLoads = 8;         // loads in flight per lane
+constexpr int kProbsBlock = 1024;      // 16 wavefronts, which add their splits before one of them stores
+constexpr int kProbsLogWaves = 4;
+constexpr int kProbsSumBins = 16;      // bins per workgroup of k_probs_sum: 128 consecutive bytes a row
+constexpr int kProbsMaxWaves = 8192;   // 8 wavefronts per SIMD of 256 CUs
+constexpr int kProbsHostBins = 4096;   // results written by the kernel into pinned host memory
+
+// Outputs of at least 128 KiB that are no less than a 128th of the state's
+// length: the lanes hold the lowest index bits (runs of 128 bytes) and those
+// of output bits 0..2 (stores of 64 bytes) instead of index bits 0..5.  The
+// output's low bits are the state's high bits for wires in increasing order,
+// so with lanes on bits 0..5 every 8-byte store has a cache line of its own
+// (26 qubits, the first 20 wires: 1341 against 806 us).  Smaller outputs are
+// bound by the reads, which are faster in runs of 1 KiB (26 qubits complex64,
+// 14 wires: 113 against 193 us).
+constexpr int kProbsWide = 14;
+constexpr int kProbsWideRest = 7;
+
+struct ProbsMap {
+    int lane_bit[6];    // index bit of each lane position
+    int nkeep;          // output wires above the lane bits
+    int keep_bit[32];   // their index bits, ascending
+    int keep_out[32];   // their output bits
+    uint32_t lane_sum;  // lane positions that are summed out
+    int lane_out[6];    // output bit of a kept lane position, -1: none
+    int nsum;           // summed bits above the lanes
+    int log_splits;
+    int sum_bit[64];    // their index bits, ascending
 };
 
-__device__ __forceinline__ uint32_t gather_bits(uint64_t i, const WireBits &wb) {
-    uint32_t o = 0;
-    for (int j = 0; j < wb.k; ++j) o |= uint32_t((i >> wb.b[j]) & 1ull) << j;
-    return o;
-}
-
-// k <= 10 output bins: LDS histogram per workgroup, then a per-bin sum over
-// workgroups.
 template <class R>
-__global__ __launch_bounds__(kBlock) void k_probs_hist(const cx<R> *__restrict__ sv, uint64_t len, uint64_t chunk,
-                                                       WireBits wb, double *__restrict__ partials) {
-    __shared__ double hist[1024];
-    const int nb = 1 << wb.k;
-    for (int t = threadIdx.x; t < nb; t += kBlock) hist[t] = 0.0;
-    __syncthreads();
-    const uint64_t lo = uint64_t(blockIdx.x) * chunk, hi = min(lo + chunk, len);
-    for (uint64_t i = lo + threadIdx.x; i < hi; i += kBlock) {
-        const cx<R> a = sv[i];
-        atomicAdd(&hist[gather_bits(i, wb)], double(a.re) * a.re + double(a.im) * a.im);
+__global__ __launch_bounds__(kProbsBlock) void k_probs(const cx<R> *__restrict__ sv, uint64_t len, uint64_t nwaves,
+                                                       ProbsMap pm, double *__restrict__ out, uint64_t bins) {
+    __shared__ double sh[1 << kProbsLogWaves][64];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint64_t wave = (uint64_t(blockIdx.x) << kProbsLogWaves) + w;
+    const bool live = wave < nwaves;
+    const uint64_t split = wave & ((1ull << pm.log_splits) - 1), kept = live ? wave >> pm.log_splits : 0;
+    uint64_t g = 0, o = 0;
+    for (int j = 0; j < pm.nkeep; ++j) {
+        const uint64_t bit = (kept >> j) & 1ull;
+        g |= bit << pm.keep_bit[j];
+        o |= bit << pm.keep_out[j];
     }
-    __syncthreads();
-    for (int t = threadIdx.x; t < nb; t += kBlock) partials[size_t(t) * gridDim.x + blockIdx.x] = hist[t];
-}
-
-// k > 10: one thread per output bin, sequential sum over the other bits.
-struct Scatter {
-    int nrest;
-    int rest[64]; // state-index bits not in the wire set, ascending
-};
-
-template <class R>
-__global__ __launch_bounds__(kBlock) void k_probs_bins(const cx<R> *__restrict__ sv, WireBits wb, Scatter sc,
-                                                       double *__restrict__ out) {
-    const uint64_t bin = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (bin >= (1ull << wb.k)) return;
-    uint64_t base = 0;
-    for (int j = 0; j < wb.k; ++j) base |= ((bin >> j) & 1ull) << wb.b[j];
-    const uint64_t m = 1ull << sc.nrest;
+    // the split's share: the highest summed bits are fixed to its number
+    const int nloop = pm.nsum - pm.log_splits;
+    uint64_t loop_mask = 0;
+    for (int j = 0; j < nloop; ++j) loop_mask |= 1ull << pm.sum_bit[j];
+    for (int j = 0; j < pm.log_splits; ++j) g |= ((split >> j) & 1ull) << pm.sum_bit[nloop + j];
+    const uint64_t iters = 1ull << nloop;
+    const bool in = uint64_t(lane) < len; // states of fewer than 6 qubits
     double s = 0.0;
-    for (uint64_t c = 0; c < m; ++c) {
-        uint64_t idx = base;
-        for (int q = 0; q < sc.nrest; ++q) idx |= ((c >> q) & 1ull) << sc.rest[q];
-        const cx<R> a = sv[idx];
-        s += double(a.re) * a.re + double(a.im) * a.im;
+    uint64_t c = 0; // the loop's bits at their places in the index
+#pragma unroll
+    for (int b = 0; b < 6; ++b) g |= uint64_t((lane >> b) & 1) << pm.lane_bit[b];
+    const cx<R> *p = sv + g;
+    if (live && iters >= kProbsLoads) {
+        for (uint64_t it = 0; it < iters; it += kProbsLoads) {
+            cx<R> v[kProbsLoads];
+#pragma unroll
+            for (int k = 0; k < kProbsLoads; ++k) {
+                v[k] = ldnt(p + c);
+                c = ((c | ~loop_mask) + 1) & loop_mask;
+            }
+#pragma unroll
+            for (int k = 0; k < kProbsLoads; ++k) s += double(v[k].re) * v[k].re + double(v[k].im) * v[k].im;
+        }
+    } else if (live) {
+        for (uint64_t it = 0; it < iters; ++it) {
+            const cx<R> v = in ? ldnt(p + c) : cx<R>{R(0), R(0)};
+            s += double(v.re) * v.re + double(v.im) * v.im;
+            c = ((c | ~loop_mask) + 1) & loop_mask;
+        }
     }
-    out[bin] = s;
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+        if ((pm.lane_sum >> b) & 1u) s += __shfl_xor(s, 1 << b, 64);
+        else if (pm.lane_out[b] >= 0) o |= uint64_t((lane >> b) & 1) << pm.lane_out[b];
+    }
+    // neighbouring wavefronts hold the splits of one set of output values
+    const int meet = 1 << min(pm.log_splits, kProbsLogWaves);
+    if (meet > 1) {
+        sh[w][lane] = s;
+        __syncthreads();
+        if ((w & (meet - 1)) == 0)
+            for (int q = 1; q < meet; ++q) s += sh[w + q][lane];
+    }
+    if (live && (w & (meet - 1)) == 0 && in && (uint32_t(lane) & pm.lane_sum) == 0)
+        out[(split / unsigned(meet)) * bins + o] = s;
+}
+
+// out[b] = sum over the splits of partials[split][b]
+__global__ __launch_bounds__(kBlock) void k_probs_sum(const double *__restrict__ partials, uint64_t bins, int splits,
+                                                      double *__restrict__ out) {
+    constexpr int kGroups = kBlock / kProbsSumBins; // threads per bin
+    __shared__ double sh[kGroups][kProbsSumBins];
+    const int q = threadIdx.x / kProbsSumBins, j = threadIdx.x % kProbsSumBins;
+    const uint64_t b = uint64_t(blockIdx.x) * kProbsSumBins + j;
+    double s = 0.0;
+    if (b < bins) {
+#pragma unroll 8
+        for (int k = q; k < splits; k += kGroups) s += partials[uint64_t(k) * bins + b];
+    }
+    sh[q][j] = s;
+    __syncthreads();
+    if (q == 0 && b < bins) {
+        for (int k = 1; k < kGroups; ++k) s += sh[k][j];
+        out[b] = s;
+    }
 }
 
 // ---------------------------------------------------------------- sampler
@@ -668,9 +738,8 @@ template <class R> void inner_t(const lgh_sv *a, const lgh_sv *b, double *re, do
     hipLaunchKernelGGL(k_inner<R>, dim3(ch.blocks), dim3(kBlock), 0, ctx->stream, cdata<R>(a), cdata<R>(b),
                        a->length(), ch.chunk, rb.partials);
     LGH_LAUNCH_CHECK();
-    launch_reduce(ctx, rb.partials, ch.blocks, 2, rb.result);
     double out[2];
-    fetch(ctx, rb.result, 2, out);
+    reduce_to_host(ctx, rb.partials, ch.blocks, 2, out);
     *re = out[0];
     *im = out[1];
 }
@@ -705,9 +774,8 @@ template <class R> void expval_t(const lgh_sv *sv, const int32_t *wires, int k, 
         else if (k == 3) run(Offs<3>{}, k_expval_reg<R, 3>);
         else run(Offs<4>{}, k_expval_reg<R, 4>);
         LGH_LAUNCH_CHECK();
-        launch_reduce(ctx, rb.partials, ch.blocks, 2, rb.result);
         double out[2];
-        fetch(ctx, rb.result, 2, out);
+        reduce_to_host(ctx, rb.partials, ch.blocks, 2, out);
         *re = out[0];
         *im = out[1];
         return;
@@ -728,9 +796,8 @@ template <class R> void expval_t(const lgh_sv *sv, const int32_t *wires, int k, 
     hipLaunchKernelGGL(k_expval_lds<R>, dim3(unsigned(ngroups)), dim3(kBlock), lds, ctx->stream, cdata<R>(sv), fx, t,
                        static_cast<const cx<double> *>(dm), rb.partials);
     LGH_LAUNCH_CHECK();
-    launch_reduce(ctx, rb.partials, int(ngroups), 2, rb.result);
     double out[2];
-    fetch(ctx, rb.result, 2, out); // synchronises: m may go out of scope
+    reduce_to_host(ctx, rb.partials, int(ngroups), 2, out); // synchronises: m may go out of scope
     *re = out[0];
     *im = out[1];
 }
@@ -817,7 +884,7 @@ int64_t plan_pauli_tiles(int n, int64_t nwords, const uint64_t *flip, int32_t *p
 struct PauliBufs {
     double *partials; // device, partials_cap doubles
     size_t partials_cap;
-    double *results;  // device, one double per word
+    double *results;  // one double per word: device memory or pinned host memory
 };
 
 // Device doubles of reduction partials the Pauli passes of an n-qubit state need.
@@ -933,14 +1000,16 @@ void pauli_t(const lgh_sv *sv, int64_t nwords, const char *paulis, const int32_t
     for (int64_t w = 0; w < nwords; ++w)
         parse_word(sv->n, paulis, wires, offsets[w], offsets[w + 1], flip[size_t(w)], zy[size_t(w)], ny[size_t(w)]);
     const size_t pcap = pauli_partials_doubles(sv->n, sv->device);
-    char *ws_base = static_cast<char *>(ctx->workspace(sizeof(double) * (pcap + nw) + 256));
-    PauliBufs bufs{reinterpret_cast<double *>(ws_base), pcap, reinterpret_cast<double *>(ws_base) + pcap};
+    double *partials = static_cast<double *>(ctx->workspace(sizeof(double) * pcap));
+    // the reductions write the words' values into pinned host memory
+    double *host = static_cast<double *>(ctx->host_buffer(sizeof(double) * std::max<size_t>(1, nw)));
+    PauliBufs bufs{partials, pcap, host};
     if (nwords > 0)
         pauli_run<R>(sv, nwords, flip.data(), zy.data(), ny.data(), pass_of.data(), pass_mask.data(), done.get(),
                      slot_word.data(), bufs);
-    std::vector<double> out(std::max<size_t>(1, nw)), vals(std::max<size_t>(1, nw));
-    if (nwords > 0) fetch(ctx, bufs.results, int(nwords), out.data());
-    for (size_t q = 0; q < nw; ++q) vals[size_t(slot_word[q])] = out[q];
+    std::vector<double> vals(std::max<size_t>(1, nw));
+    ctx->sync();
+    for (size_t q = 0; q < nw; ++q) vals[size_t(slot_word[q])] = host[q];
     *result = weighted_total(nwords, coeffs, vals.data(), per_word);
 }
 
@@ -1051,9 +1120,8 @@ template <class R> void csr_run(const lgh_csr *csr, const lgh_sv *x, lgh_sv *y, 
         csr_launch<int64_t, R>(csr, cdata<R>(x), nullptr, ctx, rb.partials, blocks);
     else
         csr_launch<int32_t, R>(csr, cdata<R>(x), nullptr, ctx, rb.partials, blocks);
-    launch_reduce(ctx, rb.partials, int(blocks), 2, rb.result);
     double out[2];
-    fetch(ctx, rb.result, 2, out);
+    reduce_to_host(ctx, rb.partials, int(blocks), 2, out);
     *re = out[0];
     *im = out[1];
 }
@@ -1061,33 +1129,65 @@ template <class R> void csr_run(const lgh_csr *csr, const lgh_sv *x, lgh_sv *y, 
 template <class R> void probs_t(const lgh_sv *sv, const int32_t *wires, int k, double *out) {
     StreamCtx *ctx = sv->ctx;
     const int n = sv->n;
-    WireBits wb{};
-    wb.k = k;
-    std::vector<bool> used(size_t(n), false);
-    for (int j = 0; j < k; ++j) {
-        wb.b[j] = n - 1 - wires[j];
-        used[size_t(wb.b[j])] = true;
+    std::vector<int> out_of(size_t(n), -1); // output bit of an index bit
+    for (int j = 0; j < k; ++j) out_of[size_t(n - 1 - wires[j])] = j;
+    ProbsMap pm{};
+    // the lanes' index bits
+    uint64_t lanes = 0;
+    int nl = 0;
+    auto lane = [&](int bit) {
+        if (nl < 6 && bit < n && !((lanes >> bit) & 1)) {
+            lanes |= 1ull << bit;
+            pm.lane_bit[nl++] = bit;
+        }
+    };
+    if (k >= kProbsWide && n - k <= kProbsWideRest) {
+        for (int b = 0; b < (sizeof(R) == 8 ? 3 : 4); ++b) lane(b);
+        for (int j = 0; j < 3; ++j) lane(n - 1 - wires[j]);
     }
-    const int nb = 1 << k;
-    if (k <= 10) {
-        Chunks ch = chunks_for(sv->length(), sv->device, 8);
-        RedBuf rb = red_buf(ctx, nb, ch.blocks);
-        hipLaunchKernelGGL(k_probs_hist<R>, dim3(ch.blocks), dim3(kBlock), 0, ctx->stream, cdata<R>(sv),
-                           sv->length(), ch.chunk, wb, rb.partials);
-        LGH_LAUNCH_CHECK();
-        launch_reduce(ctx, rb.partials, ch.blocks, nb, rb.result);
-        fetch(ctx, rb.result, nb, out);
-        return;
+    for (int b = 0; b < n; ++b) lane(b);
+    for (int b = nl; b < 6; ++b) pm.lane_bit[b] = b; // a state of fewer than 6 qubits: those lanes read nothing
+    for (int b = 0; b < 6; ++b) pm.lane_out[b] = -1;
+    for (int b = 0; b < nl; ++b) {
+        if (out_of[size_t(pm.lane_bit[b])] >= 0)
+            pm.lane_out[b] = out_of[size_t(pm.lane_bit[b])];
+        else
+            pm.lane_sum |= 1u << b;
     }
-    Scatter sc{};
-    for (int b = 0; b < n; ++b)
-        if (!used[size_t(b)]) sc.rest[sc.nrest++] = b;
-    double *dout = static_cast<double *>(ctx->workspace(sizeof(double) * size_t(nb)));
-    hipLaunchKernelGGL(k_probs_bins<R>, dim3(unsigned((nb + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
-                       cdata<R>(sv), wb, sc, dout);
+    for (int b = 0; b < n; ++b) {
+        if ((lanes >> b) & 1) continue;
+        if (out_of[size_t(b)] >= 0) {
+            pm.keep_bit[pm.nkeep] = b;
+            pm.keep_out[pm.nkeep++] = out_of[size_t(b)];
+        } else {
+            pm.sum_bit[pm.nsum++] = b;
+        }
+    }
+    // Splits of the summed bits: enough wavefronts to fill the device, each
+    // with at least kProbsLoads loads (one group in flight).
+    while (pm.log_splits < pm.nsum - 3 && (1ull << (pm.nkeep + pm.log_splits + 1)) <= uint64_t(kProbsMaxWaves))
+        ++pm.log_splits;
+    static_assert(kProbsLoads == 8, "three loop bits per group of loads");
+    const uint64_t nwaves = 1ull << (pm.nkeep + pm.log_splits), bins = 1ull << k;
+    // rows of partial sums that the workgroups leave
+    const int splits = 1 << (pm.log_splits - std::min(pm.log_splits, kProbsLogWaves));
+    const unsigned blocks = unsigned((nwaves + (1u << kProbsLogWaves) - 1) >> kProbsLogWaves);
+    const bool to_host = bins <= uint64_t(kProbsHostBins);
+    double *host = to_host ? static_cast<double *>(ctx->host_buffer(sizeof(double) * bins)) : nullptr;
+    double *ws = static_cast<double *>(ctx->workspace(sizeof(double) * bins * size_t(splits > 1 ? splits + 1 : 1)));
+    double *partials = ws, *result = to_host ? host : splits > 1 ? ws + bins * uint64_t(splits) : ws;
+    hipLaunchKernelGGL(k_probs<R>, dim3(blocks), dim3(kProbsBlock), 0, ctx->stream, cdata<R>(sv), sv->length(), nwaves,
+                       pm, splits > 1 ? partials : result, bins);
     LGH_LAUNCH_CHECK();
-    LGH_HIP(hipMemcpyAsync(out, dout, sizeof(double) * size_t(nb), hipMemcpyDeviceToHost, ctx->stream));
+    if (splits > 1) {
+        const unsigned sblocks = unsigned((bins + kProbsSumBins - 1) / kProbsSumBins);
+        hipLaunchKernelGGL(k_probs_sum, dim3(sblocks), dim3(kBlock), 0, ctx->stream, partials, bins, splits, result);
+        LGH_LAUNCH_CHECK();
+    }
+    if (!to_host)
+        LGH_HIP(hipMemcpyAsync(out, result, sizeof(double) * bins, hipMemcpyDeviceToHost, ctx->stream));
     ctx->sync();
+    if (to_host) std::memcpy(out, host, sizeof(double) * bins);
 }
 
 // Sampler workspace: [cdf (len) | tile sums | total | indices (shots) | sorted
