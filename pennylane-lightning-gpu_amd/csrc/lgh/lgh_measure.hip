@@ -17,8 +17,7 @@
 #include <algorithm>
 #include <cstring>
 #include <map>
-
-#include <rocprim/device/device_radix_sort.hpp>
+#include <type_traits>
 
 #include "lgh_internal.hpp"
 
@@ -614,107 +613,384 @@ template <class R> __device__ __forceinline__ uint64_t fixed_prob(cx<R> a) {
     return uint64_t(__dmul_rn(p, kFixedScale));
 }
 
+// Sampling by inverse CDF.  Shot s draws a threshold t_s below the total mass
+// (fixed point, so that the order of summation does not matter) and takes the
+// first index whose inclusive prefix sum exceeds t_s; the indices are returned
+// in ascending order.  The CDF is formed per tile of 2^11 amplitudes and never
+// written out: the tiles' sums are scanned, every shot finds its tile in them
+// and goes to its bin (up to 8192 bins of consecutive tiles), and one
+// workgroup per bin forms the prefix sums of each tile that got shots in LDS,
+// counts the shots per amplitude and writes them in order.  The counts come
+// out sorted, so nothing is sorted.  The shots are binned with counters in
+// LDS and a scan: one global counter per tile, added to by every shot, took
+// 0.7 ms at 2^13 tiles and 3 ms at 8.
+// Bound by two reads of the state (the second only of tiles that got shots).
+// 24 qubits, 10^6 shots, complex128: 710 us of kernels with a stored CDF,
+// a search of all of it per shot and a radix sort; 185 us here (the copy of the indices to the host, 450 us, not
+// counted).
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kBlock * kScanItems;
+constexpr int kSampleBins = 8192;
+// Shots of one bin handled by one workgroup.  A bin with more (a state with
+// few large amplitudes) is shared by several, which add their counts in
+// global memory and write their parts of its output in a second launch.
+constexpr int kLogBinShots = 12;
+// shots per workgroup of the binning kernels
+constexpr int kAssignBlock = 1024;
+constexpr int kAssignShots = 8 * kAssignBlock;
+
+__device__ __forceinline__ uint64_t wave_incl_scan(uint64_t v, int lane) {
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint64_t u = __shfl_up(v, off, 64);
+        if (lane >= off) v += u;
+    }
+    return v;
+}
+// Exclusive prefix of v over the workgroup's threads (W wavefronts); total:
+// the sum over all of them.
+template <int W> __device__ __forceinline__ uint64_t block_excl_scan(uint64_t v, uint64_t &total) {
+    __shared__ uint64_t sh[W];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const uint64_t incl = wave_incl_scan(v, lane);
+    __syncthreads(); // sh is free again
+    if (lane == 63) sh[w] = incl;
+    __syncthreads();
+    uint64_t before = 0, all = 0;
+#pragma unroll
+    for (int q = 0; q < W; ++q) {
+        if (q < w) before += sh[q];
+        all += sh[q];
+    }
+    total = all;
+    return before + incl - v;
+}
+
+// A call's device arrays, in the workspace.
+struct SampleBufs {
+    uint64_t *tile_off;    // [ntiles] tile sums, then their exclusive prefix
+    uint64_t *total;       // total mass
+    uint32_t *hist;        // [nassign][nbins] shots per bin of a binning workgroup, then their prefix over workgroups
+    uint32_t *bin_off;     // [nbins + 1] first output position of a bin
+    uint2 *heavy;          // [nheavy_max] (bin, part) of shared bins
+    uint32_t *heavy_id;    // [nbins] row of heavy_count
+    uint32_t *heavy_count; // [nrows][tiles of a bin][kScanTile] shots per amplitude of a shared bin
+    uint32_t *nitems;      // parts of shared bins, shared bins
+    uint32_t *where;       // [shots] bin << 16 | rank among the workgroup's shots of that bin
+    uint64_t *thresh;      // [shots] thresholds, by bin
+    uint64_t ntiles, nbins, nassign, shots, seed;
+    uint64_t bin_shots;    // shots per workgroup of a bin: 2^log_bin_shots
+    int log_bin_shots;
+    uint32_t nrows;
+    int log_bin_tiles;     // tiles per bin
+};
 
 template <class R>
-__global__ __launch_bounds__(kBlock) void k_scan_tile_sums(const cx<R> *__restrict__ sv, uint64_t len,
-                                                           uint64_t *__restrict__ tile_sums) {
+__global__ __launch_bounds__(kBlock) void k_sample_sums(const cx<R> *__restrict__ sv, uint64_t len, SampleBufs sb) {
     const uint64_t base = uint64_t(blockIdx.x) * kScanTile;
-    uint64_t s = 0;
+    cx<R> a[kScanItems];
+#pragma unroll
     for (int e = 0; e < kScanItems; ++e) {
         const uint64_t i = base + uint64_t(e) * kBlock + threadIdx.x;
-        if (i < len) s += fixed_prob(sv[i]);
+        a[e] = i < len ? sv[i] : cx<R>{R(0), R(0)};
     }
-    __shared__ uint64_t sh[kBlock];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = kBlock / 2; off > 0; off >>= 1) {
-        if (threadIdx.x < off) sh[threadIdx.x] += sh[threadIdx.x + off];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) tile_sums[blockIdx.x] = sh[0];
-}
-
-// exclusive scan of the tile sums in one workgroup of 1024 threads
-__global__ __launch_bounds__(1024) void k_scan_tile_offsets(uint64_t *__restrict__ tile_sums, uint64_t ntiles,
-                                                            uint64_t *__restrict__ total) {
-    __shared__ uint64_t sh[1024];
-    const uint64_t per = (ntiles + 1023) / 1024;
-    const uint64_t lo = threadIdx.x * per, hi = min(lo + per, ntiles);
-    uint64_t s = 0;
-    for (uint64_t i = lo; i < hi; ++i) s += tile_sums[i];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    // Hillis-Steele inclusive scan over 1024 thread sums
-    for (int off = 1; off < 1024; off <<= 1) {
-        uint64_t v = threadIdx.x >= unsigned(off) ? sh[threadIdx.x - off] : 0;
-        __syncthreads();
-        sh[threadIdx.x] += v;
-        __syncthreads();
-    }
-    uint64_t run = sh[threadIdx.x] - s; // exclusive prefix of this thread's segment
-    for (uint64_t i = lo; i < hi; ++i) {
-        const uint64_t t = tile_sums[i];
-        tile_sums[i] = run;
-        run += t;
-    }
-    if (threadIdx.x == 1023) *total = sh[1023];
-}
-
-template <class R>
-__global__ __launch_bounds__(kBlock) void k_scan_cdf(const cx<R> *__restrict__ sv, uint64_t len,
-                                                     const uint64_t *__restrict__ tile_offsets,
-                                                     uint64_t *__restrict__ cdf) {
-    // each thread owns kScanItems consecutive elements of the tile
-    const uint64_t base = uint64_t(blockIdx.x) * kScanTile + uint64_t(threadIdx.x) * kScanItems;
-    uint64_t q[kScanItems];
-    uint64_t s = 0;
+    uint64_t s = 0, total;
 #pragma unroll
-    for (int e = 0; e < kScanItems; ++e) {
-        const uint64_t i = base + e;
-        q[e] = i < len ? fixed_prob(sv[i]) : 0;
-        s += q[e];
-    }
-    __shared__ uint64_t sh[kBlock];
-    sh[threadIdx.x] = s;
-    __syncthreads();
-    for (int off = 1; off < kBlock; off <<= 1) {
-        uint64_t v = threadIdx.x >= unsigned(off) ? sh[threadIdx.x - off] : 0;
-        __syncthreads();
-        sh[threadIdx.x] += v;
-        __syncthreads();
-    }
-    uint64_t run = tile_offsets[blockIdx.x] + sh[threadIdx.x] - s;
-#pragma unroll
-    for (int e = 0; e < kScanItems; ++e) {
-        const uint64_t i = base + e;
-        run += q[e];
-        if (i < len) cdf[i] = run;
-    }
+    for (int e = 0; e < kScanItems; ++e) s += fixed_prob(a[e]);
+    block_excl_scan<kWaves>(s, total);
+    if (threadIdx.x == 0) sb.tile_off[blockIdx.x] = total;
+    if (blockIdx.x == 0 && threadIdx.x < 2) sb.nitems[threadIdx.x] = 0;
+    const uint64_t nzero = (uint64_t(sb.nrows) << sb.log_bin_tiles) * kScanTile;
+    for (uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x; i < nzero; i += uint64_t(gridDim.x) * kBlock)
+        sb.heavy_count[i] = 0;
 }
 
-__global__ __launch_bounds__(kBlock) void k_sample_search(const uint64_t *__restrict__ cdf, uint64_t len,
-                                                          const uint64_t *__restrict__ total_ptr, uint64_t shots,
-                                                          uint64_t seed, uint64_t *__restrict__ out) {
-    const uint64_t s = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
-    if (s >= shots) return;
-    const uint64_t total = *total_ptr;
+// Exclusive prefix of the tile sums, in place, by one workgroup.
+constexpr int kScanBlock = 1024;
+__global__ __launch_bounds__(kScanBlock) void k_sample_offsets(SampleBufs sb, uint64_t *total_host) {
+    const uint64_t ntiles = sb.ntiles;
+    constexpr int kPer = 8; // consecutive sums per thread
+    uint64_t run = 0;
+    for (uint64_t b = 0; b < ntiles; b += kScanBlock * kPer) {
+        const uint64_t i = b + uint64_t(threadIdx.x) * kPer;
+        uint64_t v[kPer], s = 0, sum;
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            v[e] = i + e < ntiles ? sb.tile_off[i + e] : 0;
+            s += v[e];
+        }
+        uint64_t x = run + block_excl_scan<kScanBlock / 64>(s, sum);
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            if (i + e < ntiles) sb.tile_off[i + e] = x;
+            x += v[e];
+        }
+        run += sum;
+    }
+    if (threadIdx.x == 0) *sb.total = *total_host = run;
+}
+
+// t = floor(u53 * total / 2^53) with a 128-bit product
+__device__ __forceinline__ uint64_t threshold(uint64_t seed, uint64_t shot, uint64_t total) {
     uint32_t r[4];
-    philox(seed, s, r);
+    philox(seed, shot, r);
     const uint64_t u53 = ((uint64_t(r[1]) << 32) | r[0]) >> 11;
-    // t = floor(u53 * total / 2^53) with a 128-bit product
     const uint64_t hi = __umul64hi(u53, total), lo = u53 * total;
-    const uint64_t t = (hi << 11) | (lo >> 53);
-    uint64_t a = 0, b = len - 1;
-    while (a < b) {
-        const uint64_t mid = a + ((b - a) >> 1);
-        if (cdf[mid] > t)
-            b = mid;
-        else
-            a = mid + 1;
+    return (hi << 11) | (lo >> 53);
+}
+
+// The bin of every shot and its rank among the workgroup's shots of the bin.
+// Lanes of one bin add to its counter together (two bins a wavefront, then
+// one by one): a state with few large amplitudes sends a wavefront's shots to
+// few bins.  The ranks depend on timing, the output does not: it only counts
+// the shots of an amplitude.
+__global__ __launch_bounds__(kAssignBlock) void k_sample_assign(SampleBufs sb) {
+    __shared__ uint32_t cnt[kSampleBins];
+    __shared__ uint64_t off[kSampleBins]; // offsets of the bins' first tiles
+    for (unsigned q = threadIdx.x; q < sb.nbins; q += kAssignBlock) {
+        cnt[q] = 0;
+        off[q] = sb.tile_off[uint64_t(q) << sb.log_bin_tiles];
     }
-    out[s] = a;
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const uint64_t total = *sb.total, s0 = uint64_t(blockIdx.x) * kAssignShots;
+    for (int e = 0; e < kAssignShots / kAssignBlock; ++e) {
+        const uint64_t s = s0 + uint64_t(e) * kAssignBlock + threadIdx.x;
+        const bool live = s < sb.shots;
+        uint32_t bin = 0;
+        if (live) {
+            const uint64_t t = threshold(sb.seed, s, total);
+            for (uint32_t step = uint32_t(sb.nbins >> 1); step > 0; step >>= 1) // nbins is a power of two
+                if (off[bin + step] <= t) bin += step; // the last bin whose offset is at most t
+        }
+        uint32_t rank = 0;
+        bool todo = live;
+        for (int round = 0; round < 2; ++round) {
+            const uint64_t open = __ballot(todo);
+            if (!open) break;
+            const int leader = __ffsll((unsigned long long)open) - 1;
+            const uint32_t lb = __shfl(bin, leader, 64);
+            const bool mine = todo && bin == lb;
+            const uint64_t group = __ballot(mine);
+            uint32_t first = 0;
+            if (lane == leader) first = atomicAdd(&cnt[lb], uint32_t(__popcll(group)));
+            first = __shfl(first, leader, 64);
+            if (mine) {
+                rank = first + uint32_t(__popcll(group & ((1ull << lane) - 1ull)));
+                todo = false;
+            }
+        }
+        if (todo) rank = atomicAdd(&cnt[bin], 1u);
+        if (live) sb.where[s] = bin << 16 | rank; // at most kAssignShots shots: 16 bits
+    }
+    __syncthreads();
+    for (unsigned q = threadIdx.x; q < sb.nbins; q += kAssignBlock) sb.hist[blockIdx.x * sb.nbins + q] = cnt[q];
+}
+static_assert(kAssignShots <= 1 << 16 && kSampleBins <= 1 << 16, "bin and rank share a word");
+
+// Per bin: the prefix of its counts over the binning workgroups, in place,
+// and its total (to bin_off, scanned by the next kernel).
+__global__ __launch_bounds__(kBlock) void k_sample_columns(SampleBufs sb) {
+    // a wavefront takes 8 bins (32 consecutive bytes), 8 rows at a time
+    const int lane = threadIdx.x & 63, r = lane >> 3;
+    const uint64_t wave = (uint64_t(blockIdx.x) * kBlock + threadIdx.x) >> 6;
+    const uint64_t bin = wave * 8 + (lane & 7);
+    uint32_t run = 0;
+    for (uint64_t b = 0; b < sb.nassign; b += 8) {
+        const bool in = bin < sb.nbins && b + r < sb.nassign;
+        const uint32_t c = in ? sb.hist[(b + r) * sb.nbins + bin] : 0;
+        uint32_t x = c;
+#pragma unroll
+        for (int off = 8; off < 64; off <<= 1) {
+            const uint32_t u = __shfl_up(x, off, 64);
+            if (lane >= off) x += u;
+        }
+        if (in) sb.hist[(b + r) * sb.nbins + bin] = run + x - c;
+        run += __shfl(x, 56 + (lane & 7), 64);
+    }
+    if (r == 0 && bin < sb.nbins) sb.bin_off[bin] = run;
+}
+
+// Output positions of the bins, by one workgroup, and the parts of shared
+// bins (their order does not matter).
+__global__ __launch_bounds__(kScanBlock) void k_sample_items(SampleBufs sb) {
+    constexpr int kPer = 8; // consecutive bins per thread
+    uint32_t run = 0;
+    for (uint64_t b = 0; b < sb.nbins; b += kScanBlock * kPer) {
+        const uint64_t i = b + uint64_t(threadIdx.x) * kPer;
+        uint32_t c[kPer];
+        uint64_t s = 0, sum;
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            c[e] = i + e < sb.nbins ? sb.bin_off[i + e] : 0;
+            s += c[e];
+        }
+        uint32_t x = run + uint32_t(block_excl_scan<kScanBlock / 64>(s, sum));
+        bool shared = false;
+#pragma unroll
+        for (int e = 0; e < kPer; ++e) {
+            if (i + e < sb.nbins) sb.bin_off[i + e] = x;
+            x += c[e];
+            shared |= c[e] > sb.bin_shots;
+        }
+        run += uint32_t(sum);
+        if (shared) {
+#pragma unroll 1
+            for (int e = 0; e < kPer && i + e < sb.nbins; ++e) {
+                const uint64_t n = (i + e + 1 < sb.nbins && e + 1 < kPer ? sb.bin_off[i + e + 1] : x) - sb.bin_off[i + e];
+                if (n <= sb.bin_shots) continue;
+                const uint32_t parts = uint32_t((n + sb.bin_shots - 1) >> sb.log_bin_shots);
+                const uint32_t at = atomicAdd(&sb.nitems[0], parts);
+                sb.heavy_id[i + e] = atomicAdd(&sb.nitems[1], 1u);
+                for (uint32_t p = 0; p < parts; ++p) sb.heavy[at + p] = make_uint2(uint32_t(i + e), p);
+            }
+        }
+    }
+    if (threadIdx.x == 0) sb.bin_off[sb.nbins] = run;
+}
+
+// Every shot's threshold to its bin.
+__global__ __launch_bounds__(kBlock) void k_sample_scatter(SampleBufs sb) {
+    const uint64_t s = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (s >= sb.shots) return;
+    const uint32_t w = sb.where[s], bin = w >> 16;
+    const uint64_t at = uint64_t(sb.bin_off[bin]) + sb.hist[(s / kAssignShots) * sb.nbins + bin] + (w & 0xffffu);
+    sb.thresh[at] = threshold(sb.seed, s, *sb.total);
+}
+
+// one u64 of padding per 8: a thread's 8 consecutive entries start on banks
+// of their own
+__device__ __forceinline__ int pad8(int i) { return i + (i >> 3); }
+
+// Writes the part of a tile's output that lies in positions [lo, hi): the
+// tile's shots have positions from `at` on, amplitude a's start at at + first[a].
+__device__ __forceinline__ void emit(const uint32_t *first, uint64_t base, uint64_t at, uint64_t count, uint64_t lo,
+                                     uint64_t hi, uint64_t *__restrict__ out) {
+    const uint64_t p0 = max(at, lo), p1 = min(at + count, hi);
+    for (uint64_t p = p0 + threadIdx.x; p < p1; p += kBlock) {
+        const uint32_t r = uint32_t(p - at);
+        int a = 0; // the last amplitude whose first position is at most p
+#pragma unroll
+        for (int step = kScanTile / 2; step > 0; step >>= 1)
+            if (first[a + step] <= r) a += step;
+        out[p] = base + uint64_t(a);
+    }
+}
+
+// Counts per amplitude become the first position of each amplitude's shots;
+// returns the tile's shots.
+__device__ __forceinline__ uint32_t scan_counts(uint32_t *cnt) {
+    uint32_t c[kScanItems];
+    uint64_t s = 0, total;
+#pragma unroll
+    for (int e = 0; e < kScanItems; ++e) {
+        c[e] = cnt[threadIdx.x * kScanItems + e];
+        s += c[e];
+    }
+    uint32_t run = uint32_t(block_excl_scan<kWaves>(s, total));
+#pragma unroll
+    for (int e = 0; e < kScanItems; ++e) {
+        cnt[threadIdx.x * kScanItems + e] = run;
+        run += c[e];
+    }
+    __syncthreads();
+    return uint32_t(total);
+}
+
+// One workgroup per bin, and after those one per part of a shared bin.
+template <class R>
+__global__ __launch_bounds__(kBlock) void k_sample_bins(const cx<R> *__restrict__ sv, uint64_t len, SampleBufs sb,
+                                                        uint64_t *__restrict__ out) {
+    __shared__ uint64_t cdf[kScanTile + kScanTile / 8];
+    __shared__ uint32_t cnt[kScanTile];
+    const bool light = blockIdx.x < sb.nbins;
+    if (!light && blockIdx.x - sb.nbins >= sb.nitems[0]) return;
+    const uint2 it = light ? make_uint2(blockIdx.x, 0u) : sb.heavy[blockIdx.x - sb.nbins];
+    const int tid = threadIdx.x;
+    // the item's shots: positions [lo, hi)
+    const uint64_t bin_lo = sb.bin_off[it.x], bin_hi = sb.bin_off[it.x + 1];
+    if (light && (bin_hi == bin_lo || bin_hi - bin_lo > sb.bin_shots)) return; // no shots, or a shared bin
+    const uint64_t lo = bin_lo + uint64_t(it.y) * sb.bin_shots, hi = min(lo + sb.bin_shots, bin_hi);
+    const uint64_t t0 = uint64_t(it.x) << sb.log_bin_tiles, t1 = min(t0 + (1ull << sb.log_bin_tiles), sb.ntiles);
+    uint64_t at = bin_lo; // output position of the tile
+    for (uint64_t tile = t0; tile < t1; ++tile) {
+        // thresholds of the tile: [off, end); the bin's first and last tiles take what lies beyond as well
+        const uint64_t off = sb.tile_off[tile];
+        const uint64_t end = tile + 1 < sb.ntiles ? sb.tile_off[tile + 1] : *sb.total;
+        const bool first = tile == t0, last = tile + 1 == t1;
+        bool any = first && last;
+        for (uint64_t p = lo + tid; p < hi && !any; p += kBlock) {
+            const uint64_t t = sb.thresh[p];
+            any = (first || t >= off) && (last || t < end);
+        }
+        if (!__syncthreads_or(any)) continue;
+        const uint64_t base = tile * kScanTile;
+#pragma unroll
+        for (int e = 0; e < kScanItems; ++e) {
+            const int j = e * kBlock + tid;
+            const uint64_t i = base + uint64_t(j);
+            cdf[pad8(j)] = i < len ? fixed_prob(sv[i]) : 0;
+            cnt[j] = 0;
+        }
+        __syncthreads();
+        uint64_t q[kScanItems], s = 0, total;
+#pragma unroll
+        for (int e = 0; e < kScanItems; ++e) {
+            q[e] = cdf[pad8(tid * kScanItems + e)];
+            s += q[e];
+        }
+        uint64_t run = block_excl_scan<kWaves>(s, total);
+#pragma unroll
+        for (int e = 0; e < kScanItems; ++e) {
+            run += q[e];
+            cdf[pad8(tid * kScanItems + e)] = run;
+        }
+        __syncthreads();
+        const int top = int(min(uint64_t(kScanTile), len - base)) - 1;
+        for (uint64_t p = lo + tid; p < hi; p += kBlock) {
+            const uint64_t t = sb.thresh[p];
+            if (!((first || t >= off) && (last || t < end))) continue;
+            int a = 0; // the first amplitude whose inclusive prefix exceeds t - off
+#pragma unroll
+            for (int step = kScanTile / 2; step > 0; step >>= 1)
+                if (cdf[pad8(a + step - 1)] <= t - off) a += step;
+            atomicAdd(&cnt[min(a, top)], 1u);
+        }
+        __syncthreads();
+        if (light) {
+            const uint32_t c = scan_counts(cnt);
+            emit(cnt, base, at, c, bin_lo, bin_hi, out);
+            at += c;
+            __syncthreads(); // the next tile clears the counts
+        } else {
+            uint32_t *row = sb.heavy_count +
+                            ((uint64_t(sb.heavy_id[it.x]) << sb.log_bin_tiles) + (tile - t0)) * kScanTile;
+            for (int j = tid; j < kScanTile; j += kBlock)
+                if (cnt[j]) atomicAdd(&row[j], cnt[j]);
+            __syncthreads();
+        }
+    }
+}
+
+// The output of shared bins, once their counts are complete.
+__global__ __launch_bounds__(kBlock) void k_sample_shared(SampleBufs sb, uint64_t *__restrict__ out) {
+    __shared__ uint32_t cnt[kScanTile];
+    if (blockIdx.x >= sb.nitems[0]) return;
+    const uint2 it = sb.heavy[blockIdx.x];
+    const uint64_t bin_lo = sb.bin_off[it.x], bin_hi = sb.bin_off[it.x + 1];
+    const uint64_t lo = bin_lo + uint64_t(it.y) * sb.bin_shots, hi = min(lo + sb.bin_shots, bin_hi);
+    const uint64_t t0 = uint64_t(it.x) << sb.log_bin_tiles, t1 = min(t0 + (1ull << sb.log_bin_tiles), sb.ntiles);
+    uint64_t at = bin_lo;
+    for (uint64_t tile = t0; tile < t1 && at < hi; ++tile) {
+        const uint32_t *row =
+            sb.heavy_count + ((uint64_t(sb.heavy_id[it.x]) << sb.log_bin_tiles) + (tile - t0)) * kScanTile;
+        for (int j = threadIdx.x; j < kScanTile; j += kBlock) cnt[j] = row[j];
+        __syncthreads();
+        const uint32_t c = scan_counts(cnt);
+        emit(cnt, tile * kScanTile, at, c, lo, hi, out);
+        at += c;
+        __syncthreads();
+    }
 }
 
 __global__ __launch_bounds__(kBlock) void k_expand_bits(const uint64_t *__restrict__ idx, uint64_t shots, int n,
@@ -1190,43 +1466,77 @@ template <class R> void probs_t(const lgh_sv *sv, const int32_t *wires, int k, d
     if (to_host) std::memcpy(out, host, sizeof(double) * bins);
 }
 
-// Sampler workspace: [cdf (len) | tile sums | total | indices (shots) | sorted
-// (shots) | radix-sort temporary].  Returns the device pointer of the
-// sorted indices.
+// Returns the device pointer of the sorted indices (in the workspace).
 template <class R> uint64_t *sample_t(const lgh_sv *sv, uint64_t shots, uint64_t seed) {
     StreamCtx *ctx = sv->ctx;
     const uint64_t len = sv->length();
-    const uint64_t ntiles = (len + kScanTile - 1) / kScanTile;
-    size_t temp_bytes = 0;
-    LGH_HIP(rocprim::radix_sort_keys(nullptr, temp_bytes, static_cast<uint64_t *>(nullptr),
-                                     static_cast<uint64_t *>(nullptr), size_t(shots), 0u, unsigned(sv->n),
-                                     ctx->stream));
+    SampleBufs sb{};
+    sb.shots = shots;
+    sb.seed = seed;
+    sb.ntiles = (len + kScanTile - 1) / kScanTile;
+    sb.nbins = std::min<uint64_t>(sb.ntiles, kSampleBins); // powers of two
+    while ((sb.nbins << sb.log_bin_tiles) < sb.ntiles) ++sb.log_bin_tiles;
+    sb.nassign = (shots + kAssignShots - 1) / kAssignShots;
+    // at most 256 shared bins however many the shots
+    sb.log_bin_shots = kLogBinShots;
+    while ((shots >> sb.log_bin_shots) > 256) ++sb.log_bin_shots;
+    sb.bin_shots = 1ull << sb.log_bin_shots;
+    const uint64_t rows = std::min<uint64_t>(sb.nbins, shots / sb.bin_shots); // bins with more shots than that
+    // parts of shared bins: each bin's last one may be short
+    const uint32_t nheavy = rows ? uint32_t(shots / sb.bin_shots + rows) : 0;
+    sb.nrows = uint32_t(rows);
     auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
-    const size_t o_tiles = al(len * 8), o_total = o_tiles + al(ntiles * 8), o_idx = o_total + 256,
-                 o_sorted = o_idx + al(shots * 8), o_temp = o_sorted + al(shots * 8);
-    char *ws = static_cast<char *>(ctx->workspace(o_temp + temp_bytes + 256));
-    uint64_t *cdf = reinterpret_cast<uint64_t *>(ws);
-    uint64_t *tiles = reinterpret_cast<uint64_t *>(ws + o_tiles);
-    uint64_t *total = reinterpret_cast<uint64_t *>(ws + o_total);
-    uint64_t *idx = reinterpret_cast<uint64_t *>(ws + o_idx);
-    uint64_t *sorted = reinterpret_cast<uint64_t *>(ws + o_sorted);
-    hipLaunchKernelGGL(k_scan_tile_sums<R>, dim3(unsigned(ntiles)), dim3(kBlock), 0, ctx->stream, cdata<R>(sv), len,
-                       tiles);
-    hipLaunchKernelGGL(k_scan_tile_offsets, dim3(1), dim3(1024), 0, ctx->stream, tiles, ntiles, total);
-    hipLaunchKernelGGL(k_scan_cdf<R>, dim3(unsigned(ntiles)), dim3(kBlock), 0, ctx->stream, cdata<R>(sv), len, tiles,
-                       cdf);
+    const size_t size[] = {al(sb.ntiles * 8),
+                           256,
+                           al(sb.nassign * sb.nbins * 4),
+                           al((sb.nbins + 1) * 4),
+                           al(nheavy * 8ull),
+                           al(sb.nbins * 4),
+                           al((rows << sb.log_bin_tiles) * kScanTile * 4),
+                           256,
+                           al(shots * 4),
+                           al(shots * 8),
+                           al(shots * 8)};
+    size_t bytes = 0;
+    for (size_t b : size) bytes += b;
+    char *p = static_cast<char *>(ctx->workspace(bytes));
+    int k = 0;
+    auto take = [&](auto *&dst) {
+        dst = reinterpret_cast<std::remove_reference_t<decltype(dst)>>(p);
+        p += size[k++];
+    };
+    uint64_t *out = nullptr;
+    take(sb.tile_off);
+    take(sb.total);
+    take(sb.hist);
+    take(sb.bin_off);
+    take(sb.heavy);
+    take(sb.heavy_id);
+    take(sb.heavy_count);
+    take(sb.nitems);
+    take(sb.where);
+    take(sb.thresh);
+    take(out);
+    uint64_t *total = static_cast<uint64_t *>(ctx->host_buffer(sizeof(uint64_t)));
+    const dim3 block(kBlock);
+    hipStream_t st = ctx->stream;
+    hipLaunchKernelGGL(k_sample_sums<R>, dim3(unsigned(sb.ntiles)), block, 0, st, cdata<R>(sv), len, sb);
+    hipLaunchKernelGGL(k_sample_offsets, dim3(1), dim3(kScanBlock), 0, st, sb, total);
+    hipLaunchKernelGGL(k_sample_assign, dim3(unsigned(sb.nassign)), dim3(kAssignBlock), 0, st, sb);
+    hipLaunchKernelGGL(k_sample_columns, dim3(unsigned((sb.nbins + 31) / 32)), block, 0, st, sb);
+    hipLaunchKernelGGL(k_sample_items, dim3(1), dim3(kScanBlock), 0, st, sb);
+    hipLaunchKernelGGL(k_sample_scatter, dim3(unsigned((shots + kBlock - 1) / kBlock)), block, 0, st, sb);
+    hipLaunchKernelGGL(k_sample_bins<R>, dim3(unsigned(sb.nbins) + nheavy), block, 0, st, cdata<R>(sv), len, sb, out);
+    if (nheavy) hipLaunchKernelGGL(k_sample_shared, dim3(nheavy), block, 0, st, sb, out);
     LGH_LAUNCH_CHECK();
-    // a state with no probability mass cannot be sampled
-    uint64_t htotal = 0;
-    LGH_HIP(hipMemcpyAsync(&htotal, total, 8, hipMemcpyDeviceToHost, ctx->stream));
-    ctx->sync();
-    LGH_REQUIRE(htotal > 0, "cannot sample from a zero state");
-    hipLaunchKernelGGL(k_sample_search, dim3(unsigned((shots + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
-                       cdf, len, total, shots, seed, idx);
-    LGH_LAUNCH_CHECK();
-    LGH_HIP(rocprim::radix_sort_keys(ws + o_temp, temp_bytes, idx, sorted, size_t(shots), 0u, unsigned(sv->n),
-                                     ctx->stream));
-    return sorted;
+    return out;
+}
+
+// Waits for the sampler; a state with no probability mass cannot be sampled
+// (the indices formed for it are not returned).
+void wait_sampled(const lgh_sv *sv) {
+    sv->ctx->sync();
+    LGH_REQUIRE(*static_cast<const uint64_t *>(sv->ctx->host) > 0, "cannot sample from a zero state");
 }
 
 template <class F> void by_dtype(const lgh_sv *sv, F &&f) {
@@ -1501,6 +1811,7 @@ lgh_status lgh_sample(const lgh_sv *sv, uint64_t shots, uint64_t seed, uint64_t 
         DeviceGuard g(sv->device);
         uint64_t *d = nullptr;
         by_dtype(sv, [&](auto r) { d = sample_t<decltype(r)>(sv, shots, seed); });
+        wait_sampled(sv);
         LGH_HIP(hipMemcpyAsync(indices, d, 8 * shots, hipMemcpyDeviceToHost, sv->ctx->stream));
         sv->ctx->sync();
     });
@@ -1514,6 +1825,7 @@ lgh_status lgh_sample_bits(const lgh_sv *sv, uint64_t shots, uint64_t seed, uint
         DeviceGuard g(sv->device);
         uint64_t *d = nullptr;
         by_dtype(sv, [&](auto r) { d = sample_t<decltype(r)>(sv, shots, seed); });
+        wait_sampled(sv);
         const uint64_t total = shots * uint64_t(sv->n);
         // the expanded bits go to a separate buffer (the workspace holds the indices)
         uint64_t *dbits = static_cast<uint64_t *>(pool_alloc(sv->device, 8 * total));

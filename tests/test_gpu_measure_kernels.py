@@ -41,3 +41,39 @@ def test_probs_edges(n, dtype):
             # sums of up to 2^n rounded positive terms: relative error below 2^n eps
             np.testing.assert_allclose(s.probs(wires), np_probs(psi, n, wires), rtol=max(1e-14, 2.0 ** n * 2.3e-16),
                                        atol=0, err_msg=f"n={n} wires={wires}")
+
+
+def concentrated(n, seed):
+    """Few large amplitudes: a tile (2^11 amplitudes) that takes most shots, one amplitude that takes a third of
+    them, zero tiles at both ends where there is room."""
+    psi = rand_state(n, seed)
+    psi[(1 << n) // 3] = 0.8
+    if n >= 13:
+        psi[:2048] = psi[-2048:] = 0
+        psi[2048 * 2:2048 * 3] *= 10
+    return psi / np.linalg.norm(psi)
+
+
+@pytest.mark.parametrize("n", [1, 6, 10, 11, 12, 15, 17])
+@pytest.mark.parametrize("shots", [1, 63, 4096, 4097, 30000])
+def test_sampler_tiles_bit_exact(n, shots):
+    """Spread and concentrated states (a tile of more than 4096 shots is shared by several workgroups), a basis
+    state, and an unnormalised state, against the oracle's inverse CDF; samples are whole numbers and stay equal."""
+    from oracle import pyoracle as po
+
+    basis = np.zeros(1 << n, dtype=np.complex128)
+    basis[(1 << n) * 2 // 3] = 1
+    for k, psi in enumerate((rand_state(n, n), concentrated(n, n + 1), basis, 0.3 * rand_state(n, n + 2))):
+        for dtype in (np.complex128, np.complex64):
+            p = psi.astype(dtype)
+            got = N.State(n, dtype).upload(p).sample(shots, 77 + k)
+            np.testing.assert_array_equal(got, po.sample(n, p, shots, 77 + k), err_msg=f"state {k} {dtype}")
+
+
+def test_sampling_a_zero_state_is_an_error():
+    s = N.State(12)
+    s.upload(np.zeros(1 << 12, dtype=np.complex128))
+    with pytest.raises(N.LghError, match="zero state"):
+        s.sample(100, 1)
+    with pytest.raises(N.LghError, match="zero state"):
+        s.sample_bits(100, 1)
