@@ -365,7 +365,7 @@ template <int K> struct Offs {
     uint64_t o[1 << K];
 };
 
-// K-target dense gate (2 <= K <= 4) with the matrix staged in LDS and the
+// K-target dense gate (K = 2, 3; 4 in complex64) with the matrix staged in LDS and the
 // 2^K amplitudes of a group held in registers.
 template <class R, int K>
 __global__ __launch_bounds__(kBlock) void k_denseK(cx<R> *__restrict__ sv, uint64_t ngroups, Fixed fx,
@@ -386,37 +386,6 @@ __global__ __launch_bounds__(kBlock) void k_denseK(cx<R> *__restrict__ sv, uint6
 #pragma unroll
         for (int c = 0; c < D; ++c) acc = cfma(sm[r * D + c], v[c], acc);
         stnt(sv + (base | offs.o[r]), acc);
-    }
-}
-
-// Large dense gates (5 <= K <= 13): one workgroup per group; the 2^K
-// amplitudes are staged in LDS and the transposed matrix is streamed from
-// global memory (coalesced across rows).
-struct Tbits {
-    int k;
-    int b[kMaxLdsK];
-};
-
-__device__ __forceinline__ uint64_t deposit(uint32_t m, const Tbits &tb) {
-    uint64_t o = 0;
-    for (int j = 0; j < tb.k; ++j)
-        if ((m >> (tb.k - 1 - j)) & 1u) o |= 1ull << tb.b[j];
-    return o;
-}
-
-template <class R>
-__global__ __launch_bounds__(kBlock) void k_denseLDS(cx<R> *__restrict__ sv, Fixed fx, uint64_t cmask, Tbits tb,
-                                                     const cx<R> *__restrict__ matT) {
-    extern __shared__ unsigned char lds_raw[];
-    cx<R> *x = reinterpret_cast<cx<R> *>(lds_raw);
-    const uint32_t D = 1u << tb.k;
-    const uint64_t base = expand(blockIdx.x, fx) | cmask;
-    for (uint32_t m = threadIdx.x; m < D; m += kBlock) x[m] = sv[base | deposit(m, tb)];
-    __syncthreads();
-    for (uint32_t r = threadIdx.x; r < D; r += kBlock) {
-        cx<R> acc{R(0), R(0)};
-        for (uint32_t c = 0; c < D; ++c) acc = cfma(matT[uint64_t(c) * D + r], x[c], acc);
-        sv[base | deposit(r, tb)] = acc;
     }
 }
 
@@ -468,7 +437,10 @@ template <class R> void launch_kop_t(lgh_sv *sv, const KOp &op) {
         LGH_LAUNCH_CHECK();
         return;
     }
-    if (op.k <= kMaxRegK) {
+    // Four targets: complex64 in registers, in single precision throughout (24
+    // qubits 71 us, 86 us as a product in double precision); complex128 as a
+    // product (102 against 115 us, low wires 102 against 834 us).
+    if (op.k <= kMaxRegK || (op.k == 4 && sizeof(R) == 4)) {
         std::vector<cx<R>> m(size_t(D) * D);
         for (size_t i = 0; i < m.size(); ++i) m[i] = to_cx<R>(op.mat[i]);
         const cx<R> *dm = static_cast<const cx<R> *>(ctx->upload(m.data(), m.size() * sizeof(cx<R>)));
@@ -491,7 +463,7 @@ template <class R> void launch_kop_t(lgh_sv *sv, const KOp &op) {
             fill(offs, 3);
             hipLaunchKernelGGL((k_denseK<R, 3>), dim3(unsigned(blocks)), dim3(kBlock), 0, st, data, ngroups, fx,
                                op.cmask, offs, dm);
-        } else {
+        } else if constexpr (sizeof(R) == 4) {
             Offs<4> offs;
             fill(offs, 4);
             hipLaunchKernelGGL((k_denseK<R, 4>), dim3(unsigned(blocks)), dim3(kBlock), 0, st, data, ngroups, fx,
@@ -500,27 +472,7 @@ template <class R> void launch_kop_t(lgh_sv *sv, const KOp &op) {
         LGH_LAUNCH_CHECK();
         return;
     }
-    // 5..13 targets: transposed matrix for coalesced row streaming
-    std::vector<cx<R>> mt(size_t(D) * D);
-    for (int r = 0; r < D; ++r)
-        for (int c = 0; c < D; ++c) mt[size_t(c) * D + r] = to_cx<R>(op.mat[size_t(r) * D + c]);
-    const size_t mbytes = mt.size() * sizeof(cx<R>);
-    void *dm;
-    if (mbytes <= (1u << 20)) {
-        dm = ctx->upload(mt.data(), mbytes);
-    } else {
-        dm = ctx->workspace(mbytes);
-        LGH_HIP(hipMemcpyAsync(dm, mt.data(), mbytes, hipMemcpyHostToDevice, st));
-        ctx->sync(); // mt is a host temporary
-    }
-    Tbits tb{};
-    tb.k = op.k;
-    for (int j = 0; j < op.k; ++j) tb.b[j] = op.tbits[j];
-    const size_t lds = size_t(D) * sizeof(cx<R>);
-    LGH_REQUIRE(lds <= 160 * 1024, "matrix gate too large for one workgroup");
-    hipLaunchKernelGGL((k_denseLDS<R>), dim3(unsigned(ngroups)), dim3(kBlock), lds, st, data, fx, op.cmask, tb,
-                       static_cast<const cx<R> *>(dm));
-    LGH_LAUNCH_CHECK();
+    dense_apply(sv, op);
 }
 
 } // namespace

@@ -205,8 +205,8 @@ template <int L, class R> __device__ __forceinline__ void row_swap_cx(cx<R> &x, 
 }
 
 constexpr int kMaxFixed = 16; // target + control bits that a kernel enumerates around
-constexpr int kMaxRegK = 4;   // dense gates held in registers up to 4 targets
-constexpr int kMaxLdsK = 13;  // dense gates staged through LDS up to 13 targets
+constexpr int kMaxRegK = 3;   // dense gates held in registers up to 3 targets
+constexpr int kMaxLdsK = 13;  // dense gates as matrix products up to 13 targets
 
 // Bit positions (ascending) where a zero is inserted into a group index.
 struct Fixed {
@@ -365,6 +365,11 @@ std::vector<std::complex<double>> full_matrix(const lgh_op &op, bool dagger);
 
 // Launch a compiled op on one state.
 void launch_kop(lgh_sv *sv, const KOp &op);
+
+// Dense matrices on kMaxRegK + 1 to kMaxLdsK target bits (lgh_dense.hip): application,
+// and <psi|M|psi> as (re, im) for a row-major matrix of interleaved doubles.
+void dense_apply(lgh_sv *sv, const KOp &op);
+void dense_expval(const lgh_sv *sv, const int *tbits, int k, const double *matrix, double *re_im);
 
 // Device-side reduction helpers (implemented in lgh_measure.hip).
 // Sums `count` partial values (stride 1) into out_dev[0] with a fixed order.

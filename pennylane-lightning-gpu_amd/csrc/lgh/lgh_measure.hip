@@ -89,11 +89,8 @@ void launch_reduce(StreamCtx *ctx, const double *partials, int nparts, int nvals
 struct RedBuf {
     double *partials;
 };
-static RedBuf red_buf(StreamCtx *ctx, int nvals, int nparts, size_t extra_offset = 0) {
-    char *ws = static_cast<char *>(ctx->workspace(extra_offset + sizeof(double) * size_t(nvals) * nparts + 256));
-    RedBuf r;
-    r.partials = reinterpret_cast<double *>(ws + extra_offset);
-    return r;
+static RedBuf red_buf(StreamCtx *ctx, int nvals, int nparts) {
+    return {static_cast<double *>(ctx->workspace(sizeof(double) * size_t(nvals) * nparts))};
 }
 
 // Sums each of the nvals rows of partials and returns the values: the
@@ -194,46 +191,6 @@ __global__ __launch_bounds__(kBlock) void k_expval_reg(const cx<R> *__restrict__
             acc[0] += v[r].re * y.re + v[r].im * y.im;
             acc[1] += v[r].re * y.im - v[r].im * y.re;
         }
-    }
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        partials[blockIdx.x] = acc[0];
-        partials[gridDim.x + blockIdx.x] = acc[1];
-    }
-}
-
-struct Tbits {
-    int k;
-    int b[kMaxLdsK];
-};
-__device__ __forceinline__ uint64_t deposit(uint32_t m, const Tbits &tb) {
-    uint64_t o = 0;
-    for (int j = 0; j < tb.k; ++j)
-        if ((m >> (tb.k - 1 - j)) & 1u) o |= 1ull << tb.b[j];
-    return o;
-}
-
-// 5..13 targets: one workgroup per group, amplitudes in LDS, transposed
-// matrix streamed from global memory.
-template <class R>
-__global__ __launch_bounds__(kBlock) void k_expval_lds(const cx<R> *__restrict__ sv, Fixed fx, Tbits tb,
-                                                       const cx<double> *__restrict__ matT,
-                                                       double *__restrict__ partials) {
-    extern __shared__ unsigned char lds_raw[];
-    cx<double> *x = reinterpret_cast<cx<double> *>(lds_raw);
-    const uint32_t D = 1u << tb.k;
-    const uint64_t base = expand(blockIdx.x, fx);
-    for (uint32_t m = threadIdx.x; m < D; m += kBlock) {
-        cx<R> t = sv[base | deposit(m, tb)];
-        x[m] = cx<double>{double(t.re), double(t.im)};
-    }
-    __syncthreads();
-    double acc[2] = {0.0, 0.0};
-    for (uint32_t r = threadIdx.x; r < D; r += kBlock) {
-        cx<double> y{0.0, 0.0};
-        for (uint32_t c = 0; c < D; ++c) y = cfma(matT[uint64_t(c) * D + r], x[c], y);
-        acc[0] += x[r].re * y.re + x[r].im * y.im;
-        acc[1] += x[r].re * y.im - x[r].im * y.re;
     }
     block_sum<2>(acc);
     if (threadIdx.x == 0) {
@@ -1027,10 +984,10 @@ template <class R> void expval_t(const lgh_sv *sv, const int32_t *wires, int k, 
     const int D = 1 << k;
     std::vector<int> tb(k);
     for (int j = 0; j < k; ++j) tb[j] = n - 1 - wires[j];
-    Fixed fx = make_fixed(tb);
-    const uint64_t ngroups = 1ull << (n - k);
-    std::vector<cx<double>> m(size_t(D) * D);
     if (k <= kMaxRegK) {
+        const Fixed fx = make_fixed(tb);
+        const uint64_t ngroups = 1ull << (n - k);
+        std::vector<cx<double>> m(size_t(D) * D);
         for (size_t i = 0; i < m.size(); ++i) m[i] = cx<double>{matrix[2 * i], matrix[2 * i + 1]};
         const cx<double> *dm = static_cast<const cx<double> *>(ctx->upload(m.data(), m.size() * sizeof(m[0])));
         Chunks ch = chunks_for(ngroups, sv->device, 2);
@@ -1047,8 +1004,7 @@ template <class R> void expval_t(const lgh_sv *sv, const int32_t *wires, int k, 
         };
         if (k == 1) run(Offs<1>{}, k_expval_reg<R, 1>);
         else if (k == 2) run(Offs<2>{}, k_expval_reg<R, 2>);
-        else if (k == 3) run(Offs<3>{}, k_expval_reg<R, 3>);
-        else run(Offs<4>{}, k_expval_reg<R, 4>);
+        else run(Offs<3>{}, k_expval_reg<R, 3>);
         LGH_LAUNCH_CHECK();
         double out[2];
         reduce_to_host(ctx, rb.partials, ch.blocks, 2, out);
@@ -1056,24 +1012,8 @@ template <class R> void expval_t(const lgh_sv *sv, const int32_t *wires, int k, 
         *im = out[1];
         return;
     }
-    for (int r = 0; r < D; ++r)
-        for (int c = 0; c < D; ++c)
-            m[size_t(c) * D + r] = cx<double>{matrix[2 * (size_t(r) * D + c)], matrix[2 * (size_t(r) * D + c) + 1]};
-    const size_t mbytes = m.size() * sizeof(m[0]);
-    const size_t moff = (mbytes + 255) & ~size_t(255);
-    RedBuf rb = red_buf(ctx, 2, int(ngroups), moff);
-    void *dm = ctx->workspace(moff); // matrix at the start of the workspace
-    LGH_HIP(hipMemcpyAsync(dm, m.data(), mbytes, hipMemcpyHostToDevice, ctx->stream));
-    Tbits t{};
-    t.k = k;
-    for (int j = 0; j < k; ++j) t.b[j] = tb[j];
-    const size_t lds = size_t(D) * sizeof(cx<double>);
-    LGH_REQUIRE(lds <= 160 * 1024, "observable matrix too large");
-    hipLaunchKernelGGL(k_expval_lds<R>, dim3(unsigned(ngroups)), dim3(kBlock), lds, ctx->stream, cdata<R>(sv), fx, t,
-                       static_cast<const cx<double> *>(dm), rb.partials);
-    LGH_LAUNCH_CHECK();
     double out[2];
-    reduce_to_host(ctx, rb.partials, int(ngroups), 2, out); // synchronises: m may go out of scope
+    dense_expval(sv, tb.data(), k, matrix, out);
     *re = out[0];
     *im = out[1];
 }

@@ -77,3 +77,53 @@ def test_sampling_a_zero_state_is_an_error():
         s.sample(100, 1)
     with pytest.raises(N.LghError, match="zero state"):
         s.sample_bits(100, 1)
+
+
+def np_matrix(psi, n, wires, m, ctrl=()):
+    """m on `wires` (first: most significant) where the control wires are 1."""
+    k = len(wires)
+    rest = [w for w in range(n) if w not in wires and w not in ctrl]
+    order = list(ctrl) + list(wires) + rest
+    t = np.ascontiguousarray(psi.astype(np.complex128).reshape([2] * n).transpose(order)).reshape(1 << len(ctrl),
+                                                                                               1 << k, -1)
+    t[-1] = m @ t[-1]
+    return t.reshape([2] * n).transpose(np.argsort(order)).reshape(-1)
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("n,k", [(4, 4), (5, 4), (9, 4), (13, 4), (5, 5), (6, 5), (9, 5), (13, 5), (6, 6), (11, 6), (14, 6), (7, 7), (12, 7), (15, 7),
+                                 (9, 8), (14, 8), (10, 10), (16, 10)])
+def test_dense_matrices_on_many_wires(n, k, dtype):
+    """Matrix gates and expectations on four and more wires: one group, fewer groups than a tile's columns, tiles
+    and remainders; the lowest wires, the highest, scattered ones in a scrambled order; controls; the adjoint.
+    Products of 2^k terms of unitary rows: error below 2^(k/2 + 2) eps of the amplitudes' scale."""
+    rng = np.random.default_rng(100 * n + k)
+    psi = rand_state(n, n + k, dtype)
+    D = 1 << k
+    u, _ = np.linalg.qr(rng.normal(size=(D, D)) + 1j * rng.normal(size=(D, D)))
+    eps = np.finfo(np.float64 if dtype == np.complex128 else np.float32).eps
+    tol = 4 * np.sqrt(D) * eps
+    for wires in (list(range(k)), list(range(n - k, n)), [int(x) for x in rng.permutation(n)[:k]]):
+        s = N.State(n, dtype).upload(psi)
+        # not Hermitian: both parts of the value; evaluated in double for complex64 states as well
+        ev = s.expval_matrix(wires, u)
+        assert abs(ev - np.vdot(psi.astype(np.complex128), np_matrix(psi, n, wires, u))) < 4 * np.sqrt(D) * 2.3e-16
+        s.apply([("QubitUnitary", wires, [], False, u)])
+        np.testing.assert_allclose(s.download(), np_matrix(psi, n, wires, u), atol=tol, rtol=0)
+        s.apply([("QubitUnitary", wires, [], True, u)])
+        np.testing.assert_allclose(s.download(), psi, atol=2 * tol, rtol=0)
+
+
+@pytest.mark.parametrize("n,k,ctrl", [(5, 4, 1), (12, 4, 3), (7, 5, 1), (12, 5, 2), (13, 6, 1), (12, 7, 2), (16, 7, 1)])
+def test_controlled_dense_matrices_on_many_wires(n, k, ctrl):
+    rng = np.random.default_rng(n + k)
+    psi = rand_state(n, n + k)
+    D = 1 << k
+    u, _ = np.linalg.qr(rng.normal(size=(D, D)) + 1j * rng.normal(size=(D, D)))
+    w = [int(x) for x in rng.permutation(n)[:k + ctrl]]
+    arr, keep = N.make_ops([("QubitUnitary", w, [], False, u)])
+    arr[0].num_ctrl = ctrl
+    s = N.State(n).upload(psi)
+    N.check(N.lib().lgh_apply(s.handle, arr, 1))
+    np.testing.assert_allclose(s.download(), np_matrix(psi, n, w[ctrl:], u, w[:ctrl]),
+                               atol=4 * np.sqrt(D) * 2.3e-16, rtol=0)
