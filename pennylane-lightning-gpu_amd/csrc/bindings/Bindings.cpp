@@ -162,6 +162,26 @@ template <class PrecisionT, class ParamT> void bind_precision(py::module_ &m) {
             },
             ("Apply the " + name + " gate.").c_str());
     }
+    // A circuit at once: named gates, and explicit matrices where `matrices`
+    // has one, in fused passes.  Complex128 only: gates applied together in
+    // another order of operations round differently, which complex64 results
+    // would show at 1e-7.
+    if constexpr (std::is_same_v<PrecisionT, double>)
+        sv_cls.def(
+            "applySequence",
+            [](SV &sv, const std::vector<std::string> &names, const std::vector<std::vector<std::size_t>> &wires,
+               const std::vector<bool> &inverses, const std::vector<std::vector<PrecisionT>> &params,
+               const std::vector<np_arr_c> &matrices) {
+                std::vector<std::vector<CT>> mats;
+                mats.reserve(matrices.size());
+                for (const auto &m : matrices) {
+                    auto v = to_vec<ParamT>(m);
+                    mats.emplace_back(v.begin(), v.end());
+                }
+                py::gil_scoped_release release;
+                sv.applySequence(names, wires, inverses, params, mats);
+            },
+            "Apply a sequence of gates in order.");
     sv_cls
         .def("apply",
              py::overload_cast<const std::vector<std::string> &, const std::vector<std::vector<std::size_t>> &,

@@ -297,6 +297,21 @@ template <class PrecisionT> class StateVectorHIPManaged {
         }
         if (b.size()) check(lgh_apply(sv_, b.data(), static_cast<int64_t>(b.size())));
     }
+    // A sequence of named gates and explicit matrices (where matrices[i] is
+    // not empty), applied together.
+    void applySequence(const std::vector<std::string> &opNames, const std::vector<std::vector<std::size_t>> &wires,
+                       const std::vector<bool> &adjoints, const std::vector<std::vector<PrecisionT>> &params,
+                       const std::vector<std::vector<ComplexT>> &matrices) {
+        PL_HIP_ABORT_IF(opNames.size() != wires.size() || opNames.size() != adjoints.size() ||
+                            opNames.size() != params.size() || opNames.size() != matrices.size(),
+                        "Incompatible number of ops, wires, adjoints, parameters and matrices");
+        OpBuilder b;
+        for (std::size_t i = 0; i < opNames.size(); ++i) {
+            PL_HIP_ABORT_IF(isStatePrep(opNames[i]), "State preparation is not a gate: " + opNames[i]);
+            if (opNames[i] != "Identity") b.add<PrecisionT>(opNames[i], wires[i], adjoints[i], params[i], matrices[i]);
+        }
+        if (b.size()) check(lgh_apply(sv_, b.data(), static_cast<int64_t>(b.size())));
+    }
     void applyOperation(const std::vector<std::string> &opNames, const std::vector<std::vector<std::size_t>> &wires,
                         const std::vector<bool> &adjoints) {
         applyOperation(opNames, wires, adjoints, std::vector<std::vector<PrecisionT>>(opNames.size()));

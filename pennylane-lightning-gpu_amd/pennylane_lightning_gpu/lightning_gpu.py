@@ -42,6 +42,10 @@ from . import _serialize as ser
 _name_map = {"PauliX": "X", "PauliY": "Y", "PauliZ": "Z", "Identity": "I"}
 _STATE_PREP = ("StatePrep", "QubitStateVector")
 _PREP_ALL = _STATE_PREP + ("BasisState",)
+_NO_MATRIX = np.zeros(0, dtype=np.complex128)
+# gates handed to the backend at once: bounds the time its scheduler takes for
+# a circuit that it has not seen (milliseconds per thousand gates)
+_SEQUENCE_MAX = 2048
 _SHOTS_WARNING = ("Requested adjoint differentiation to be computed with finite shots. The derivative is always "
                   "exact when using the adjoint differentiation method.")
 
@@ -164,7 +168,10 @@ class LightningGPU:
 
     # --- operations ----------------------------------------------------------------
     def apply_cq(self, operations, **kwargs):
-        """lightning_gpu.py:519-555."""
+        """lightning_gpu.py:519-555.  A backend state that takes a sequence of
+        gates gets them together and applies them in fused passes."""
+        sequence = getattr(self._gpu_state, "applySequence", None)
+        pending = []
         for o in operations:
             if o.name == "Identity":
                 continue
@@ -172,13 +179,26 @@ class LightningGPU:
             name = o.base.name if invert else o.name
             method = getattr(self._gpu_state, name, None)
             wires = self.map_wires(o.wires)
+            mat, params = _NO_MATRIX, []
             if method is None:
+                invert = False
                 mat = np.asarray(o.matrix(), dtype=self.C_DTYPE)  # already holds the adjoint
                 if mat.size == 0:
                     raise DeviceError("Unsupported operation")
-                self._gpu_state.apply(name, wires, False, [], mat.ravel(order="C"))
+                mat = mat.ravel(order="C")
+            elif o.parameters:
+                params = [float(p) for p in np.ravel(o.parameters)]
+            if sequence is not None:
+                pending.append((name, wires, invert, params, mat))
+                if len(pending) == _SEQUENCE_MAX:
+                    sequence(*zip(*pending))
+                    pending = []
+            elif method is None:
+                self._gpu_state.apply(name, wires, False, [], mat)
             else:
-                method(wires, invert, [float(p) for p in np.ravel(o.parameters)] if o.parameters else [])
+                method(wires, invert, params)
+        if pending:
+            sequence(*zip(*pending))
 
     def apply(self, operations, **kwargs):
         """lightning_gpu.py:557-575."""
