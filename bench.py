@@ -233,7 +233,7 @@ def bench_measurements(N, args):
     words, wires, coeffs = random_pauli_hamiltonian(n, 256, seed=args.seed)
     psi.expval_pauli_words(words, wires, coeffs)  # warm
     ms = sorted(timer.time(lambda: psi.expval_pauli_words(words, wires, coeffs)) for _ in range(5))[2]
-    # one read of the state per launch: tile passes of up to 32 words, pair
+    # one read of the state per launch: tile passes of up to 64 words, pair
     # passes of up to 8 words sharing a flip mask
     plan = N.pauli_plan(n, words, wires)
     passes = plan["tile_launches"] + plan["pair_launches"]

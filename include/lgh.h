@@ -262,7 +262,7 @@ lgh_status lgh_expval_pauli_words(const lgh_sv *sv, int64_t num_words, const cha
                                   const double *coeffs, double *per_word, double *result);
 /* Host-only plan of lgh_expval_pauli_words (no device needed): tile passes
  * (words grouped by the index bits their flips touch; each pass reads the
- * state once per launch of up to 32 words) and the pair-kernel launches of
+ * state once per launch of up to 64 words) and the pair-kernel launches of
  * words whose flips span more bits than a tile holds (one pass per flip
  * mask, up to 8 words per launch).  No counterpart in the reference; for
  * byte accounting and tests. */
@@ -273,9 +273,9 @@ lgh_status lgh_pauli_plan(int32_t num_qubits, int64_t num_words, const char *pau
  * reference.  For callers that cannot allocate device memory (code under HIP
  * graph capture, tight serving loops, harnesses that forbid hipMalloc).  Same
  * arguments and results (bit for bit) as lgh_expval_pauli_words; at most 1024
- * words, and the reduction partials of a pass plus 16 B per word must fit a
- * fixed 512 KiB device scratch array (16 B * 16 * 8 * CUs + 16 B * words;
- * 256 KiB of partials on a 256-CU device), else LGH_ERR_INVALID_ARGUMENT.
+ * words, and the reduction partials of a launch plus 8 B per word plus the
+ * launch's word records (6 KiB) must fit a fixed 512 KiB device scratch array
+ * (256 KiB of partials on a 256-CU device), else LGH_ERR_INVALID_ARGUMENT.
  * The scratch array is shared by every call on a device: calls that overlap
  * on one device race and must be serialised by the caller.  The first call
  * on a device looks up the array's address; later calls allocate nothing. */

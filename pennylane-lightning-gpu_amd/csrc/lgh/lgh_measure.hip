@@ -18,6 +18,7 @@
 #include <cstring>
 #include <map>
 #include <type_traits>
+#include <utility>
 
 #include "lgh_internal.hpp"
 
@@ -209,113 +210,168 @@ __global__ __launch_bounds__(kBlock) void k_expval_reg(const cx<R> *__restrict__
 // nY mod 4: +re, -im, -re, +im).
 //
 // Words are grouped into passes by tiles: a pass holds a set of index bits
-// (the three lowest, so that loads cover 128-byte runs, and up to eight more
-// chosen per pass); a workgroup stages each tile of 2^11 amplitudes (all
+// (the three lowest, so that loads cover 128-byte runs, and up to nine more
+// chosen per pass); a workgroup stages each tile of 2^12 amplitudes (all
 // combinations of the pass's bits for one value of the others) in LDS, and
 // every word of the pass whose flip bits are tile bits finds each partner
 // i ^ f in the tile.  One read of the state then serves every word of the
 // pass, whatever their flip masks.  Words with more flip bits than a tile
 // holds take the pair kernel below, one pass per flip mask.
-
-constexpr int kPTileBits = 11;       // amplitudes per tile: 2^11
+//
+// Each wavefront of a workgroup has words of its own and walks the whole tile
+// for them, 64 pairs (i, i ^ f) at a time in 32 steps:
+//  - the terms of i and i ^ f are equal, so one bit of f (the pivot) is kept
+//    clear in i, and the sum over pairs counts twice;
+//  - words of one flip mask (and the same parity of nY) that a wavefront holds
+//    share the pair products conj(psi_{i^f}) psi_i, kept in registers; words
+//    without flips take |psi_i|^2 of two amplitudes a step;
+//  - a word's sign is (-1)^parity of the index bits outside the tile (one
+//    scalar per tile), of the five bits that the steps run over (one FMA with
+//    +1 or -1 per level of a binary tree over the 32 products) and of the
+//    lane's bits (a constant of the whole sum, applied once at the end).
+// So a word costs 31 FMAs a lane and tile, a flip mask 64 LDS reads and 64
+// FMAs more.  64 KiB of LDS: two workgroups of eight wavefronts per CU.
+// Bound by the state reads, one per launch.  24 qubits, 256 words,
+// complex128: 3712 us in 16 launches with tiles of 2^11 and an LDS read per
+// word and amplitude, 1091 us in 11 launches here.
+constexpr int kPTileBits = 12;       // amplitudes per tile: 2^12
 constexpr int kPFixedBits = 3;       // lowest index bits in every tile
-constexpr int kPassWords = 32;       // words per tile launch
+constexpr int kPBlock = 512;
+constexpr int kPWaves = kPBlock / 64;
+constexpr int kPSlots = 8;           // words per wavefront and launch
+constexpr int kPassWords = kPWaves * kPSlots;
+constexpr int kPSteps = 1 << (kPTileBits - 7);
+constexpr int kPLevels = kPTileBits - 7; // bits the steps run over
 constexpr int kMaxWordsPerPass = 8;  // words per pair-kernel launch
 
-// a pass's words as kernel arguments
-struct PWords {
-    int count;
-    uint32_t flip[kPassWords];  // flip mask in tile-local bits
-    uint32_t zyl[kPassWords];   // Z/Y mask in tile-local bits
-    uint32_t phase[kPassWords]; // nY mod 4
-    uint64_t zy[kPassWords];    // Z/Y mask over global index bits (only those outside the tile are read)
+enum : uint32_t { kPEven = 0, kPOdd = 1, kPSquare = 2, kPSquareDiff = 3 }; // products of a flip mask
+
+// One word of a launch, in device memory; read with scalar loads.
+struct alignas(16) PWord {
+    double sign[kPLevels]; // +1 / -1 by the Z/Y mask over the bits that the steps run over
+    double scale;          // real part of i^nY or -i^nY, times two for pairs
+    uint64_t zy;           // Z/Y mask over the index bits outside the tile
+    uint32_t flip;         // flip mask in tile-local bits (the pivot bit where the word has no flips)
+    uint32_t pivot;        // the bit kept clear
+    uint32_t zlane;        // Z/Y mask over the lane's bits
+    uint32_t kind;         // kPEven..kPSquareDiff; bit 4: first word of its products in the wavefront
+    uint32_t row;          // row of the partials
+    uint32_t pad;
 };
-// tile-local bit r is global index bit bit[r]
+// the launch's words, [wavefront][slot]
+struct PLaunch {
+    uint32_t slots[kPWaves];
+    PWord word[kPWaves][kPSlots];
+};
+typedef __attribute__((address_space(4))) const PWord CPWord;
+typedef __attribute__((address_space(4))) const PLaunch CPLaunch;
+
+// tile-local bit r is global index bit bit[r] (ascending)
 struct PTile {
     int g;
     int bit[kPTileBits];
 };
 
-// Sign flip of a double by an integer xor of its high word (bit 31 of
-// `neg`): one instruction instead of a multiply by -1.
-__device__ __forceinline__ double flip_sign(double x, uint32_t neg) {
-    const long long b = __double_as_longlong(x) ^ (static_cast<long long>(neg & 0x80000000u) << 32);
-    return __longlong_as_double(b);
+// The products of a flip mask, 32 pairs per lane.
+template <class R, uint32_t Kind>
+__device__ __forceinline__ void pair_products(const char *tile, uint32_t pivot, uint32_t flip, int lane,
+                                              double (&x)[kPSteps]) {
+    constexpr uint32_t A = sizeof(cx<R>);
+    // the lane's part of i: its six bits around the pivot; then the steps
+    // count in the bits above, around the pivot too
+    const uint32_t low = uint32_t(lane) & ((1u << pivot) - 1u), high = uint32_t(lane) >> pivot;
+    const uint32_t at = pivot < 6 ? (high << (pivot + 1)) | low : uint32_t(lane);
+    const uint32_t pm = pivot < 6 ? 0u : A << pivot, step = pivot < 6 ? 128 * A : 64 * A, fl = flip * A;
+    uint32_t c = 0;
+#pragma unroll
+    for (int k = 0; k < kPSteps; ++k) {
+        const uint32_t i = at * A + c;
+        const cx<R> a = *reinterpret_cast<const cx<R> *>(tile + i);
+        const cx<R> b = *reinterpret_cast<const cx<R> *>(tile + (i ^ fl));
+        if constexpr (Kind == kPEven)
+            x[k] = double(b.re) * a.re + double(b.im) * a.im;
+        else if constexpr (Kind == kPOdd)
+            x[k] = double(b.re) * a.im - double(b.im) * a.re;
+        else if constexpr (Kind == kPSquare)
+            x[k] = (double(a.re) * a.re + double(a.im) * a.im) + (double(b.re) * b.re + double(b.im) * b.im);
+        else
+            x[k] = (double(a.re) * a.re + double(a.im) * a.im) - (double(b.re) * b.re + double(b.im) * b.im);
+        c = ((c | pm) + step) & ~pm;
+    }
 }
 
 template <class R>
-__global__ __launch_bounds__(kBlock) void k_pauli_tile(const cx<R> *__restrict__ sv, uint64_t ntiles,
-                                                       uint64_t tiles_per_block, Fixed tfx, PTile tm, PWords pw,
-                                                       double *__restrict__ partials) {
-    constexpr int kAmps = 1 << kPTileBits;
-    constexpr int kPer = kAmps / kBlock;
-    __shared__ cx<R> tile[kAmps];
-    const int tid = threadIdx.x;
-    const int tsz = 1 << tm.g;
-    uint64_t off[kPer];
+__global__ __launch_bounds__(kPBlock, 4) void k_pauli_tile(const cx<R> *__restrict__ sv, uint64_t ntiles,
+                                                           uint64_t tiles_per_block, Fixed tfx, PTile tm,
+                                                           const PLaunch *__restrict__ launch,
+                                                           double *__restrict__ partials) {
+    __shared__ cx<R> tile[1 << kPTileBits];
+    constexpr int kPer = (1 << kPTileBits) / kPBlock;
+    const int tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const CPLaunch *cl = (const CPLaunch *)launch;
+    const CPWord *cw = &cl->word[w][0];
+    const int slots = int(cl->slots[w]);
+    const uint32_t tsz = 1u << tm.g;
+    uint64_t off = 0, koff[3];
 #pragma unroll
-    for (int k = 0; k < kPer; ++k) {
-        const int j = tid + k * kBlock;
-        uint64_t o = 0;
+    for (int r = 0; r < 9; ++r)
+        if (r < tm.g && ((tid >> r) & 1)) off |= 1ull << tm.bit[r];
 #pragma unroll
-        for (int r = 0; r < kPTileBits; ++r)
-            if (r < tm.g && ((j >> r) & 1)) o |= 1ull << tm.bit[r];
-        off[k] = o;
-    }
-    double acc[kPassWords];
+    for (int r = 0; r < 3; ++r) koff[r] = 9 + r < tm.g ? 1ull << tm.bit[9 + r] : 0;
+    static_assert(kPBlock == 512 && kPer == 8, "nine bits on the threads, three on the loads");
+    double acc[kPSlots];
 #pragma unroll
-    for (int q = 0; q < kPassWords; ++q) acc[q] = 0.0;
+    for (int q = 0; q < kPSlots; ++q) acc[q] = 0.0;
     const uint64_t t0 = uint64_t(blockIdx.x) * tiles_per_block, t1 = min(t0 + tiles_per_block, ntiles);
     for (uint64_t t = t0; t < t1; ++t) {
         const uint64_t base = expand(t, tfx);
-        cx<R> v[kPer];
+        {
+            cx<R> v[kPer];
 #pragma unroll
-        for (int k = 0; k < kPer; ++k) {
-            const int j = tid + k * kBlock;
-            v[k] = cx<R>{R(0), R(0)};
-            if (j < tsz) {
-                v[k] = ldnt(sv + (base | off[k]));
-                tile[j] = v[k];
+            for (int k = 0; k < kPer; ++k) {
+                const uint64_t ko = (k & 1 ? koff[0] : 0) | (k & 2 ? koff[1] : 0) | (k & 4 ? koff[2] : 0);
+                v[k] = uint32_t(tid + k * kPBlock) < tsz ? ldnt(sv + (base | off | ko)) : cx<R>{R(0), R(0)};
             }
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) tile[tid + k * kPBlock] = v[k];
         }
         __syncthreads();
-#pragma unroll
-        for (int q = 0; q < kPassWords; ++q) {
-            if (q >= pw.count) break;
-            const uint32_t f = pw.flip[q], zl = pw.zyl[q], ph = pw.phase[q];
-            // the word's sign outside the tile is uniform over the tile
-            const uint32_t pbase = uint32_t(__popcll(base & pw.zy[q]) & 1) << 31;
-            // only the component i^nY turns into the real part is summed
-            double sum = 0.0;
-            if ((ph & 1u) == 0) {
-#pragma unroll
-                for (int k = 0; k < kPer; ++k) {
-                    const int j = tid + k * kBlock;
-                    if (j < tsz) {
-                        const cx<R> p = tile[j ^ int(f)];
-                        const double x = double(p.re) * v[k].re + double(p.im) * v[k].im;
-                        sum += flip_sign(x, (uint32_t(__popc(uint32_t(j) & zl)) << 31) ^ pbase);
-                    }
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < kPer; ++k) {
-                    const int j = tid + k * kBlock;
-                    if (j < tsz) {
-                        const cx<R> p = tile[j ^ int(f)];
-                        const double x = double(p.re) * v[k].im - double(p.im) * v[k].re;
-                        sum += flip_sign(x, (uint32_t(__popc(uint32_t(j) & zl)) << 31) ^ pbase);
-                    }
+        double x[kPSteps];
+#pragma unroll 1
+        for (int q = 0; q < slots; ++q) {
+            const uint32_t kind = cw[q].kind;
+            if (kind & 16u) {
+                const char *tp = reinterpret_cast<const char *>(tile);
+                const uint32_t pivot = cw[q].pivot, flip = cw[q].flip;
+                switch (kind & 3u) {
+                case kPEven: pair_products<R, kPEven>(tp, pivot, flip, lane, x); break;
+                case kPOdd: pair_products<R, kPOdd>(tp, pivot, flip, lane, x); break;
+                case kPSquare: pair_products<R, kPSquare>(tp, pivot, flip, lane, x); break;
+                default: pair_products<R, kPSquareDiff>(tp, pivot, flip, lane, x); break;
                 }
             }
-            // i^nY: +re, -im, -re, +im
-            acc[q] += (ph == 1u || ph == 2u) ? -sum : sum;
+            // sum over the steps with the sign of each of their bits
+            double y[kPSteps / 2];
+#pragma unroll
+            for (int k = 0; k < kPSteps / 2; ++k) y[k] = fma(x[2 * k + 1], cw[q].sign[0], x[2 * k]);
+#pragma unroll
+            for (int l = 1; l < kPLevels; ++l)
+#pragma unroll
+                for (int k = 0; k < (kPSteps >> (l + 1)); ++k) y[k] = fma(y[2 * k + 1], cw[q].sign[l], y[2 * k]);
+            const double s = (__popcll(base & cw[q].zy) & 1) ? -y[0] : y[0];
+#pragma unroll
+            for (int u = 0; u < kPSlots; ++u)
+                if (u == q) acc[u] += s;
         }
         __syncthreads(); // the next tile overwrites the LDS copy
     }
-    block_sum<kPassWords>(acc);
-    if (tid == 0)
-        for (int q = 0; q < pw.count; ++q) partials[size_t(q) * gridDim.x + blockIdx.x] = acc[q];
+#pragma unroll
+    for (int q = 0; q < kPSlots; ++q) {
+        if (q >= slots) break;
+        const bool neg = __popc(uint32_t(lane) & cw[q].zlane) & 1;
+        const double s = wave_sum(neg ? -acc[q] : acc[q]);
+        if (lane == 0) partials[size_t(cw[q].row) * gridDim.x + blockIdx.x] = cw[q].scale * s;
+    }
 }
 
 struct WordSet {
@@ -1097,17 +1153,99 @@ int64_t plan_pauli_tiles(int n, int64_t nwords, const uint64_t *flip, int32_t *p
     return np;
 }
 
+// Workgroups of a tile launch: the two that a CU holds.
+constexpr unsigned kPauliBlocksPerCU = 2;
+
+// Tile-local bits of a pass, ascending.
+PTile pauli_layout(const PGeo &geo, int n, uint64_t chosen) {
+    PTile tm{};
+    tm.g = geo.g;
+    int r = 0;
+    for (int b = 0; b < n; ++b)
+        if (b < geo.fixed || ((chosen >> b) & 1)) tm.bit[r++] = b;
+    LGH_REQUIRE(r == geo.g, "Pauli tile: bad bit count");
+    return tm;
+}
+
+uint32_t to_tile(const PTile &tm, uint64_t mask) {
+    uint32_t m = 0;
+    for (int q = 0; q < tm.g; ++q) m |= uint32_t((mask >> tm.bit[q]) & 1u) << q;
+    return m;
+}
+
+// One word's record for the pivot bit `pivot`.
+PWord pauli_word(const PTile &tm, uint64_t tile_mask, uint64_t flip, uint64_t zy, int32_t ny, uint32_t pivot) {
+    PWord pw{};
+    const uint32_t fl = to_tile(tm, flip), zl = to_tile(tm, zy), ph = uint32_t(ny & 3);
+    pw.pivot = pivot;
+    pw.flip = fl ? fl : 1u << pivot;
+    pw.kind = fl ? (ph & 1u ? kPOdd : kPEven) : (zl >> pivot) & 1u ? kPSquareDiff : kPSquare;
+    // lane bits, then step bits, are the tile's bits without the pivot
+    int at = 0;
+    for (uint32_t b = 0; b < uint32_t(kPTileBits); ++b) {
+        if (b == pivot) continue;
+        const bool z = (zl >> b) & 1u;
+        if (at < 6)
+            pw.zlane |= uint32_t(z) << at;
+        else
+            pw.sign[at - 6] = z ? -1.0 : 1.0;
+        ++at;
+    }
+    // i^nY: +re, -im, -re, +im
+    pw.scale = (ph == 1 || ph == 2 ? -1.0 : 1.0) * (fl ? 2.0 : 1.0);
+    pw.zy = zy & ~tile_mask;
+    return pw;
+}
+
+// Records of up to kPassWords words (sorted by flip mask and parity of nY)
+// spread over the wavefronts: words that share products stay together, in
+// groups of at most the wavefronts' mean, each group on the wavefront with
+// the least to do (products weigh as three words) that has room.
+void pauli_fill(PLaunch &l, const PTile &tm, uint64_t tile_mask, const int32_t *words, int count, const uint64_t *flip,
+                const uint64_t *zy, const int32_t *ny) {
+    l = PLaunch{};
+    int load[kPWaves] = {};
+    const int most = std::min(kPSlots, (count + kPWaves - 1) / kPWaves);
+    for (int s = 0; s < count;) {
+        // the pivot: the highest flipped bit; without flips the highest bit
+        // outside the word's own mask, kept while the next words allow it
+        const int32_t w0 = words[s];
+        const uint32_t fl = to_tile(tm, flip[w0]), z0 = to_tile(tm, zy[w0]), all = (1u << kPTileBits) - 1u;
+        const uint32_t from = fl ? fl : (~z0 & all) ? (~z0 & all) : all;
+        const uint32_t pivot = 31u - uint32_t(__builtin_clz(from));
+        const uint32_t kind = pauli_word(tm, tile_mask, flip[w0], zy[w0], ny[w0], pivot).kind;
+        int best = -1;
+        for (int w = 0; w < kPWaves; ++w)
+            if (l.slots[w] < uint32_t(kPSlots) && (best < 0 || load[w] < load[best])) best = w;
+        LGH_REQUIRE(best >= 0, "Pauli words: no room");
+        load[best] += 3;
+        for (int taken = 0; s < count && taken < most && l.slots[best] < uint32_t(kPSlots); ++taken, ++s) {
+            const int32_t w = words[s];
+            if (flip[w] != flip[w0]) break;
+            PWord pw = pauli_word(tm, tile_mask, flip[w], zy[w], ny[w], pivot);
+            if (pw.kind != kind) break;
+            pw.kind |= taken == 0 ? 16u : 0u;
+            pw.row = uint32_t(s);
+            l.word[best][l.slots[best]++] = pw;
+            ++load[best];
+        }
+    }
+}
+
 struct PauliBufs {
     double *partials; // device, partials_cap doubles
     size_t partials_cap;
     double *results;  // one double per word: device memory or pinned host memory
+    // copies a launch's records to the device (stream ordered) and returns their address there
+    const PLaunch *(*upload)(StreamCtx *ctx, const PLaunch &launch, void *arg);
+    void *arg;
 };
 
 // Device doubles of reduction partials the Pauli passes of an n-qubit state need.
 size_t pauli_partials_doubles(int n, int device) {
     const uint64_t len = 1ull << n;
     const unsigned pair_blocks = chunks_for(len, device).blocks;
-    const unsigned tile_blocks = unsigned(std::max(1, sm_count(device))) * 4;
+    const unsigned tile_blocks = unsigned(std::max(1, sm_count(device))) * kPauliBlocksPerCU;
     return std::max(size_t(kMaxWordsPerPass) * pair_blocks, size_t(kPassWords) * tile_blocks);
 }
 
@@ -1126,47 +1264,42 @@ void pauli_run(const lgh_sv *sv, int64_t nwords, const uint64_t *flip, const uin
     int64_t nslots = 0;
     // tile passes
     const uint64_t ntiles = len >> geo.g;
-    const unsigned max_blocks = unsigned(std::max(1, sm_count(sv->device))) * 4;
+    const unsigned max_blocks = unsigned(std::max(1, sm_count(sv->device))) * kPauliBlocksPerCU;
     const uint64_t per_block = (ntiles + max_blocks - 1) / max_blocks;
     const unsigned tblocks = unsigned((ntiles + per_block - 1) / per_block);
     LGH_REQUIRE(size_t(kPassWords) * tblocks <= bufs.partials_cap, "Pauli partials buffer too small");
+    // the words of each pass, by flip mask (slot_word: result slot -> word)
     for (int64_t p = 0; p < npasses; ++p) {
-        PTile tm{};
-        tm.g = geo.g;
-        int r = 0;
-        for (int b = 0; b < geo.fixed; ++b) tm.bit[r++] = b;
-        for (int b = geo.fixed; b < n; ++b)
-            if ((pass_mask[p] >> b) & 1) tm.bit[r++] = b;
-        LGH_REQUIRE(r == geo.g, "Pauli tile: bad bit count");
+        const int64_t first = nslots;
+        for (int64_t w = 0; w < nwords; ++w)
+            if (pass_of[w] == p) slot_word[nslots++] = int32_t(w);
+        std::sort(slot_word + first, slot_word + nslots, [&](int32_t x, int32_t y) {
+            if (flip[x] != flip[y]) return flip[x] < flip[y];
+            if ((ny[x] & 1) != (ny[y] & 1)) return (ny[x] & 1) < (ny[y] & 1);
+            return x < y;
+        });
+    }
+    for (int64_t first = 0, end; first < nslots; first = end) {
+        const int32_t p = pass_of[slot_word[first]];
+        for (end = first; end < nslots && pass_of[slot_word[end]] == p;) ++end;
+        const PTile tm = pauli_layout(geo, n, pass_mask[p]);
+        uint64_t tile_mask = 0;
         Fixed tfx{};
         tfx.cnt = geo.g;
-        for (int q = 0; q < geo.g; ++q) tfx.pos[q] = tm.bit[q]; // ascending
-        PWords pw{};
-        auto launch = [&] {
-            hipLaunchKernelGGL(k_pauli_tile<R>, dim3(tblocks), dim3(kBlock), 0, ctx->stream, cdata<R>(sv), ntiles,
-                               per_block, tfx, tm, pw, bufs.partials);
-            LGH_LAUNCH_CHECK();
-            launch_reduce(ctx, bufs.partials, int(tblocks), pw.count, bufs.results + (nslots - pw.count));
-            pw.count = 0;
-        };
-        for (int64_t w = 0; w < nwords; ++w) {
-            if (pass_of[w] != p) continue;
-            uint32_t fl = 0, zl = 0;
-            uint64_t tile_mask = 0;
-            for (int q = 0; q < geo.g; ++q) {
-                if ((flip[w] >> tm.bit[q]) & 1) fl |= 1u << q;
-                if ((zy[w] >> tm.bit[q]) & 1) zl |= 1u << q;
-                tile_mask |= 1ull << tm.bit[q];
-            }
-            pw.flip[pw.count] = fl;
-            pw.zyl[pw.count] = zl;
-            pw.zy[pw.count] = zy[w] & ~tile_mask;
-            pw.phase[pw.count] = uint32_t(ny[w] & 3);
-            ++pw.count;
-            slot_word[nslots++] = int32_t(w);
-            if (pw.count == kPassWords) launch();
+        for (int q = 0; q < geo.g; ++q) {
+            tfx.pos[q] = tm.bit[q];
+            tile_mask |= 1ull << tm.bit[q];
         }
-        if (pw.count > 0) launch();
+        for (int64_t s = first; s < end; s += kPassWords) {
+            const int nw = int(std::min<int64_t>(kPassWords, end - s));
+            PLaunch launch;
+            pauli_fill(launch, tm, tile_mask, slot_word + s, nw, flip, zy, ny);
+            const PLaunch *dl = bufs.upload(ctx, launch, bufs.arg);
+            hipLaunchKernelGGL(k_pauli_tile<R>, dim3(tblocks), dim3(kPBlock), 0, ctx->stream, cdata<R>(sv), ntiles,
+                               per_block, tfx, tm, dl, bufs.partials);
+            LGH_LAUNCH_CHECK();
+            launch_reduce(ctx, bufs.partials, int(tblocks), nw, bufs.results + s);
+        }
     }
     // words wider than a tile: one pair pass per flip mask, ascending
     for (int64_t w = 0; w < nwords; ++w) done[w] = pass_of[w] >= 0;
@@ -1219,7 +1352,11 @@ void pauli_t(const lgh_sv *sv, int64_t nwords, const char *paulis, const int32_t
     double *partials = static_cast<double *>(ctx->workspace(sizeof(double) * pcap));
     // the reductions write the words' values into pinned host memory
     double *host = static_cast<double *>(ctx->host_buffer(sizeof(double) * std::max<size_t>(1, nw)));
-    PauliBufs bufs{partials, pcap, host};
+    PauliBufs bufs{partials, pcap, host,
+                   [](StreamCtx *c, const PLaunch &l, void *) {
+                       return static_cast<const PLaunch *>(c->upload(&l, sizeof(l)));
+                   },
+                   nullptr};
     if (nwords > 0)
         pauli_run<R>(sv, nwords, flip.data(), zy.data(), ny.data(), pass_of.data(), pass_mask.data(), done.get(),
                      slot_word.data(), bufs);
@@ -1240,7 +1377,7 @@ void pauli_t(const lgh_sv *sv, int64_t nwords, const char *paulis, const int32_t
 // the device's CU count used to size the passes).
 //
 // Layout of `scratch` for one call: reduction partials of one launch |
-// one result per word.  Every entry a call reads was written earlier in the
+// one result per word | the launch's word records.  Every entry a call reads was written earlier in the
 // same call (each launch writes all its partials, each reduction its
 // words' results), so nothing needs clearing; two calls that overlap on one
 // device race on the array.
@@ -1282,11 +1419,20 @@ void pauli_noalloc_t(const lgh_sv *sv, int64_t nwords, const char *paulis, const
     bool done[kNoAllocMaxWords];
     for (int64_t w = 0; w < nwords; ++w) parse_word(sv->n, paulis, wires, offsets[w], offsets[w + 1], flip[w], zy[w], ny[w]);
     const size_t pcap = pauli_partials_doubles(sv->n, sv->device);
-    const size_t need = sizeof(double) * (pcap + size_t(nwords));
+    // partials | results | a launch's records
+    const size_t o_words = (sizeof(double) * (pcap + size_t(nwords)) + 255) & ~size_t(255);
+    const size_t need = o_words + sizeof(PLaunch);
     LGH_REQUIRE(need <= kNoAllocScratchBytes, "lgh_expval_pauli_words_noalloc: " + std::to_string(need) +
                                                   " bytes of scratch needed, " +
                                                   std::to_string(kNoAllocScratchBytes) + " available");
-    PauliBufs bufs{reinterpret_cast<double *>(base), pcap, reinterpret_cast<double *>(base) + pcap};
+    PauliBufs bufs{reinterpret_cast<double *>(base), pcap, reinterpret_cast<double *>(base) + pcap,
+                   [](StreamCtx *c, const PLaunch &l, void *dst) {
+                       // pageable memory of the calling thread: wait until it has been read
+                       LGH_HIP(hipMemcpyAsync(dst, &l, sizeof(l), hipMemcpyHostToDevice, c->stream));
+                       c->sync();
+                       return static_cast<const PLaunch *>(dst);
+                   },
+                   base + o_words};
     if (nwords > 0) pauli_run<R>(sv, nwords, flip, zy, ny, pass_of, pass_mask, done, slot_word, bufs);
     double out[kNoAllocMaxWords];
     double vals[kNoAllocMaxWords];

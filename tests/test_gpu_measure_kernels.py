@@ -127,3 +127,41 @@ def test_controlled_dense_matrices_on_many_wires(n, k, ctrl):
     N.check(N.lib().lgh_apply(s.handle, arr, 1))
     np.testing.assert_allclose(s.download(), np_matrix(psi, n, w[ctrl:], u, w[:ctrl]),
                                atol=4 * np.sqrt(D) * 2.3e-16, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("n", [2, 7, 9, 11, 12, 13, 16])
+def test_pauli_words_by_flip_mask(n, dtype):
+    """States smaller than, equal to and larger than a tile (2^12 amplitudes); many words of one flip mask (a launch
+    holds 64 words, a wavefront 8 of them), Z words up to the one on every wire (every tile bit signed), flips on
+    every wire, every number of Y factors."""
+    rng = np.random.default_rng(n)
+    psi = rand_state(n, 5 * n, dtype)
+    every = list(range(n))
+    words, wires = ["Z" * n, "X" * n, "Y" * n, "", "I"], [every, every, every, [], [0]]
+    for k in range(80):  # Z words
+        ws = [int(x) for x in rng.permutation(n)[:int(rng.integers(1, n + 1))]]
+        words.append("Z" * len(ws))
+        wires.append(ws)
+    for k in range(90):  # few masks, many words of each
+        ws = [int(x) for x in rng.permutation(n)[:int(rng.integers(1, min(n, 6) + 1))]]
+        letters = ["XY"[int(rng.integers(2))] if w < min(n, 3) else "Z" for w in ws]
+        words.append("".join(letters))
+        wires.append(ws)
+    for k in range(90):
+        ws = [int(x) for x in rng.permutation(n)[:int(rng.integers(1, min(n, 4) + 1))]]
+        words.append("".join(rng.choice(list("XYZI"), len(ws))))
+        wires.append(ws)
+    total, per = N.State(n, dtype).upload(psi).expval_pauli_words(words, wires, np.arange(len(words)) * 0.01)
+    p = psi.astype(np.complex128)
+    idx = np.arange(1 << n)
+    ref = []
+    for word, ws in zip(words, wires):
+        flip = sum(1 << (n - 1 - w) for c, w in zip(word, ws) if c in "XY")
+        zy = sum(1 << (n - 1 - w) for c, w in zip(word, ws) if c in "YZ")
+        par = np.array([bin(int(i) & zy).count("1") & 1 for i in idx]) if n <= 9 else \
+            np.bitwise_count(idx & zy).astype(np.int64) & 1
+        ref.append(np.real(1j ** word.count("Y") * np.sum((1 - 2 * par) * np.conj(p[idx ^ flip]) * p)))
+    # sums of 2^n products of total size 1
+    np.testing.assert_allclose(per, ref, atol=2.0 ** (n / 2) * 4e-16, rtol=0)
+    np.testing.assert_allclose(total, np.dot(np.arange(len(words)) * 0.01, ref), atol=2.0 ** (n / 2) * 4e-14, rtol=0)
