@@ -27,6 +27,8 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kBras = 8; // observable states per launch
+// bytes of lambda and observable states of the fused sweeps that run side by side
+constexpr size_t kSideBySide = size_t(4) << 30;
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -419,22 +421,28 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
     StreamCtx *ctx = psi_in->ctx;
     for (int j = 0; j < nobs; ++j)
         if (bras[j]->ctx != ctx) bras[j]->ctx->sync();
-    // lambda: working copy of psi
-    lgh_sv lam = *psi_in;
-    lam.data = pool_alloc(psi_in->device, psi_in->bytes);
-    struct Free {
-        lgh_sv *s;
-        ~Free() {
-            (void)hipStreamSynchronize(s->ctx->stream);
-            pool_free(s->device, s->data, s->bytes);
+    const bool fused_path = fusion_enabled() && fused_partials_bytes(n, psi_in->device) > 0 && nobs > 0;
+    // Working copies of psi, freed once the stream has been waited for.
+    struct Buffers {
+        const lgh_sv *like;
+        std::vector<void *> ptrs;
+        void *take() {
+            ptrs.push_back(pool_alloc(like->device, like->bytes));
+            return ptrs.back();
         }
-    } free_lam{&lam};
+        ~Buffers() {
+            (void)hipStreamSynchronize(like->ctx->stream);
+            for (void *p : ptrs) pool_free(like->device, p, like->bytes);
+        }
+    } buffers{psi_in, {}};
     // The fused sweep reads lambda's starting values from psi itself when no
     // forward application is asked for; the other forms work on a copy.
-    const bool fused_path = fusion_enabled() && fused_partials_bytes(n, psi_in->device) > 0 && nobs > 0;
-    const bool from_psi = fused_path && !apply_ops;
-    if (!from_psi)
+    lgh_sv lam = *psi_in;
+    const void *start = psi_in->data;
+    if (!fused_path || apply_ops) {
+        start = lam.data = buffers.take();
         LGH_HIP(hipMemcpyAsync(lam.data, psi_in->data, psi_in->bytes, hipMemcpyDeviceToDevice, ctx->stream));
+    }
     if (apply_ops)
         for (int64_t i = 0; i < nops; ++i)
             if (!is_prep(ops[i])) launch_kop(&lam, compile_op(ops[i], n, false));
@@ -442,31 +450,43 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
     if (zmasks && !fused_path)
         for (int j = 0; j < nobs; ++j) zsign<R>(bras[j], lam.data, zmasks[j], ctx->stream);
 
-    // workspace: [jac (nobs*ntp) | bra pointers | partials]
+    // Sweeps that run side by side in the fused path share the launches of a
+    // pass: a small state leaves the device idle on its own, a large one at
+    // the end of every pass.  Two layers of StronglyEntanglingLayers with
+    // <Z_w> on every wire, complex128, one sweep after another and side by
+    // side: 12 qubits 3180 and 570 us (the sweeps of a 4-layer ring circuit),
+    // 18 qubits 3329 and 1269, 20 qubits 4677 and 2785, 22 qubits 12.3 and
+    // 10.0 ms, 24 qubits 43 and 40.5 ms.  The limit bounds the memory: a
+    // lambda for each sweep of a group, half of it.
+    int group = fused_path ? int(std::max<size_t>(1, std::min<size_t>({size_t(nobs), size_t(65535),
+                                                                             kSideBySide / (2 * psi_in->bytes)})))
+                                 : 1;
+    // workspace: [jac (nobs*ntp) | bra pointers | partials of the steps | slices | fused partials | sweep table]
     // the widest step shape has one thread per amplitude
     const unsigned max_blocks = unsigned(((1ull << n) + kBlock - 1) / kBlock);
     const int nbatches = std::max(1, (nobs + kBras - 1) / kBras);
     auto al = [](size_t b) { return (b + 255) & ~size_t(255); };
     const size_t b_jac = al(sizeof(double) * size_t(std::max<int64_t>(1, nobs * ntp)));
     const size_t b_ptr = al(sizeof(void *) * size_t(nbatches * kBras));
-    const size_t b_part = al(sizeof(double) * size_t(nbatches) * kBras * max_blocks);
+    // the fused path's standalone steps take one observable at a time
+    const size_t b_part = al(sizeof(double) * (fused_path ? 1 : size_t(nbatches) * kBras) * max_blocks);
     const size_t b_slices = al(sizeof(double) * kBras * kSlices);
-    const size_t b_fused = al(fused_partials_bytes(n, psi_in->device));
-    char *ws = static_cast<char *>(ctx->workspace(b_jac + b_ptr + b_part + b_slices + b_fused));
-    double *slices = reinterpret_cast<double *>(ws + b_jac + b_ptr + b_part);
-    double *fpartials = reinterpret_cast<double *>(ws + b_jac + b_ptr + b_part + b_slices);
+    const size_t b_fused = al(fused_partials_bytes(n, psi_in->device) * size_t(group));
+    const size_t b_tab = fused_path ? al(AdjPasses::kTableBytes * size_t(group)) : 0;
+    char *ws = static_cast<char *>(ctx->workspace(b_jac + b_ptr + b_part + b_slices + b_fused + b_tab));
     double *jac_dev = reinterpret_cast<double *>(ws);
     cx<R> **bras_dev = reinterpret_cast<cx<R> **>(ws + b_jac);
     double *partials = reinterpret_cast<double *>(ws + b_jac + b_ptr);
+    double *slices = reinterpret_cast<double *>(ws + b_jac + b_ptr + b_part);
+    double *fpartials = reinterpret_cast<double *>(ws + b_jac + b_ptr + b_part + b_slices);
+    void *table = ws + b_jac + b_ptr + b_part + b_slices + b_fused;
     std::vector<void *> hp(size_t(nbatches * kBras), nullptr);
     for (int j = 0; j < nobs; ++j) hp[size_t(j)] = bras[j]->data;
-    LGH_HIP(hipMemcpyAsync(bras_dev, hp.data(), sizeof(void *) * hp.size(), hipMemcpyHostToDevice, ctx->stream));
+    ctx->copy_in(bras_dev, hp.data(), sizeof(void *) * hp.size());
     LGH_HIP(hipMemsetAsync(jac_dev, 0, sizeof(double) * size_t(std::max<int64_t>(1, nobs * ntp)), ctx->stream));
-    ctx->sync(); // hp is a host temporary
 
     if (fused_path) {
-        // Fused reverse sweep, one observable state at a time on a fresh copy
-        // of lambda.  Ops before the earliest trainable one are never visited.
+        // Fused reverse sweeps.  Ops before the earliest trainable one are never visited.
         std::vector<KOp> udag;
         std::vector<KGen> gens;
         std::vector<int> slot;
@@ -493,50 +513,51 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
             }
             slot.push_back(col);
         }
-        lgh_sv lam0 = lam; // forward state every observable sweep starts from (after apply_ops)
-        lam0.data = nullptr;
-        if (nobs > 1 && !from_psi) {
-            lam0.data = pool_alloc(psi_in->device, psi_in->bytes);
-            LGH_HIP(hipMemcpyAsync(lam0.data, lam.data, lam.bytes, hipMemcpyDeviceToDevice, ctx->stream));
+        const AdjPasses passes(psi_in, udag, gens, slot, fac);
+        // lambda per sweep of a group; a single sweep may use up the forward state formed above
+        std::vector<lgh_sv> lams(size_t(group), *psi_in);
+        const bool own = apply_ops && nobs == 1;
+        for (int j = 0; j < group; ++j) {
+            try {
+                lams[size_t(j)].data = own ? lam.data : buffers.take();
+            } catch (const Error &e) {
+                if (j == 0 || e.code != LGH_ERR_OUT_OF_MEMORY) throw;
+                group = j; // what memory is left takes fewer at a time
+            }
         }
-        struct Free0 {
-            lgh_sv *s;
-            ~Free0() {
-                if (!s->data) return;
-                (void)hipStreamSynchronize(s->ctx->stream);
-                pool_free(s->device, s->data, s->bytes);
+        auto standalone = [&](const AdjSweep &sw, const KOp &u, const KGen *g, int64_t col, double f) {
+            const bool fusedk = u.kind == KOp::DIAG || (u.kind == KOp::DENSE && (u.k == 1 || u.k == 2 || u.k == 4));
+            if (!fusedk) {
+                launch_kop(sw.lam, u);
+                launch_kop(sw.bra, u);
+                return;
             }
-        } free_lam0{&lam0};
-        for (int j = 0; j < nobs; ++j) {
-            if (j > 0 && !from_psi)
-                LGH_HIP(hipMemcpyAsync(lam.data, lam0.data, lam.bytes, hipMemcpyDeviceToDevice, ctx->stream));
-            double *jrow = jac_dev + size_t(j) * ntp;
-            auto standalone = [&](const KOp &u, const KGen *g, int64_t col, double f) {
-                const bool fusedk = u.kind == KOp::DIAG || (u.kind == KOp::DENSE && (u.k == 1 || u.k == 2 || u.k == 4));
-                if (!fusedk) {
-                    launch_kop(&lam, u);
-                    launch_kop(bras[j], u);
-                    return;
-                }
-                fused_step<R>(&lam, bras_dev + j, 1, u, g, partials);
-                if (g) {
-                    const unsigned blocks = step_shape(n, u).blocks;
-                    hipLaunchKernelGGL(k_row_chunks, dim3(kSlices, 1), dim3(kBlock), 0, ctx->stream, partials,
-                                       int(blocks), slices);
-                    hipLaunchKernelGGL(k_jac_store, dim3(1), dim3(kBlock), 0, ctx->stream, slices, jrow, ntp, col, f);
-                    LGH_LAUNCH_CHECK();
-                }
-            };
-            if (zmasks) {
-                // the sweep's starting lambda: psi itself, or lam's copy of it
-                const void *start = from_psi ? psi_in->data : lam.data;
-                BraFromZ bz{zmasks[j], [&, j, start] { zsign<R>(bras[j], start, zmasks[j], ctx->stream); }};
-                fused_adjoint_one(&lam, from_psi ? psi_in->data : nullptr, bras[j], udag, gens, slot, fac, jrow,
-                                  fpartials, standalone, &bz);
-            } else {
-                fused_adjoint_one(&lam, from_psi ? psi_in->data : nullptr, bras[j], udag, gens, slot, fac, jrow,
-                                  fpartials, standalone);
+            const ptrdiff_t j = (sw.jac_row - jac_dev) / ntp;
+            fused_step<R>(sw.lam, bras_dev + j, 1, u, g, partials);
+            if (g) {
+                const unsigned blocks = step_shape(n, u).blocks;
+                hipLaunchKernelGGL(k_row_chunks, dim3(kSlices, 1), dim3(kBlock), 0, ctx->stream, partials, int(blocks),
+                                   slices);
+                hipLaunchKernelGGL(k_jac_store, dim3(1), dim3(kBlock), 0, ctx->stream, slices, sw.jac_row, ntp, col, f);
+                LGH_LAUNCH_CHECK();
             }
+        };
+        for (int j0 = 0; j0 < nobs; j0 += group) {
+            std::vector<AdjSweep> sweeps;
+            for (int j = j0; j < std::min(nobs, j0 + group); ++j) {
+                AdjSweep sw;
+                sw.lam = &lams[size_t(j - j0)];
+                sw.lam_src = own ? nullptr : start;
+                sw.bra = bras[j];
+                sw.jac_row = jac_dev + size_t(j) * size_t(ntp);
+                if (zmasks) {
+                    sw.bra_from_z = true;
+                    sw.zmask = zmasks[j];
+                    sw.materialize = [&, j] { zsign<R>(bras[j], start, zmasks[j], ctx->stream); };
+                }
+                sweeps.push_back(std::move(sw));
+            }
+            passes.run(sweeps.data(), int(sweeps.size()), fpartials, table, standalone);
         }
         if (nobs * ntp > 0)
             LGH_HIP(hipMemcpyAsync(jac_host, jac_dev, sizeof(double) * size_t(nobs * ntp), hipMemcpyDeviceToHost,

@@ -469,28 +469,42 @@ __global__ __launch_bounds__(kBlock) void k_fused_pass(cx<R> *__restrict__ sv, u
     }
 }
 
-// Reverse pass of the adjoint sweep on lambda and one observable state.  The
-// ops of the pass are stored in reverse order with U^dagger matrices.  Each
+// One sweep's arrays (device table, one entry per blockIdx.y).
+struct AdjArrays {
+    const void *lam_src; // lambda's starting values
+    void *lam, *bra;
+    uint64_t zmask;
+    double *jac_row;
+};
+typedef __attribute__((address_space(4))) const AdjArrays CAdjArrays;
+
+// Reverse pass of the adjoint sweep on lambda and one observable state; the
+// sweeps of blockIdx.y run side by side (observables of a state too small to
+// fill the device).  The ops of the pass are stored in reverse order with
+// U^dagger matrices.  Each
 // lane accumulates its overlap contributions in its own LDS column; the
 // reduction over lanes and wavefronts happens once at the end.
-// lam_in: where lambda is read (lam itself, or the forward state for the
-// first pass of a sweep, which then needs no copy of it); lam: where it is
-// written.  Each thread reads and writes its own amplitudes only, so the two
-// may be the same array.
-// bra_zmask != 0 with bra_from_lam: the observable state is not read but
-// formed from lambda's loaded values as Z-word(bra_zmask) lambda (the sign
-// (-1)^popcount(index & bra_zmask) per amplitude), then written like any
-// pass's output: the first reverse pass of a sweep with a Z-word observable
-// needs no separate pass that forms it.
+// from_src: lambda is read from lam_src (the forward state, for the first pass
+// of a sweep, which then needs no copy of it) and written to lam.  Each thread
+// reads and writes its own amplitudes only, so the two may be the same array.
+// bra_from_lam: the observable state is not read but formed from lambda's
+// loaded values as Z-word(zmask) lambda (the sign (-1)^popcount(index & zmask)
+// per amplitude), then written like any pass's output: the first reverse pass
+// of a sweep with a Z-word observable needs no separate pass that forms it.
 template <class R, int RB, int Lv>
-__device__ __forceinline__ void fused_adj_body(const cx<R> *lam_in, cx<R> *lam, cx<R> *__restrict__ bra,
-                                               uint64_t ntiles, uint64_t chunk, const PassDesc *__restrict__ pd,
-                                               const FOp *__restrict__ ops, const FGen *__restrict__ gens,
-                                               double *__restrict__ partials, uint64_t bra_zmask, int bra_from_lam) {
+__device__ __forceinline__ void fused_adj_body(const AdjArrays *__restrict__ arrays, uint64_t ntiles, uint64_t chunk,
+                                               const PassDesc *__restrict__ pd, const FOp *__restrict__ ops,
+                                               const FGen *__restrict__ gens, double *__restrict__ partials_all,
+                                               uint64_t partials_stride, int from_src, int bra_from_lam) {
     static_assert(kAccCols * kAccLanes == kBlock, "one accumulator column per lane quad");
     __shared__ double acc[adj_slot_cap(RB)][kAccCols];
     __shared__ double sink[kBlock];
     const AccCols cols{acc, sink};
+    const CAdjArrays *ar = (const CAdjArrays *)arrays + blockIdx.y;
+    cx<R> *lam = static_cast<cx<R> *>(ar->lam), *__restrict__ bra = static_cast<cx<R> *>(ar->bra);
+    const cx<R> *lam_in = from_src ? static_cast<const cx<R> *>(ar->lam_src) : lam;
+    const uint64_t bra_zmask = ar->zmask;
+    double *__restrict__ partials = partials_all + blockIdx.y * partials_stride;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const CFOp *cops = (const CFOp *)ops;
     const CFGen *cgens = (const CFGen *)gens;
@@ -617,30 +631,33 @@ __device__ __forceinline__ void fused_adj_body(const cx<R> *lam_in, cx<R> *lam, 
 // Lv: lean level of the pass (0: any fusable gate).
 template <class R, int Lv = 0>
 __global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 5 : 3) void k_fused_adj3(
-    const cx<R> *lam_in, cx<R> *lam, cx<R> *__restrict__ bra, uint64_t ntiles, uint64_t chunk,
-    const PassDesc *__restrict__ pd, const FOp *__restrict__ ops, const FGen *__restrict__ gens,
-    double *__restrict__ partials, uint64_t bra_zmask, int bra_from_lam) {
-    fused_adj_body<R, 3, Lv>(lam_in, lam, bra, ntiles, chunk, pd, ops, gens, partials, bra_zmask, bra_from_lam);
+    const AdjArrays *__restrict__ arrays, uint64_t ntiles, uint64_t chunk, const PassDesc *__restrict__ pd,
+    const FOp *__restrict__ ops, const FGen *__restrict__ gens, double *__restrict__ partials, uint64_t partials_stride,
+    int from_src, int bra_from_lam) {
+    fused_adj_body<R, 3, Lv>(arrays, ntiles, chunk, pd, ops, gens, partials, partials_stride, from_src, bra_from_lam);
 }
 // Four register bits: the complex128 lean kernels are held to 168 VGPRs for
 // three wavefronts per SIMD (39 dwords spilled to scratch at level 1; 4.50
 // against 4.88 ms per 28-qubit pass at two wavefronts).
 template <class R, int Lv = 0>
-__global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 3 : 1) void k_fused_adj4(const cx<R> *lam_in, cx<R> *lam, cx<R> *__restrict__ bra,
-                                                    uint64_t ntiles, uint64_t chunk, const PassDesc *__restrict__ pd,
-                                                    const FOp *__restrict__ ops, const FGen *__restrict__ gens,
-                                                    double *__restrict__ partials, uint64_t bra_zmask,
-                                                    int bra_from_lam) {
-    fused_adj_body<R, 4, Lv>(lam_in, lam, bra, ntiles, chunk, pd, ops, gens, partials, bra_zmask, bra_from_lam);
+__global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 3 : 1) void k_fused_adj4(
+    const AdjArrays *__restrict__ arrays, uint64_t ntiles, uint64_t chunk, const PassDesc *__restrict__ pd,
+    const FOp *__restrict__ ops, const FGen *__restrict__ gens, double *__restrict__ partials, uint64_t partials_stride,
+    int from_src, int bra_from_lam) {
+    fused_adj_body<R, 4, Lv>(arrays, ntiles, chunk, pd, ops, gens, partials, partials_stride, from_src, bra_from_lam);
 }
 
-// slot sums -> jac[col[s]] * factor[s]
-__global__ __launch_bounds__(kBlock) void k_slot_store(const double *__restrict__ partials, int nparts, int nslots,
+// slot sums -> jac[row][col[s]] * factor[s]; blockIdx.y: the sweep
+__global__ __launch_bounds__(kBlock) void k_slot_store(const double *__restrict__ partials_all,
+                                                       uint64_t partials_stride, int nparts, int nslots,
                                                        const int64_t *__restrict__ cols,
-                                                       const double *__restrict__ factors, double *__restrict__ jac) {
+                                                       const double *__restrict__ factors,
+                                                       const AdjArrays *__restrict__ arrays) {
     __shared__ double sh[kWavesPerBlock];
     const int s = blockIdx.x;
     if (s >= nslots) return;
+    const double *__restrict__ partials = partials_all + blockIdx.y * partials_stride;
+    double *__restrict__ jac = arrays[blockIdx.y].jac_row;
     double v = 0.0;
     for (int b = threadIdx.x; b < nparts; b += kBlock) v += partials[size_t(s) * nparts + b];
     v = wave_sum(v);
@@ -1183,43 +1200,33 @@ FusionPlan plan_passes(const lgh_op *ops, int64_t num_ops, int n, bool adjoint, 
     return plan;
 }
 
-template <class R>
-static void adjoint_one(lgh_sv *lam, const void *lam_src, lgh_sv *bra, const std::vector<KOp> &udag,
-                        const std::vector<KGen> &gens, const std::vector<int> &slot_col,
-                        const std::vector<double> &factor, double *jac_row_dev, double *partials,
-                        StandaloneStep standalone, const BraFromZ *bra_z) {
-    // `udag` lists the ops in forward order with U^dagger matrices; the passes
-    // are scheduled on that order and executed backwards.
-    StreamCtx *ctx = lam->ctx;
-    const int n = lam->n;
-    const FusedCfg cfg = fused_cfg(lam->device, n, lam->dtype, 1);
-    const int rb = cfg.rb;
+// The passes are scheduled on the forward order and executed backwards.
+AdjPasses::AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std::vector<KGen> &gens,
+                     const std::vector<int> &slot_col, const std::vector<double> &factor)
+    : udag_(udag), gens_(gens), slot_col_(slot_col), factor_(factor), ctx_(like->ctx), n_(like->n),
+      device_(like->device), dtype_(like->dtype) {
+    const FusedCfg cfg = fused_cfg(device_, n_, dtype_, 1);
+    rb_ = cfg.rb;
+    waves_per_cu_ = cfg.waves_per_cu;
     // the kernel's LDS holds adj_slot_cap(rb) slots
-    const auto passes = schedule_passes_cached(udag, n, slot_col, rb, fixed_lanes(lam->dtype),
-                                               std::min(cfg.slots, adj_slot_cap(rb)));
-    const Geometry geo = geometry(n, lam->device, rb, cfg.waves_per_cu, g_waves_adj.load());
-    // lambda still to be read from lam_src (until the first pass has run)
-    const void *src = lam_src;
-    // the observable state still to be formed from lambda (first pass only)
-    bool bra_pending = bra_z != nullptr;
+    const auto passes = schedule_passes_cached(udag, n_, slot_col, rb_, fixed_lanes(dtype_),
+                                               std::min(cfg.slots, adj_slot_cap(rb_)));
+    std::vector<unsigned char> blob;
+    auto put = [&](const void *src, size_t bytes) {
+        const size_t at = blob.size();
+        blob.resize(at + ((bytes + 255) & ~size_t(255)));
+        if (bytes) std::memcpy(blob.data() + at, src, bytes);
+        return at;
+    };
     for (auto it = passes->rbegin(); it != passes->rend(); ++it) {
-        const Pass &p = *it;
-        if (p.standalone) {
-            if (bra_pending) {
-                bra_z->materialize(); // before lambda's first change
-                bra_pending = false;
-            }
-            if (src) {
-                LGH_HIP(hipMemcpyAsync(lam->data, src, lam->bytes, hipMemcpyDeviceToDevice, ctx->stream));
-                src = nullptr;
-            }
-            const int i = p.ops[0];
-            standalone(udag[size_t(i)], slot_col[size_t(i)] >= 0 ? &gens[size_t(i)] : nullptr, slot_col[size_t(i)],
-                       factor[size_t(i)]);
+        Step st;
+        if (it->standalone) {
+            st.op = it->ops[0];
+            steps_.push_back(st);
             continue;
         }
-        Built b = build_pass(p, udag, n, true, &gens, &slot_col, rb, true, true, lam->dtype == LGH_C64);
-        LGH_REQUIRE(b.pd.nslots <= adj_slot_cap(rb), "fused adjoint pass: more trainable gates than LDS slots");
+        const Built b = build_pass(*it, udag, n_, true, &gens, &slot_col, rb_, true, true, dtype_ == LGH_C64);
+        LGH_REQUIRE(b.pd.nslots <= adj_slot_cap(rb_), "fused adjoint pass: more trainable gates than LDS slots");
         std::vector<int64_t> cols;
         std::vector<double> facs;
         for (size_t s = 0; s < b.slot_ops.size(); ++s) {
@@ -1227,51 +1234,94 @@ static void adjoint_one(lgh_sv *lam, const void *lam_src, lgh_sv *bra, const std
             cols.push_back(slot_col[size_t(oi)]);
             facs.push_back(factor[size_t(oi)] * b.slot_scale[s]);
         }
-        const size_t pb = (sizeof(PassDesc) + 255) & ~size_t(255);
-        const size_t ob = (b.ops.size() * sizeof(FOp) + 255) & ~size_t(255);
-        const size_t gb = (b.gens.size() * sizeof(FGen) + 255) & ~size_t(255);
-        const size_t cb = (cols.size() * 8 + 255) & ~size_t(255);
-        std::vector<unsigned char> blob(pb + ob + gb + 2 * cb + 256);
-        std::memcpy(blob.data(), &b.pd, sizeof(PassDesc));
-        std::memcpy(blob.data() + pb, b.ops.data(), b.ops.size() * sizeof(FOp));
-        std::memcpy(blob.data() + pb + ob, b.gens.data(), b.gens.size() * sizeof(FGen));
-        std::memcpy(blob.data() + pb + ob + gb, cols.data(), cols.size() * 8);
-        std::memcpy(blob.data() + pb + ob + gb + cb, facs.data(), facs.size() * 8);
-        unsigned char *d = static_cast<unsigned char *>(ctx->upload(blob.data(), blob.size()));
+        st.o_desc = put(&b.pd, sizeof(PassDesc));
+        st.o_ops = put(b.ops.data(), b.ops.size() * sizeof(FOp));
+        st.o_gens = put(b.gens.data(), b.gens.size() * sizeof(FGen));
+        st.o_cols = put(cols.data(), cols.size() * 8);
+        st.o_facs = put(facs.data(), facs.size() * 8);
+        st.nslots = int(cols.size());
+        st.level = g_lean.load() ? lean_level(b.ops, true) : 0;
+        steps_.push_back(st);
+    }
+    if (blob.empty()) return;
+    bytes_ = blob.size();
+    dev_ = static_cast<unsigned char *>(pool_alloc(device_, bytes_));
+    try {
+        ctx_->copy_in(dev_, blob.data(), bytes_);
+    } catch (...) {
+        pool_free(device_, dev_, bytes_);
+        throw;
+    }
+}
+
+AdjPasses::~AdjPasses() {
+    if (!dev_) return;
+    (void)hipStreamSynchronize(ctx_->stream);
+    pool_free(device_, dev_, bytes_);
+}
+
+template <class R>
+void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void *table,
+                      const StandaloneStep &standalone) const {
+    static_assert(sizeof(AdjArrays) <= kTableBytes, "a table entry per sweep");
+    const Geometry geo = geometry(n_, device_, rb_, waves_per_cu_, g_waves_adj.load());
+    const uint64_t stride = fused_partials_bytes(n_, device_) / sizeof(double);
+    std::vector<AdjArrays> tab;
+    bool src = false, from_z = false;
+    for (int j = 0; j < count; ++j) {
+        const AdjSweep &s = sweeps[j];
+        tab.push_back({s.lam_src ? s.lam_src : s.lam->data, s.lam->data, s.bra->data, s.zmask, s.jac_row});
+        src |= s.lam_src != nullptr;
+        LGH_REQUIRE(j == 0 || s.bra_from_z == from_z, "adjoint sweeps side by side must be of one kind");
+        from_z = s.bra_from_z;
+    }
+    ctx_->copy_in(table, tab.data(), tab.size() * sizeof(AdjArrays));
+    const AdjArrays *dtab = static_cast<const AdjArrays *>(table);
+    for (const Step &st : steps_) {
+        if (st.op >= 0) {
+            for (int j = 0; j < count; ++j) {
+                const AdjSweep &s = sweeps[j];
+                if (from_z) s.materialize(); // before lambda's first change
+                if (src && s.lam_src)
+                    LGH_HIP(hipMemcpyAsync(s.lam->data, s.lam_src, s.lam->bytes, hipMemcpyDeviceToDevice, ctx_->stream));
+                const size_t i = size_t(st.op);
+                standalone(s, udag_[i], slot_col_[i] >= 0 ? &gens_[i] : nullptr, slot_col_[i], factor_[i]);
+            }
+            from_z = src = false;
+            continue;
+        }
         {
-            ProfScope prof(kProfFusedAdj, ctx->stream);
-            const int lv = g_lean.load() ? lean_level(b.ops, true) : 0;
-            auto kern = rb == 4 ? (lv == 1 ? k_fused_adj4<R, 1> : lv == 2 ? k_fused_adj4<R, 2> : k_fused_adj4<R>)
-                                : (lv == 1 ? k_fused_adj3<R, 1> : lv == 2 ? k_fused_adj3<R, 2> : k_fused_adj3<R>);
-            const cx<R> *lam_in = static_cast<const cx<R> *>(src ? src : lam->data);
-            src = nullptr;
-            const uint64_t zmask = bra_pending ? bra_z->zmask : 0ull;
-            hipLaunchKernelGGL(kern, dim3(geo.blocks), dim3(kBlock), 0, ctx->stream, lam_in,
-                               static_cast<cx<R> *>(lam->data), static_cast<cx<R> *>(bra->data), geo.ntiles,
-                               geo.chunk, reinterpret_cast<const PassDesc *>(d), reinterpret_cast<const FOp *>(d + pb),
-                               reinterpret_cast<const FGen *>(d + pb + ob), partials, zmask, int(bra_pending));
-            bra_pending = false;
+            ProfScope prof(kProfFusedAdj, ctx_->stream);
+            auto kern = rb_ == 4 ? (st.level == 1   ? k_fused_adj4<R, 1>
+                                    : st.level == 2 ? k_fused_adj4<R, 2>
+                                                    : k_fused_adj4<R>)
+                                 : (st.level == 1   ? k_fused_adj3<R, 1>
+                                    : st.level == 2 ? k_fused_adj3<R, 2>
+                                                    : k_fused_adj3<R>);
+            hipLaunchKernelGGL(kern, dim3(geo.blocks, unsigned(count)), dim3(kBlock), 0, ctx_->stream, dtab, geo.ntiles,
+                               geo.chunk, reinterpret_cast<const PassDesc *>(dev_ + st.o_desc),
+                               reinterpret_cast<const FOp *>(dev_ + st.o_ops),
+                               reinterpret_cast<const FGen *>(dev_ + st.o_gens), partials, stride, int(src),
+                               int(from_z));
+            from_z = src = false;
             LGH_LAUNCH_CHECK();
         }
-        if (!cols.empty()) {
-            hipLaunchKernelGGL(k_slot_store, dim3(unsigned(cols.size())), dim3(kBlock), 0, ctx->stream, partials,
-                               int(geo.blocks), int(cols.size()), reinterpret_cast<const int64_t *>(d + pb + ob + gb),
-                               reinterpret_cast<const double *>(d + pb + ob + gb + cb), jac_row_dev);
+        if (st.nslots > 0) {
+            hipLaunchKernelGGL(k_slot_store, dim3(unsigned(st.nslots), unsigned(count)), dim3(kBlock), 0, ctx_->stream,
+                               partials, stride, int(geo.blocks), st.nslots,
+                               reinterpret_cast<const int64_t *>(dev_ + st.o_cols),
+                               reinterpret_cast<const double *>(dev_ + st.o_facs), dtab);
             LGH_LAUNCH_CHECK();
         }
     }
 }
 
-void fused_adjoint_one(lgh_sv *lam, const void *lam_src, lgh_sv *bra, const std::vector<KOp> &udag,
-                       const std::vector<KGen> &gens, const std::vector<int> &slot_col,
-                       const std::vector<double> &factor, double *jac_row_dev, double *partials,
-                       StandaloneStep standalone, const BraFromZ *bra_z) {
-    if (lam->dtype == LGH_C128)
-        adjoint_one<double>(lam, lam_src, bra, udag, gens, slot_col, factor, jac_row_dev, partials, standalone,
-                            bra_z);
+void AdjPasses::run(const AdjSweep *sweeps, int count, double *partials, void *table,
+                    const StandaloneStep &standalone) const {
+    if (dtype_ == LGH_C128)
+        run_t<double>(sweeps, count, partials, table, standalone);
     else
-        adjoint_one<float>(lam, lam_src, bra, udag, gens, slot_col, factor, jac_row_dev, partials, standalone,
-                           bra_z);
+        run_t<float>(sweeps, count, partials, table, standalone);
 }
 
 size_t fused_partials_bytes(int n, int device) {

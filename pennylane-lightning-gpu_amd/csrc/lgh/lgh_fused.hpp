@@ -58,27 +58,60 @@ FusionPlan plan_passes(const lgh_op *ops, int64_t num_ops, int n, bool adjoint, 
 // Forward application of a compiled op list through fused passes.
 void fused_apply(lgh_sv *sv, const std::vector<KOp> &kops);
 
-// Applies U^dagger of one non-fusable gate to lambda and the observable
-// state; with a generator, stores factor * Im<bra|G lambda> into jac_row[col].
-using StandaloneStep = std::function<void(const KOp &udag, const KGen *gen, int64_t col, double factor)>;
-
-// An observable state that the sweep forms itself: bra = Z-word(zmask)
-// lambda, inside the first reverse pass when that pass is fused; otherwise
-// `materialize` forms it before lambda first changes.
-struct BraFromZ {
-    uint64_t zmask;
+// One observable's reverse sweep.
+struct AdjSweep {
+    lgh_sv *lam;         // lambda: written by every pass
+    const void *lam_src; // where the first pass reads it (null: lam's own contents)
+    lgh_sv *bra;         // the observable's state
+    double *jac_row;     // device row of the Jacobian
+    // An observable state that the sweep forms itself: bra = Z-word(zmask)
+    // lambda, inside the first reverse pass when that pass is fused; otherwise
+    // `materialize` forms it before lambda first changes.
+    bool bra_from_z = false;
+    uint64_t zmask = 0;
     std::function<void()> materialize;
 };
 
-// Reverse sweep of one observable state through fused passes.  udag: the
-// ops in forward order compiled as U^dagger; slot_col[i]: Jacobian column of
-// a trainable gate or -1; factor[i] = -2 s (inverse ? -1 : 1).  lam_src: if
-// not null, lambda's starting values, read by the first pass (or copied
-// before a first standalone step) instead of lam's own contents.
-void fused_adjoint_one(lgh_sv *lam, const void *lam_src, lgh_sv *bra, const std::vector<KOp> &udag,
-                       const std::vector<KGen> &gens, const std::vector<int> &slot_col,
-                       const std::vector<double> &factor, double *jac_row_dev, double *partials,
-                       StandaloneStep standalone, const BraFromZ *bra_z = nullptr);
+// Applies U^dagger of one non-fusable gate to a sweep's lambda and observable
+// state; with a generator, stores factor * Im<bra|G lambda> into jac_row[col].
+using StandaloneStep =
+    std::function<void(const AdjSweep &sweep, const KOp &udag, const KGen *gen, int64_t col, double factor)>;
+
+// The fused reverse passes of a circuit: scheduled, built and uploaded once,
+// run for any number of sweeps.  udag: the ops in forward order compiled as
+// U^dagger; slot_col[i]: Jacobian column of a trainable gate or -1;
+// factor[i] = -2 s (inverse ? -1 : 1).
+class AdjPasses {
+  public:
+    AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std::vector<KGen> &gens,
+              const std::vector<int> &slot_col, const std::vector<double> &factor);
+    ~AdjPasses();
+    AdjPasses(const AdjPasses &) = delete;
+    // Runs the sweeps side by side, one launch per pass for all of them.
+    // partials: count * fused_partials_bytes() bytes; table: count *
+    // kTableBytes bytes, both on the device and the call's own.
+    static constexpr size_t kTableBytes = 64;
+    void run(const AdjSweep *sweeps, int count, double *partials, void *table, const StandaloneStep &standalone) const;
+
+  private:
+    struct Step {
+        int op = -1;              // a standalone gate, or -1
+        size_t o_ops = 0, o_gens = 0, o_cols = 0, o_facs = 0, o_desc = 0;
+        int nslots = 0, level = 0;
+    };
+    template <class R>
+    void run_t(const AdjSweep *sweeps, int count, double *partials, void *table, const StandaloneStep &s) const;
+    const std::vector<KOp> &udag_;
+    const std::vector<KGen> &gens_;
+    const std::vector<int> &slot_col_;
+    const std::vector<double> &factor_;
+    StreamCtx *ctx_;
+    int n_, device_, rb_, waves_per_cu_;
+    lgh_dtype dtype_;
+    std::vector<Step> steps_;     // in execution order
+    unsigned char *dev_ = nullptr; // descriptors of every pass
+    size_t bytes_ = 0;
+};
 size_t fused_partials_bytes(int n, int device);
 
 } // namespace lgh

@@ -247,12 +247,16 @@ struct StreamCtx {
     size_t up_bytes = 0;
     size_t up_off = 0;
 
+    void ring_room(size_t need);
     void *workspace(size_t bytes);
     void *host_buffer(size_t bytes);
     // Copies `bytes` from host memory into the device ring (stream ordered)
     // and returns the device address.  Valid until the ring wraps, which
     // synchronises the stream first.
     void *upload(const void *src, size_t bytes);
+    // Copies host memory to `dst` on the device, stream ordered; `src` may be
+    // changed or freed afterwards.
+    void copy_in(void *dst, const void *src, size_t bytes);
     void sync();
 };
 

@@ -277,9 +277,8 @@ void *StreamCtx::host_buffer(size_t bytes) {
     return host;
 }
 
-void *StreamCtx::upload(const void *src, size_t bytes) {
-    const size_t need = (bytes + 255) & ~size_t(255);
-    DeviceGuard g(device);
+// Room for `need` bytes in the upload ring, at up_off.
+void StreamCtx::ring_room(size_t need) {
     if (need > up_bytes) {
         sync();
         if (up_host) LGH_HIP(hipHostFree(up_host));
@@ -295,12 +294,33 @@ void *StreamCtx::upload(const void *src, size_t bytes) {
         sync(); // every earlier copy out of the ring has completed
         up_off = 0;
     }
+}
+
+void *StreamCtx::upload(const void *src, size_t bytes) {
+    const size_t need = (bytes + 255) & ~size_t(255);
+    DeviceGuard g(device);
+    ring_room(need);
     char *h = static_cast<char *>(up_host) + up_off;
     char *d = static_cast<char *>(up_dev) + up_off;
     std::memcpy(h, src, bytes);
     LGH_HIP(hipMemcpyAsync(d, h, bytes, hipMemcpyHostToDevice, stream));
     up_off += need;
     return d;
+}
+
+void StreamCtx::copy_in(void *dst, const void *src, size_t bytes) {
+    const size_t need = (bytes + 255) & ~size_t(255);
+    DeviceGuard g(device);
+    if (need > (size_t(1) << 20)) { // too large for the ring: wait for the copy out of pageable memory
+        LGH_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, stream));
+        sync();
+        return;
+    }
+    ring_room(need);
+    char *h = static_cast<char *>(up_host) + up_off;
+    std::memcpy(h, src, bytes);
+    LGH_HIP(hipMemcpyAsync(dst, h, bytes, hipMemcpyHostToDevice, stream));
+    up_off += need;
 }
 
 } // namespace lgh
