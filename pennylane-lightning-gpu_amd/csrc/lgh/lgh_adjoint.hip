@@ -241,6 +241,63 @@ __global__ __launch_bounds__(kBlock) void k_adj_diag(cx<R> *__restrict__ psi, cx
         for (int j = 0; j < nb; ++j) partials[size_t(j) * gridDim.x + blockIdx.x] = acc[j];
 }
 
+// The step for a gate that mixes pairs of basis states (KOp::npair): reads and
+// writes the pairs' amplitudes only, in the order of operations of k_adj_dense;
+// blockIdx.y: the sweep, each with a lambda and an observable state of its own.
+// A double excitation on 18 qubits: k_adj_dense 21 us and two more launches
+// for its sum (8 us), 4.4 us here, the sums of a run of gates stored together.
+template <class R> struct PairGen {
+    cx<double> g[2][4];
+};
+template <class R, int NP>
+__global__ __launch_bounds__(kBlock) void k_adj_pairs(const AdjArrays *__restrict__ table, PairArgs<R> p, PairGen<R> gen,
+                                                      int with_gen, double *__restrict__ partials, uint64_t stride) {
+    const AdjArrays &ar = table[blockIdx.y];
+    cx<R> *psi = static_cast<cx<R> *>(ar.lam), *bra = static_cast<cx<R> *>(ar.bra);
+    double acc[1] = {0.0};
+    const uint64_t g = xcd_block() * kBlock + threadIdx.x;
+    if (g < p.ngroups) {
+        const uint64_t base = expand(g, p.fx) | p.cmask;
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            const uint64_t i = base | p.lo[q], j = base | p.hi[q];
+            const cx<R> a0 = ldnt(psi + i), a1 = ldnt(psi + j), b0 = ldnt(bra + i), b1 = ldnt(bra + j);
+            const cx<R> *m = p.m[q];
+            if (with_gen) {
+                const cx<double> *gm = gen.g[q];
+                acc[0] += im_dot(b0, cfma(gm[1], up(a1), cmul(gm[0], up(a0))));
+                acc[0] += im_dot(b1, cfma(gm[3], up(a1), cmul(gm[2], up(a0))));
+            }
+            stnt(bra + i, cfma(m[1], b1, cmul(m[0], b0)));
+            stnt(bra + j, cfma(m[3], b1, cmul(m[2], b0)));
+            stnt(psi + i, cfma(m[1], a1, cmul(m[0], a0)));
+            stnt(psi + j, cfma(m[3], a1, cmul(m[2], a0)));
+        }
+    }
+    if (!with_gen) return;
+    block_sum<1>(acc);
+    if (threadIdx.x == 0) partials[blockIdx.y * stride + blockIdx.x] = acc[0];
+}
+
+template <class R>
+void adj_pairs_t(StreamCtx *ctx, int n, const KOp &udag, const KGen *gen, const AdjArrays *table, int count,
+                 double *partials, uint64_t stride) {
+    const PairArgs<R> p = pair_args<R>(udag, n);
+    PairGen<R> pg{};
+    const size_t D = size_t(1) << udag.k;
+    for (int q = 0; gen && q < udag.npair; ++q) {
+        const size_t r = size_t(udag.pair_row[q]), s = r ^ size_t(udag.pair_flip);
+        pg.g[q][0] = to_cx<double>(gen->mat[r * D + r]);
+        pg.g[q][1] = to_cx<double>(gen->mat[r * D + s]);
+        pg.g[q][2] = to_cx<double>(gen->mat[s * D + r]);
+        pg.g[q][3] = to_cx<double>(gen->mat[s * D + s]);
+    }
+    auto kern = udag.npair == 1 ? k_adj_pairs<R, 1> : k_adj_pairs<R, 2>;
+    hipLaunchKernelGGL(kern, dim3(unsigned((p.ngroups + kBlock - 1) / kBlock), unsigned(count)), dim3(kBlock), 0,
+                       ctx->stream, table, p, pg, int(gen != nullptr), partials, stride);
+    LGH_LAUNCH_CHECK();
+}
+
 // Row sums of the per-workgroup partials in two deterministic stages:
 // k_row_chunks sums fixed contiguous slices of each row (grid: slices x rows),
 // k_jac_store sums the slice results of row j and scales them into the
@@ -611,6 +668,23 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
 }
 
 } // namespace
+
+namespace lgh {
+
+unsigned adj_pairs_blocks(int n, const KOp &udag) {
+    const uint64_t groups = 1ull << (n - udag.k - int(udag.cbits.size()));
+    return unsigned((groups + kBlock - 1) / kBlock);
+}
+
+void launch_adj_pairs(StreamCtx *ctx, lgh_dtype dtype, int n, const KOp &udag, const KGen *gen,
+                      const AdjArrays *table, int count, double *partials, uint64_t stride) {
+    if (dtype == LGH_C128)
+        adj_pairs_t<double>(ctx, n, udag, gen, table, count, partials, stride);
+    else
+        adj_pairs_t<float>(ctx, n, udag, gen, table, count, partials, stride);
+}
+
+} // namespace lgh
 
 extern "C" {
 

@@ -469,13 +469,7 @@ __global__ __launch_bounds__(kBlock) void k_fused_pass(cx<R> *__restrict__ sv, u
     }
 }
 
-// One sweep's arrays (device table, one entry per blockIdx.y).
-struct AdjArrays {
-    const void *lam_src; // lambda's starting values
-    void *lam, *bra;
-    uint64_t zmask;
-    double *jac_row;
-};
+// (blockIdx.y: the sweep)
 typedef __attribute__((address_space(4))) const AdjArrays CAdjArrays;
 
 // Reverse pass of the adjoint sweep on lambda and one observable state; the
@@ -1221,7 +1215,37 @@ AdjPasses::AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std
     for (auto it = passes->rbegin(); it != passes->rend(); ++it) {
         Step st;
         if (it->standalone) {
-            st.op = it->ops[0];
+            const int i = it->ops[0];
+            if (udag[size_t(i)].npair == 0) {
+                st.op = i;
+            } else {
+                // a run's partial sums, a row of one double per workgroup for
+                // every trainable gate, fit the partials of a fused pass
+                size_t room = fused_partials_bytes(n_, device_) / sizeof(double);
+                for (auto next = it; next != passes->rend() && next->standalone; ++next) {
+                    const size_t g = size_t(next->ops[0]);
+                    if (udag[g].npair == 0) break;
+                    if (slot_col[g] >= 0) {
+                        const unsigned blocks = adj_pairs_blocks(n_, udag[g]);
+                        if (blocks > room || (st.blocks && blocks != st.blocks)) break;
+                        st.blocks = blocks;
+                        room -= blocks;
+                    }
+                    st.pairs.push_back(int(g));
+                    it = next;
+                }
+                if (st.pairs.empty()) st.op = i;
+            }
+            std::vector<int64_t> cols;
+            std::vector<double> facs;
+            for (int g : st.pairs)
+                if (slot_col[size_t(g)] >= 0) {
+                    cols.push_back(slot_col[size_t(g)]);
+                    facs.push_back(factor[size_t(g)]);
+                }
+            st.nslots = int(cols.size());
+            st.o_cols = put(cols.data(), cols.size() * 8);
+            st.o_facs = put(facs.data(), facs.size() * 8);
             steps_.push_back(st);
             continue;
         }
@@ -1277,17 +1301,42 @@ void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void 
     }
     ctx_->copy_in(table, tab.data(), tab.size() * sizeof(AdjArrays));
     const AdjArrays *dtab = static_cast<const AdjArrays *>(table);
+    auto store = [&](const Step &st, unsigned blocks) {
+        if (st.nslots == 0) return;
+        hipLaunchKernelGGL(k_slot_store, dim3(unsigned(st.nslots), unsigned(count)), dim3(kBlock), 0, ctx_->stream,
+                           partials, stride, int(blocks), st.nslots,
+                           reinterpret_cast<const int64_t *>(dev_ + st.o_cols),
+                           reinterpret_cast<const double *>(dev_ + st.o_facs), dtab);
+        LGH_LAUNCH_CHECK();
+    };
+    // the sweeps' own lambda and observable states, where a pass would read them elsewhere or form them
+    auto settle = [&] {
+        for (int j = 0; j < count; ++j) {
+            const AdjSweep &s = sweeps[j];
+            if (from_z) s.materialize(); // before lambda's first change
+            if (src && s.lam_src)
+                LGH_HIP(hipMemcpyAsync(s.lam->data, s.lam_src, s.lam->bytes, hipMemcpyDeviceToDevice, ctx_->stream));
+        }
+        from_z = src = false;
+    };
     for (const Step &st : steps_) {
-        if (st.op >= 0) {
-            for (int j = 0; j < count; ++j) {
-                const AdjSweep &s = sweeps[j];
-                if (from_z) s.materialize(); // before lambda's first change
-                if (src && s.lam_src)
-                    LGH_HIP(hipMemcpyAsync(s.lam->data, s.lam_src, s.lam->bytes, hipMemcpyDeviceToDevice, ctx_->stream));
-                const size_t i = size_t(st.op);
-                standalone(s, udag_[i], slot_col_[i] >= 0 ? &gens_[i] : nullptr, slot_col_[i], factor_[i]);
+        if (!st.pairs.empty()) {
+            settle();
+            uint64_t row = 0;
+            for (int i : st.pairs) {
+                const bool train = slot_col_[size_t(i)] >= 0;
+                launch_adj_pairs(ctx_, dtype_, n_, udag_[size_t(i)], train ? &gens_[size_t(i)] : nullptr, dtab, count,
+                                 partials + row, stride);
+                if (train) row += st.blocks;
             }
-            from_z = src = false;
+            store(st, st.blocks);
+            continue;
+        }
+        if (st.op >= 0) {
+            settle();
+            const size_t i = size_t(st.op);
+            for (int j = 0; j < count; ++j)
+                standalone(sweeps[j], udag_[i], slot_col_[i] >= 0 ? &gens_[i] : nullptr, slot_col_[i], factor_[i]);
             continue;
         }
         {
@@ -1306,13 +1355,7 @@ void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void 
             from_z = src = false;
             LGH_LAUNCH_CHECK();
         }
-        if (st.nslots > 0) {
-            hipLaunchKernelGGL(k_slot_store, dim3(unsigned(st.nslots), unsigned(count)), dim3(kBlock), 0, ctx_->stream,
-                               partials, stride, int(geo.blocks), st.nslots,
-                               reinterpret_cast<const int64_t *>(dev_ + st.o_cols),
-                               reinterpret_cast<const double *>(dev_ + st.o_facs), dtab);
-            LGH_LAUNCH_CHECK();
-        }
+        store(st, geo.blocks);
     }
 }
 

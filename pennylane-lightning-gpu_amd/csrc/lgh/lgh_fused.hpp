@@ -72,6 +72,22 @@ struct AdjSweep {
     std::function<void()> materialize;
 };
 
+// One sweep's arrays (device table, one entry per sweep of a launch).
+struct AdjArrays {
+    const void *lam_src; // lambda's starting values
+    void *lam, *bra;
+    uint64_t zmask;
+    double *jac_row;
+};
+
+// A reverse step of a gate that mixes pairs of basis states (KOp::npair), on
+// lambda and the observable state of `count` sweeps (lgh_adjoint.hip): with a
+// generator, workgroup b of sweep y leaves its share of Im<bra|G lambda> in
+// partials[y * stride + b].
+unsigned adj_pairs_blocks(int n, const KOp &udag);
+void launch_adj_pairs(StreamCtx *ctx, lgh_dtype dtype, int n, const KOp &udag, const KGen *gen,
+                      const AdjArrays *table, int count, double *partials, uint64_t stride);
+
 // Applies U^dagger of one non-fusable gate to a sweep's lambda and observable
 // state; with a generator, stores factor * Im<bra|G lambda> into jac_row[col].
 using StandaloneStep =
@@ -94,8 +110,12 @@ class AdjPasses {
     void run(const AdjSweep *sweeps, int count, double *partials, void *table, const StandaloneStep &standalone) const;
 
   private:
+    // A fused pass, a gate on its own, or a run of gates that mix pairs of
+    // basis states, whose overlaps are summed and stored together at its end.
     struct Step {
-        int op = -1;              // a standalone gate, or -1
+        std::vector<int> pairs;   // that run's gates, in execution order
+        int op = -1;              // a gate on its own, or -1
+        unsigned blocks = 0;      // workgroups of each of the run's trainable gates
         size_t o_ops = 0, o_gens = 0, o_cols = 0, o_facs = 0, o_desc = 0;
         int nslots = 0, level = 0;
     };

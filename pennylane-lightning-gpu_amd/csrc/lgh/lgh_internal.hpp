@@ -347,7 +347,48 @@ struct KOp {
     std::vector<std::complex<double>> mat;
     uint64_t pmask = 0;
     std::complex<double> d_even{1, 0}, d_odd{1, 0};
+    // DENSE on two and more targets that mixes only pairs of basis states,
+    // (r, r ^ pair_flip) for the npair matrix rows r of pair_row, and leaves
+    // all others alone (excitations, swaps, IsingXX / YY).
+    int npair = 0;
+    int pair_row[2] = {0, 0};
+    int pair_flip = 0;
 };
+
+// The pairs of a KOp as kernel arguments: 2x2 matrices on the amplitudes at
+// base | lo[q] and base | hi[q].
+template <class R> struct PairArgs {
+    Fixed fx;        // targets and controls
+    uint64_t cmask;
+    uint64_t ngroups;
+    uint64_t lo[2], hi[2];
+    cx<R> m[2][4];
+};
+template <class R> PairArgs<R> pair_args(const KOp &op, int n) {
+    PairArgs<R> a{};
+    std::vector<int> fixed_bits = op.cbits;
+    auto offset = [&](int row) {
+        uint64_t o = 0;
+        for (int j = 0; j < op.k; ++j)
+            if ((row >> (op.k - 1 - j)) & 1) o |= 1ull << op.tbits[j];
+        return o;
+    };
+    for (int i = 0; i < op.k; ++i) fixed_bits.push_back(op.tbits[i]);
+    a.fx = make_fixed(fixed_bits);
+    a.cmask = op.cmask;
+    a.ngroups = 1ull << (n - a.fx.cnt);
+    const size_t D = size_t(1) << op.k;
+    for (int q = 0; q < op.npair; ++q) {
+        const size_t r = size_t(op.pair_row[q]), s = r ^ size_t(op.pair_flip);
+        a.lo[q] = offset(int(r));
+        a.hi[q] = offset(int(s));
+        a.m[q][0] = to_cx<R>(op.mat[r * D + r]);
+        a.m[q][1] = to_cx<R>(op.mat[r * D + s]);
+        a.m[q][2] = to_cx<R>(op.mat[s * D + r]);
+        a.m[q][3] = to_cx<R>(op.mat[s * D + s]);
+    }
+    return a;
+}
 
 // Generator data aligned with a KOp of the same op: for DENSE a 2^k x 2^k
 // matrix on the same targets (restricted to the control subspace), for DIAG
