@@ -249,6 +249,16 @@ lgh_status lgh_scale(lgh_sv *x, double alpha_re, double alpha_im);
 lgh_status lgh_sv_pauli_word_from(lgh_sv *dst, const lgh_sv *src, const char *paulis, const int32_t *wires,
                                   int32_t num_wires);
 
+/* dst = sum_w coeffs[w] P_w src for Pauli words as in lgh_expval_pauli_words
+ * (word w is paulis[offsets[w]..offsets[w+1]) on the wires at the same
+ * positions; real coefficients); dst and src are different states of the same
+ * size.  The words are grouped into passes over the state as for the
+ * expectation.  It replaces one copy, gate sequence and axpy per term when the
+ * adjoint Jacobian forms H|lambda> for a Hamiltonian (ObservablesGPU.hpp:290-
+ * 420); no single reference function corresponds to it. */
+lgh_status lgh_sv_pauli_sum_from(lgh_sv *dst, const lgh_sv *src, int64_t num_words, const char *paulis,
+                                 const int32_t *wires, const int64_t *offsets, const double *coeffs);
+
 /* ---- measurements (SVCM:702-1148) ------------------------------------ */
 /* expval(wires, matrix) / getExpectationValueDeviceMatrix (SVCM:755-780, :1649-1713) */
 lgh_status lgh_expval_matrix(const lgh_sv *sv, const int32_t *wires, int32_t num_wires,

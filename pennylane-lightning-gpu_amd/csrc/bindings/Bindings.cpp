@@ -374,7 +374,8 @@ template <class PrecisionT, class ParamT> void bind_precision(py::module_ &m) {
         });
 
     using Adj = AdjointJacobianHIP<PrecisionT>;
-    py::class_<Adj>(m, ("AdjointJacobianGPU_C" + bits).c_str(), py::module_local())
+    py::class_<Adj> adj_cls(m, ("AdjointJacobianGPU_C" + bits).c_str(), py::module_local());
+    adj_cls
         .def(py::init<>())
         .def("create_ops_list",
              [](Adj &, const std::vector<std::string> &names, const std::vector<np_arr_r> &params,
@@ -413,6 +414,19 @@ template <class PrecisionT, class ParamT> void bind_precision(py::module_ &m) {
                  }
                  return py::array_t<ParamT>(py::cast(jac));
              });
+    // rows [offsets[k], offsets[k + 1]) of `obs` added up in one sweep;
+    // complex128 only, as applySequence
+    if constexpr (std::is_same_v<PrecisionT, double>)
+        adj_cls.def("adjoint_jacobian_summed",
+                    [](Adj &adj, const SV &sv, const std::vector<ObsPtr> &obs, const std::vector<std::size_t> &offsets,
+                       const Ops &ops, const std::vector<std::size_t> &tp) {
+                        std::vector<std::vector<PrecisionT>> jac;
+                        {
+                            py::gil_scoped_release release;
+                            jac = adj.adjointJacobianSummed(sv, obs, offsets, ops, tp);
+                        }
+                        return py::array_t<ParamT>(py::cast(jac));
+                    });
 }
 
 } // namespace

@@ -141,6 +141,38 @@ template <class T> class AdjointJacobianHIP {
         return out;
     }
 
+    // Jacobian rows added up: row k of the result is the sum of the rows of
+    // obs[offsets[k]..offsets[k+1]), found in one sweep of their sum.  For the
+    // rows that the device splits a Hamiltonian into.
+    std::vector<std::vector<T>> adjointJacobianSummed(const StateVectorHIPManaged<T> &sv,
+                                                      const std::vector<ObsPtr> &obs,
+                                                      const std::vector<std::size_t> &offsets, const OpsData<T> &ops,
+                                                      const std::vector<std::size_t> &trainable) const {
+        PL_HIP_ABORT_IF(offsets.empty() || offsets.front() != 0 || offsets.back() != obs.size(),
+                        "Row offsets do not match the observables");
+        std::vector<ObsPtr> sums;
+        for (std::size_t k = 0; k + 1 < offsets.size(); ++k) {
+            PL_HIP_ABORT_IF(offsets[k] > offsets[k + 1], "Row offsets must not decrease");
+            if (offsets[k + 1] - offsets[k] == 1) {
+                sums.push_back(obs[offsets[k]]);
+                continue;
+            }
+            std::vector<T> coeffs;
+            std::vector<ObsPtr> terms;
+            for (std::size_t r = offsets[k]; r < offsets[k + 1]; ++r) {
+                if (auto h = std::dynamic_pointer_cast<HamiltonianHIP<T>>(obs[r])) {
+                    coeffs.insert(coeffs.end(), h->getCoeffs().begin(), h->getCoeffs().end());
+                    terms.insert(terms.end(), h->getObs().begin(), h->getObs().end());
+                } else {
+                    coeffs.push_back(T(1));
+                    terms.push_back(obs[r]);
+                }
+            }
+            sums.push_back(std::make_shared<HamiltonianHIP<T>>(std::move(coeffs), std::move(terms)));
+        }
+        return adjointJacobian(sv, sums, ops, trainable, false);
+    }
+
     // batchAdjointJacobian (AdjointDiffGPU.hpp:392-473): the reference spreads
     // observables over GPUs with one thread each.  With one GPU the
     // observables are processed in chunks that bound the number of resident

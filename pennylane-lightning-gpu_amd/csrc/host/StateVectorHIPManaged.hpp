@@ -182,6 +182,20 @@ class OpBuilder {
     std::vector<std::size_t> mat_index_;
 };
 
+// A real-weighted sum of Pauli words in the layout of the C ABI.
+template <class T> struct PauliSum {
+    std::string letters;
+    std::vector<int32_t> wires;
+    std::vector<int64_t> offsets{0};
+    std::vector<double> coeffs;
+    void add(T coeff, const std::string &word, const std::vector<std::size_t> &word_wires) {
+        letters += word;
+        for (auto w : word_wires) wires.push_back(static_cast<int32_t>(w));
+        offsets.push_back(static_cast<int64_t>(letters.size()));
+        coeffs.push_back(static_cast<double>(coeff));
+    }
+};
+
 template <class PrecisionT> class StateVectorHIPManaged {
   public:
     static_assert(std::is_same_v<PrecisionT, float> || std::is_same_v<PrecisionT, double>);
@@ -270,6 +284,12 @@ template <class PrecisionT> class StateVectorHIPManaged {
                         const std::vector<std::size_t> &wires) {
         std::vector<int32_t> w(wires.begin(), wires.end());
         check(lgh_sv_pauli_word_from(sv_, other.sv_, letters.data(), w.data(), static_cast<int32_t>(w.size())));
+    }
+
+    // this <- sum_w c_w P_w other, in few passes over the state
+    void setPauliSumOf(const StateVectorHIPManaged &other, const PauliSum<PrecisionT> &sum) {
+        check(lgh_sv_pauli_sum_from(sv_, other.sv_, static_cast<int64_t>(sum.coeffs.size()), sum.letters.data(),
+                                    sum.wires.data(), sum.offsets.data(), sum.coeffs.data()));
     }
 
     // ---- gates (SVCM:198-315)

@@ -414,14 +414,21 @@ class LightningGPU:
         params, columns = self._parameter_columns(tape, 1 if has_prep else 0)
 
         batches = self._observable_batches(len(rows))
-        if batches is None:
-            raw = adj.adjoint_jacobian(self._gpu_state, rows, ops, params)
+        summed = getattr(adj, "adjoint_jacobian_summed", None)
+        if batches is None and summed is not None and len(rows) > len(offsets) - 1:
+            # the backend adds up the rows of a split sum in one sweep of the sum
+            per_ob = np.asarray(summed(self._gpu_state, rows, offsets, ops, params), dtype=np.float64)
+            per_ob = per_ob.reshape(len(offsets) - 1, len(params))
         else:
-            raw = [r for b in batches for r in adj.adjoint_jacobian_batched(self._gpu_state, rows[b], ops, params)]
-        per_row = np.asarray(raw, dtype=np.float64).reshape(len(rows), len(params))
-        # rows of one tape observable (a split sum has several) add up
-        per_ob = np.stack([per_row[lo:hi].sum(axis=0) for lo, hi in zip(offsets[:-1], offsets[1:])]) \
-            if len(offsets) > 1 else np.zeros((0, len(params)))
+            if batches is None:
+                raw = adj.adjoint_jacobian(self._gpu_state, rows, ops, params)
+            else:
+                raw = [r for b in batches
+                       for r in adj.adjoint_jacobian_batched(self._gpu_state, rows[b], ops, params)]
+            per_row = np.asarray(raw, dtype=np.float64).reshape(len(rows), len(params))
+            # rows of one tape observable (a split sum has several) add up
+            per_ob = np.stack([per_row[lo:hi].sum(axis=0) for lo, hi in zip(offsets[:-1], offsets[1:])]) \
+                if len(offsets) > 1 else np.zeros((0, len(params)))
         full = np.zeros((len(offsets) - 1, len(tape.trainable_params)))
         full[:, columns] = per_ob
         return self._adjoint_jacobian_processing(full)
