@@ -14,9 +14,8 @@
 // pulled from an atomic counter: |0..0>, the forward passes, bra = P psi
 // with <P> = <psi|bra>, and the reverse passes on (psi, bra) that accumulate
 // d<P>/d theta for every trainable gate.  All passes of a circuit run inside
-// one workgroup, separated by a workgroup barrier and a device-scope fence,
-// so states of up to 2^20 amplitudes stay in L2 / MALL between passes and no
-// circuit waits for a launch.  Circuits below 9 qubits (one 512-amplitude
+// one workgroup, separated by a workgroup barrier, so states of up to 2^20
+// amplitudes stay in L2 / MALL between passes and no circuit waits for a launch.  Circuits below 9 qubits (one 512-amplitude
 // tile) run on 9 qubits with idle low-order wires; their results are those of
 // the smaller circuit.
 //
@@ -160,11 +159,14 @@ __global__ __launch_bounds__(kBlock) void k_batch_prep(const CircDev *__restrict
     }
 }
 
-// Stores of this workgroup become visible to its other wavefronts' loads.
-__device__ __forceinline__ void block_fence() {
-    __threadfence();
-    __syncthreads();
-}
+// Stores of this workgroup become visible to its other wavefronts' loads.  A
+// circuit's arrays are touched by one workgroup only, whose wavefronts share
+// the CU's vector cache (written through, in order), so the barrier's own
+// workgroup-scope fence is all it takes: a device-scope fence also writes back
+// the XCD's L2 and invalidates caches after every pass.  512 circuits of 12
+// qubits with gradients, complex128: 2.36 ms with device-scope fences, 0.97
+// without; 512 of 16 qubits 13.3 and 11.9 ms.
+__device__ __forceinline__ void block_fence() { __syncthreads(); }
 
 template <class R>
 __device__ __forceinline__ void load_tile(const cx<R> *p, const uint64_t (&roff)[NR], cx<R> (&v)[NR]) {
@@ -386,8 +388,7 @@ __global__ __launch_bounds__(kBlock) void k_batch(const CircDev *__restrict__ ci
                 const int ns = tp->nslots, s0 = tp->slot_begin;
                 for (int s = 0; s < ns; ++s) acc[s][tid] = 0.0;
                 rev_pass<R, Lv>(tp, fops, gens + s0, psi, bra, ntiles, w, lane, acc);
-                __threadfence();
-                __syncthreads();
+                block_fence();
                 for (int s = w; s < ns; s += kWaves) {
                     double v = acc[s][lane] + acc[s][lane + 64] + acc[s][lane + 128] + acc[s][lane + 192];
                     v = wave_sum(v);
