@@ -386,8 +386,8 @@ lgh_status lgh_batch_run_serial(lgh_tmpl *const *tmpls, int32_t num_circuits, lg
  * pinned host buffers and captures the launch sequence (parameter upload,
  * descriptor preparation, persistent launch, result download) in a HIP
  * graph on a stream of the plan's own; it also autotunes the persistent
- * launch's grid (one or two resident workgroups per CU), timing both on the
- * plan's circuits and keeping the faster.  Each run replays the graph: the
+ * launch's grid (one to three resident workgroups per CU), timing each on the
+ * plan's circuits and keeping the fastest.  Each run replays the graph: the
  * results equal lgh_batch_run's bit for bit.  No counterpart in the
  * reference (see lgh_batch_run).  A plan must not be run from two threads at
  * once, and its templates must outlive it. */
@@ -398,8 +398,9 @@ lgh_status lgh_batch_plan_create(lgh_batch_plan **out, lgh_tmpl *const *tmpls, i
  * jac must be NULL for a plan created without gradients. */
 lgh_status lgh_batch_plan_run(lgh_batch_plan *plan, const double *params, const int64_t *param_offset,
                               double *expval, double *jac, const int64_t *jac_offset);
-/* The tuned grid (workgroups per CU) and the timed candidates (ms, one and
- * two workgroups per CU). */
+/* The tuned grid (workgroups per CU, 1 to 3; 3 only where there are circuits
+ * for it) and the timed candidates (ms: one workgroup per CU; the better of
+ * two and three). */
 lgh_status lgh_batch_plan_info(const lgh_batch_plan *plan, int32_t *grid_per_cu, double *tuned_ms);
 lgh_status lgh_batch_plan_destroy(lgh_batch_plan *plan);
 

@@ -38,8 +38,11 @@ HIP_FLAGS = [
 # The fused kernels branch on per-gate descriptor fields that are uniform
 # across the wavefront; leaving those regions unstructurized keeps the
 # register arrays in place across the branches instead of duplicating them.
+# (the batch kernel of complex128 circuits: 249 vector registers without it,
+# 167 with it, which lets a third wavefront onto each SIMD)
 FILE_FLAGS = {
     "lgh_fused.hip": ["-mllvm", "-structurizecfg-skip-uniform-regions=true"],
+    "lgh_batch.hip": ["-mllvm", "-structurizecfg-skip-uniform-regions=true"],
 }
 
 
