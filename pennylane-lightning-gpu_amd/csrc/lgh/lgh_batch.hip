@@ -98,6 +98,25 @@ struct CircDev {
     void *bra;
     double *jac; // nparams entries, or null without gradient
     double *expval;
+    double *scales; // see Scales; null: every gate in its whole form
+};
+
+// Rotations with their cosine taken out (complex128, lean kernels).  RX, RY
+// and RZ become c times [[1, iu], [iu, 1]], [[1, -t], [t, 1]] and
+// (1 - iu, 1 + iu): one FMA per component of the result instead of two
+// (four for RX).  The cosines are not applied: the registers hold the state
+// divided by their running product, and what is read from them is corrected:
+// <P> and every overlap by the product's square at its place.  A pass takes
+// out at most 2^-100 (past it, its gates stay whole), and every fourth pass
+// multiplies the product of the four before it back in where it loads its
+// tiles, so the values stay within 2^400 of the state's.  A tile of 8 registers
+// spends 48 FMAs per state on RX, RY, RZ instead of 128.
+constexpr int kScaleGroup = 4;
+constexpr double kScaleFloor = 0x1p-100;
+struct Scales { // a circuit's scale array, by pass (forward, then reverse)
+    __host__ __device__ static int64_t count(int64_t passes, int64_t slots) { return 2 * passes + 1 + slots; }
+    // [0, passes): a pass's product; [passes, 2 passes): factor on its loads;
+    // [2 passes]: factor of <P>; then one factor per slot
 };
 
 Form form_of(int gate) {
@@ -116,46 +135,126 @@ typedef __attribute__((address_space(4))) const CircDev CCirc;
 typedef __attribute__((address_space(4))) const TmplDev CTmpl;
 typedef __attribute__((address_space(4))) const TPass CTPass;
 typedef __attribute__((address_space(4))) const TSlot CTSlot;
+typedef __attribute__((address_space(4))) const double CDouble;
+
+// descriptor of a parametrised gate (c: its factor taken out, or 0)
+__device__ __forceinline__ void set_gate(FOp &f, int form, double c, double s, double th, bool unit) {
+    const double cc = unit ? 1.0 : c, ss = unit ? s / c : s;
+    switch (form) {
+    case kPhase: {
+        double s1, c1;
+        sincos(th, &s1, &c1);
+        f.m[0] = f.m[1] = cx<double>{c1, s1};
+        break;
+    }
+    case kRotDiag:
+        f.m[0] = cx<double>{cc, -ss};
+        f.m[1] = cx<double>{cc, ss};
+        break;
+    case kRX:
+        f.m[0] = f.m[3] = cx<double>{cc, 0.0};
+        f.m[1] = f.m[2] = cx<double>{0.0, -ss};
+        break;
+    default: // kRY
+        f.m[0] = f.m[3] = cx<double>{cc, 0.0};
+        f.m[1] = cx<double>{-ss, 0.0};
+        f.m[2] = cx<double>{ss, 0.0};
+        break;
+    }
+    bool real = (f.meta & 15u) != kDiag;
+    for (int q = 0; q < 4; ++q) real = real && f.m[q].im == 0.0;
+    const bool dsym = (f.meta & 15u) == kDiag && f.m[1].re == f.m[0].re && f.m[1].im == -f.m[0].im;
+    // (parametric gates are never exactly X: bit 23 stays as compiled, clear)
+    f.meta = (f.meta & ~(7u << 21)) | (uint32_t(real) << 21) | (uint32_t(dsym) << 22);
+    if (unit) f.meta |= (form == kRX ? 3u : 1u) << 28;
+}
 
 __global__ __launch_bounds__(kBlock) void k_batch_prep(const CircDev *__restrict__ circs, uint32_t *counter) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;
     const CircDev &cd = circs[blockIdx.x];
     const TmplDev *t = cd.t;
-    for (int i = threadIdx.x; i < t->nfops; i += kBlock) {
-        const Recipe &r = t->recipes[i];
-        FOp f = r.base;
-        if (r.form != kFixed) {
-            const double th = r.sign * cd.params[r.pidx];
-            double s, c;
-            sincos(0.5 * th, &s, &c);
-            switch (r.form) {
-            case kPhase: {
-                double s1, c1;
-                sincos(th, &s1, &c1);
-                f.m[0] = f.m[1] = cx<double>{c1, s1};
-                break;
+    if (!cd.scales) {
+        for (int i = threadIdx.x; i < t->nfops; i += kBlock) {
+            const Recipe &r = t->recipes[i];
+            FOp f = r.base;
+            if (r.form != kFixed) {
+                const double th = r.sign * cd.params[r.pidx];
+                double s, c;
+                sincos(0.5 * th, &s, &c);
+                set_gate(f, r.form, c, s, th, false);
             }
-            case kRotDiag:
-                f.m[0] = cx<double>{c, -s};
-                f.m[1] = cx<double>{c, s};
-                break;
-            case kRX:
-                f.m[0] = f.m[3] = cx<double>{c, 0.0};
-                f.m[1] = f.m[2] = cx<double>{0.0, -s};
-                break;
-            default: // kRY
-                f.m[0] = f.m[3] = cx<double>{c, 0.0};
-                f.m[1] = cx<double>{-s, 0.0};
-                f.m[2] = cx<double>{s, 0.0};
-                break;
-            }
-            bool real = (f.meta & 15u) != kDiag;
-            for (int q = 0; q < 4; ++q) real = real && f.m[q].im == 0.0;
-            const bool dsym = (f.meta & 15u) == kDiag && f.m[1].re == f.m[0].re && f.m[1].im == -f.m[0].im;
-            // (parametric gates are never exactly X: bit 23 stays as compiled, clear)
-            f.meta = (f.meta & ~(7u << 21)) | (uint32_t(real) << 21) | (uint32_t(dsym) << 22);
+            cd.fops[i] = f;
         }
-        cd.fops[i] = f;
+        return;
+    }
+    // A wavefront per pass, 64 gates at a time: the running product of the
+    // cosines by a scan over the lanes.
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, nf = t->nfwd, np = nf + t->nrev;
+    double *pend = cd.scales, *load = pend + np, *slots = load + np + 1;
+    for (int p = w; p <= np; p += kWaves) {
+        const TPass &tp = p < nf ? t->fwd[p] : p < np ? t->rev[p - nf] : *t->obs;
+        double run = 1.0;
+        for (int o0 = 0; o0 < tp.nops; o0 += 64) {
+            const int o = o0 + lane;
+            const bool live = o < tp.nops;
+            FOp f{};
+            int form = kFixed;
+            double th = 0.0, s = 0.0, c = 1.0;
+            if (live) {
+                const Recipe &r = t->recipes[tp.op_begin + o];
+                f = r.base;
+                form = r.form;
+                if (form != kFixed) {
+                    th = r.sign * cd.params[r.pidx];
+                    sincos(0.5 * th, &s, &c);
+                }
+            }
+            const bool rot = form == kRX || form == kRY || form == kRotDiag;
+            double incl = rot ? c : 1.0;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) {
+                const double up = __shfl_up(incl, d, 64);
+                if (lane >= d) incl *= up;
+            }
+            const double prev = __shfl_up(incl, 1, 64);
+            // the products only shrink: the gates above the floor come first
+            // (a NaN is not above it)
+            const bool above = fabs(run * incl) >= kScaleFloor;
+            const uint64_t low = __ballot(!above);
+            const int kept = low ? __ffsll((unsigned long long)low) - 1 : 64;
+            const double last = __shfl(incl, kept ? kept - 1 : 0, 64);
+            const double end = kept ? run * last : run;
+            const bool unit = rot && lane < kept;
+            if (live) {
+                if (form != kFixed) set_gate(f, form, c, s, th, unit);
+                cd.fops[tp.op_begin + o] = f;
+                const int slot = int((f.meta >> 8) & 255u) - 1;
+                if (p >= nf && p < np && slot >= 0) {
+                    const double before = lane <= kept ? (lane ? run * prev : run) : end;
+                    slots[tp.slot_begin + slot] = before * before;
+                }
+            }
+            run = end;
+        }
+        if (p < np && lane == 0) pend[p] = run;
+    }
+    __syncthreads();
+    for (int p = threadIdx.x; p <= np; p += kBlock) {
+        // p == np stands for the observable, after the last forward pass
+        const int q = p < np ? p : nf, g0 = q / kScaleGroup * kScaleGroup;
+        double base = 1.0, back = 1.0;
+        for (int r = g0; r < q; ++r) base *= pend[r];
+        if (q == g0 && q > 0)
+            for (int r = g0 - kScaleGroup; r < g0; ++r) back *= pend[r];
+        if (p == np) { // its state is read as it lies
+            load[np] = base * base * back * back;
+            continue;
+        }
+        load[p] = back;
+        if (p >= nf) {
+            const TPass &tp = t->rev[p - nf];
+            for (int s = 0; s < tp.nslots; ++s) slots[tp.slot_begin + s] *= base * base;
+        }
     }
 }
 
@@ -177,6 +276,11 @@ template <class R>
 __device__ __forceinline__ void store_tile(cx<R> *p, const uint64_t (&roff)[NR], const cx<R> (&v)[NR]) {
 #pragma unroll
     for (int k = 0; k < NR; ++k) stnt(p + roff[k], v[k]);
+}
+
+template <class R> __device__ __forceinline__ void scale_tile(R c, cx<R> (&v)[NR]) {
+#pragma unroll
+    for (int k = 0; k < NR; ++k) v[k] = rmul(c, v[k]);
 }
 
 // Tile geometry of one pass: register offsets, all tile bits, and this
@@ -213,7 +317,8 @@ __device__ __forceinline__ uint64_t tile_step(uint64_t g, uint64_t tmask) {
 
 // Lv > 0: every gate of the pass has a form of that lean level (see lean_level)
 template <class R, int Lv>
-__device__ __forceinline__ void fwd_pass(const CTPass *tp, const CFOp *fops, cx<R> *psi, uint64_t ntiles, int w, int lane) {
+__device__ __forceinline__ void fwd_pass(const CTPass *tp, const CFOp *fops, cx<R> *psi, uint64_t ntiles, int w, int lane,
+                         double sc) {
     const PassGeo g = pass_geo(tp, lane);
     const int nops = tp->nops;
     const CFOp *ops = fops + tp->op_begin;
@@ -223,12 +328,14 @@ __device__ __forceinline__ void fwd_pass(const CTPass *tp, const CFOp *fops, cx<
         cx<R> *p = psi + base;
         cx<R> v[NR];
         load_tile(p, g.roff, v);
+        if constexpr (Lv > 0 && sizeof(R) == 8)
+            if (sc != 1.0) scale_tile(R(sc), v);
         if (nops > 0) {
             FOp cur = load_op(ops);
             for (int o = 0; o < nops; ++o) {
                 const FOp nxt = load_op(ops + (o + 1 < nops ? o + 1 : o));
                 if constexpr (Lv > 0)
-                    apply_lean<R, NR, Lv>(cur, lane, base, v);
+                    apply_lean<R, NR, Lv, sizeof(R) == 8>(cur, lane, base, v);
                 else
                     apply_fop<R, NR>(cur, lane, base, v);
                 cur = nxt;
@@ -265,7 +372,7 @@ __device__ __forceinline__ double obs_pass(const CTPass *tp, const CFOp *fops, c
 
 template <class R, int Lv>
 __device__ __forceinline__ void rev_pass(const CTPass *tp, const CFOp *fops, const CFGen *gens, cx<R> *lam, cx<R> *bra,
-                         uint64_t ntiles, int w, int lane, double (*acc)[kBlock]) {
+                         uint64_t ntiles, int w, int lane, double (*acc)[kBlock], double sc) {
     const PassGeo g = pass_geo(tp, lane);
     const int nops = tp->nops;
     const CFOp *ops = fops + tp->op_begin;
@@ -277,13 +384,28 @@ __device__ __forceinline__ void rev_pass(const CTPass *tp, const CFOp *fops, con
         cx<R> a[NR], b[NR];
         load_tile(pa, g.roff, a);
         load_tile(pb, g.roff, b);
+        if constexpr (Lv > 0 && sizeof(R) == 8)
+            if (sc != 1.0) {
+                scale_tile(R(sc), a);
+                scale_tile(R(sc), b);
+            }
         if (nops > 0) {
             FOp cur = load_op(ops);
             for (int o = 0; o < nops; ++o) {
                 const FOp nxt = load_op(ops + (o + 1 < nops ? o + 1 : o));
                 const int slot = f_slot(cur);
                 if constexpr (Lv > 0) {
-                    if (f_kind(cur) == kDiag) { // a phase on at most one register bit
+                    if (sizeof(R) == 8 && f_kind(cur) == kDiag && f_rot(cur)) { // its unit form
+                        if constexpr (sizeof(R) == 8) {
+                            if (slot >= 0) {
+                                const CFGen *gp = gens + slot;
+                                acc[slot][tid] +=
+                                    adj_diag_step<R, NR, true, true>(cur, gp->g[0].re, gp->g[1].re, base, a, b);
+                            } else {
+                                adj_diag_step<R, NR, false, true>(cur, 0.0, 0.0, base, a, b);
+                            }
+                        }
+                    } else if (f_kind(cur) == kDiag) { // a phase on at most one register bit
                         if (slot >= 0) {
                             const CFGen *gp = gens + slot;
                             acc[slot][tid] += adj_diag_step<R, NR, true>(cur, gp->g[0].re, gp->g[1].re, base, a, b);
@@ -338,16 +460,16 @@ __device__ __forceinline__ void rev_pass(const CTPass *tp, const CFOp *fops, con
 
 // Bound by the gate loop's vector instructions and the latency of a tile's
 // loads, which other wavefronts have to cover.  Uniform branches are left
-// unstructurized in this file: 249 vector registers become 167 (complex128;
-// 128 in complex64), three wavefronts per SIMD for two, without a spill
-// (forcing three with launch bounds spilled inside the gate loop and halved
-// the throughput).  4096 circuits of 8 to 20 qubits, forward and adjoint:
-// 227 -> 196 ms in complex128, 173 -> 143 in complex64; 512 of 20 qubits
-// 212 -> 179 ms.
+// unstructurized in this file: 249 vector registers become 168 (complex128;
+// 128 in complex64), three wavefronts per SIMD for two, without a spill.
+// 4096 circuits of 8 to 20 qubits, forward and adjoint: 227 -> 196 ms in
+// complex128, 173 -> 141 in complex64.  With the rotations' cosines taken out
+// (see Scales; complex128) 196 -> 163 ms, 512 circuits of 20 qubits
+// 179 -> 157 ms.
 // Lv: lean level of every forward and reverse pass of the batch's templates
 // (0: any fusable gate); the observable pass always takes the general form.
 template <class R, int Lv = 0>
-__global__ __launch_bounds__(kBlock) void k_batch(const CircDev *__restrict__ circs, int ncirc,
+__global__ __launch_bounds__(kBlock, Lv > 0 && sizeof(R) == 8 ? 3 : 1) void k_batch(const CircDev *__restrict__ circs, int ncirc,
                                                   uint32_t *__restrict__ counter, int grad) {
     __shared__ double acc[kMaxSlots][kBlock];
     __shared__ double red[kMaxSlots];
@@ -368,6 +490,15 @@ __global__ __launch_bounds__(kBlock) void k_batch(const CircDev *__restrict__ ci
         cx<R> *psi = static_cast<cx<R> *>(cd->psi);
         cx<R> *bra = static_cast<cx<R> *>(cd->bra);
         double *jac = cd->jac;
+        // entry i of the circuit's factors (see Scales), read where it is used:
+        // scalar registers are short here
+        auto factor = [&](int i) {
+            if constexpr (Lv > 0 && sizeof(R) == 8) {
+                const CDouble *sc = (const CDouble *)cd->scales;
+                return sc ? sc[nfwd + nrev + i] : 1.0;
+            }
+            return 1.0;
+        };
         // |0..0>
         const uint64_t N = 1ull << nq;
         for (uint64_t i = tid; i < N; i += kBlock) psi[i] = cx<R>{R(i == 0 ? 1 : 0), R(0)};
@@ -375,7 +506,7 @@ __global__ __launch_bounds__(kBlock) void k_batch(const CircDev *__restrict__ ci
             for (int j = tid; j < nparams; j += kBlock) jac[j] = 0.0;
         block_fence();
         for (int p = 0; p < nfwd; ++p) {
-            fwd_pass<R, Lv>((const CTPass *)t->fwd + p, fops, psi, ntiles, w, lane);
+            fwd_pass<R, Lv>((const CTPass *)t->fwd + p, fops, psi, ntiles, w, lane, factor(p));
             block_fence();
         }
         const double e = wave_sum(obs_pass<R>((const CTPass *)t->obs, fops, psi, bra, ntiles, w, lane));
@@ -384,7 +515,7 @@ __global__ __launch_bounds__(kBlock) void k_batch(const CircDev *__restrict__ ci
         if (tid == 0) {
             double s = 0.0;
             for (int q = 0; q < kWaves; ++q) s += red_e[q];
-            *cd->expval = s;
+            *cd->expval = s * factor(nfwd + nrev);
         }
         if (grad && jac) {
             const CTSlot *slots = (const CTSlot *)t->slots;
@@ -393,12 +524,13 @@ __global__ __launch_bounds__(kBlock) void k_batch(const CircDev *__restrict__ ci
                 const CTPass *tp = (const CTPass *)t->rev + p;
                 const int ns = tp->nslots, s0 = tp->slot_begin;
                 for (int s = 0; s < ns; ++s) acc[s][tid] = 0.0;
-                rev_pass<R, Lv>(tp, fops, gens + s0, psi, bra, ntiles, w, lane, acc);
+                rev_pass<R, Lv>(tp, fops, gens + s0, psi, bra, ntiles, w, lane, acc,
+                                factor(nfwd + p));
                 block_fence();
                 for (int s = w; s < ns; s += kWaves) {
                     double v = acc[s][lane] + acc[s][lane + 64] + acc[s][lane + 128] + acc[s][lane + 192];
                     v = wave_sum(v);
-                    if (lane == 0) red[s] = v;
+                    if (lane == 0) red[s] = v * factor(nfwd + nrev + 1 + s0 + s);
                 }
                 __syncthreads();
                 if (tid == 0)
@@ -532,13 +664,14 @@ struct BatchLayout {
     int dev = 0;
     int32_t ncirc = 0;
     bool grad = false;
-    std::vector<int64_t> p_off, f_off, j_off;
+    std::vector<int64_t> p_off, f_off, j_off, c_off;
     std::vector<uint64_t> s_off;
-    int64_t np = 0, nf = 0, nj = 0;
+    int64_t np = 0, nf = 0, nj = 0, nc = 0;
     uint64_t ns = 0;
-    size_t b_circ = 0, b_par = 0, b_fop = 0, b_jac = 0, b_exp = 0, total = 0, sbytes = 0;
+    size_t b_circ = 0, b_par = 0, b_fop = 0, b_jac = 0, b_exp = 0, b_sc = 0, total = 0, sbytes = 0;
     std::vector<int32_t> order;
     int lean = 0; // the kernel's lean level: the highest of the templates', 0 if any has none
+    bool unit = false; // rotations with their cosines taken out (see Scales)
     char *d = nullptr;
     void *states = nullptr;
 
@@ -546,7 +679,8 @@ struct BatchLayout {
     FOp *d_fop() const { return reinterpret_cast<FOp *>(d + b_circ + b_par); }
     double *d_jac() const { return reinterpret_cast<double *>(d + b_circ + b_par + b_fop); }
     double *d_exp() const { return reinterpret_cast<double *>(d + b_circ + b_par + b_fop + b_jac); }
-    uint32_t *d_cnt() const { return reinterpret_cast<uint32_t *>(d + b_circ + b_par + b_fop + b_jac + b_exp); }
+    double *d_sc() const { return reinterpret_cast<double *>(d + b_circ + b_par + b_fop + b_jac + b_exp); }
+    uint32_t *d_cnt() const { return reinterpret_cast<uint32_t *>(d + b_circ + b_par + b_fop + b_jac + b_exp + b_sc); }
 
     template <class R> void plan(lgh_tmpl *const *tmpls, int32_t n, bool with_grad) {
         dev = tmpls[0]->device;
@@ -564,6 +698,10 @@ struct BatchLayout {
         f_off.resize(size_t(n));
         j_off.resize(size_t(n));
         s_off.resize(size_t(n));
+        c_off.resize(size_t(n));
+        // single precision keeps every gate whole: its values' range is too
+        // short for the factors of several passes
+        unit = lean > 0 && sizeof(R) == 8;
         for (int32_t c = 0; c < n; ++c) {
             const lgh_tmpl *t = tmpls[c];
             p_off[size_t(c)] = np;
@@ -574,13 +712,16 @@ struct BatchLayout {
             nj += grad ? t->nparams : 0;
             s_off[size_t(c)] = ns;
             ns += 2ull << t->nq; // psi and bra
+            c_off[size_t(c)] = nc;
+            nc += unit ? Scales::count(int64_t(t->fwd.size() + t->rev.size()), int64_t(t->slots.size())) : 0;
         }
         b_circ = al256(sizeof(CircDev) * size_t(n));
         b_par = al256(sizeof(double) * size_t(std::max<int64_t>(1, np)));
         b_fop = al256(sizeof(FOp) * size_t(std::max<int64_t>(1, nf)));
         b_jac = al256(sizeof(double) * size_t(std::max<int64_t>(1, nj)));
         b_exp = al256(sizeof(double) * size_t(n));
-        total = b_circ + b_par + b_fop + b_jac + b_exp + 256;
+        b_sc = al256(sizeof(double) * size_t(nc));
+        total = b_circ + b_par + b_fop + b_jac + b_exp + b_sc + 256;
         sbytes = sizeof(cx<R>) * ns;
         order.resize(size_t(n));
         std::iota(order.begin(), order.end(), 0);
@@ -618,6 +759,7 @@ struct BatchLayout {
             cd.bra = st + s_off[size_t(c)] + (1ull << t->nq);
             cd.jac = grad ? d_jac() + j_off[size_t(c)] : nullptr;
             cd.expval = d_exp() + c;
+            cd.scales = unit ? d_sc() + c_off[size_t(c)] : nullptr;
         }
         return hc;
     }

@@ -73,7 +73,9 @@ __device__ __forceinline__ bool f_dsym(const FOp &o) { return (o.meta >> 22) & 1
 // dense 2x2 equal to [[0, 1], [1, 0]] (X, CNOT, Toffoli)
 __device__ __forceinline__ bool f_isx(const FOp &o) { return (o.meta >> 23) & 1u; }
 // rotation with a factor moved by the host into a scale of the whole pass:
-// 1: [[1, -t], [t, 1]] (t in m[2]), 2: [[t, -1], [1, t]] (t in m[0]), 0: neither
+// 1: [[1, -t], [t, 1]] (t in m[2]), 2: [[t, -1], [1, t]] (t in m[0]),
+// 3: [[1, iu], [iu, 1]] (u in m[1].im; complex128 only), 0: none of them.  On
+// a diagonal gate (batched kernel, complex128), 1: (1 - iu, 1 + iu), u in m[1].im
 __device__ __forceinline__ int f_rot(const FOp &o) { return int((o.meta >> 28) & 3u); }
 // every register satisfies the register-bit controls (the controls, if any,
 // are on lane or higher bits)
@@ -193,6 +195,10 @@ template <class R> struct M2 {
 template <class R> __device__ __forceinline__ M2<R> m2(const FOp &op) {
     return M2<R>{lo<R>(op.m[0]), lo<R>(op.m[1]), lo<R>(op.m[2]), lo<R>(op.m[3])};
 }
+// x + i u y
+template <class R> __device__ __forceinline__ cx<R> ifma(R u, cx<R> y, cx<R> x) {
+    return cx<R>{fma(-u, y.im, x.re), fma(u, y.re, x.im)};
+}
 template <class R, bool Real, int Rot = 0>
 __device__ __forceinline__ void mat2(const M2<R> &m, cx<R> &x0, cx<R> &x1) {
     cx<R> y0, y1;
@@ -202,6 +208,9 @@ __device__ __forceinline__ void mat2(const M2<R> &m, cx<R> &x0, cx<R> &x1) {
     } else if constexpr (Rot == 2) {
         y0 = rfma(m.m00.re, x0, neg(x1));
         y1 = rfma(m.m11.re, x1, x0);
+    } else if constexpr (Rot == 3) {
+        y0 = ifma(m.m01.im, x1, x0);
+        y1 = ifma(m.m01.im, x0, x1);
     } else if constexpr (Real) {
         y0 = rfma(m.m01.re, x1, rmul(m.m00.re, x0));
         y1 = rfma(m.m11.re, x1, rmul(m.m10.re, x0));
@@ -218,6 +227,8 @@ template <class R, bool Real, int Rot = 0>
 __device__ __forceinline__ cx<R> row2(cx<R> cs, cx<R> cp, cx<R> own, cx<R> partner) {
     if constexpr (Rot == 1)
         return rfma(cp.re, partner, own);
+    else if constexpr (Rot == 3)
+        return ifma(cp.im, partner, own);
     else if constexpr (Real)
         return rfma(cp.re, partner, rmul(cs.re, own));
     else
@@ -244,7 +255,7 @@ __device__ __forceinline__ void lane_plain(const M2<R> &m, int lane, cx<R> (&v)[
         const bool hi = (lane >> L) & 1;
         const cx<R> cs = hi ? m.m11 : m.m00, cp = hi ? m.m10 : m.m01;
 #pragma unroll
-        for (int k = 0; k < NR; ++k) v[k] = row2<R, Real, Rot == 1 ? 1 : 0>(cs, cp, v[k], xor_lane_cx<L>(v[k], lane));
+        for (int k = 0; k < NR; ++k) v[k] = row2<R, Real, Rot == 2 ? 0 : Rot>(cs, cp, v[k], xor_lane_cx<L>(v[k], lane));
     }
 }
 
@@ -300,13 +311,17 @@ constexpr int kDiagNoReg = 7;
 template <class R> __device__ __forceinline__ cx<R> phase_cs(cx<R> x, R c, R s) {
     return cx<R>{c * x.re - s * x.im, c * x.im + s * x.re};
 }
-template <class R, int NR, int B>
+// Unit: c = 1 (its factor taken out by the host or the preparation kernel)
+template <class R, int NR, int B, bool Unit = false>
 __device__ __forceinline__ void diag_sym(const FOp &op, bool lpar, cx<R> (&v)[NR]) {
     const R c = R(op.m[1].re), s = R(op.m[1].im);
     const R s0 = flip(s, lpar ? 0u : kSignBit); // registers with even register parity
     const R s1 = flip(s, lpar ? kSignBit : 0u);
 #pragma unroll
-    for (int k = 0; k < NR; ++k) v[k] = phase_cs(v[k], c, (B >= 0 && ((k >> B) & 1)) ? s1 : s0);
+    for (int k = 0; k < NR; ++k) {
+        const R sk = (B >= 0 && ((k >> B) & 1)) ? s1 : s0;
+        v[k] = Unit ? ifma(sk, v[k], v[k]) : phase_cs(v[k], c, sk);
+    }
 }
 
 template <class R, int NR>
@@ -582,8 +597,8 @@ __device__ __forceinline__ double adj_lane_plain(const M2<R> &m, uint32_t gk, co
         const bool hi = (lane >> L) & 1;
         const cx<R> cs = hi ? m.m11 : m.m00, cp = hi ? m.m10 : m.m01;
         auto step = [&](int k, const cx<R> &pa) {
-            a[k] = row2<R, Real, Rot == 1 ? 1 : 0>(cs, cp, a[k], pa);
-            b[k] = row2<R, Real, Rot == 1 ? 1 : 0>(cs, cp, b[k], xor_lane_cx<L>(b[k], lane));
+            a[k] = row2<R, Real, Rot == 2 ? 0 : Rot>(cs, cp, a[k], pa);
+            b[k] = row2<R, Real, Rot == 2 ? 0 : Rot>(cs, cp, b[k], xor_lane_cx<L>(b[k], lane));
         };
         if constexpr (Gen) {
             // X and Y generators: one chain of two FMAs per register; the Y
@@ -682,13 +697,14 @@ __device__ __forceinline__ double adj_plain_dense(const FOp &op, const FGen *g, 
 }
 
 // Adjoint: a lean pass's dense gate (uncontrolled: rotation form 1 or 2, a
-// plain real matrix (F = 0) or a complex one (F = 3); trainable ones with an
-// X or Y generator).
+// plain real matrix (F = 0), a complex one (F = 3) or rotation form 3 (F = 4,
+// a trainable one with an X generator); trainable ones with an X or Y generator).
 template <class R, int NR, int B, bool Gen, int F>
 __device__ __forceinline__ double adj_reg_lean(const M2<R> &m, uint32_t gk, cx<R> (&a)[NR], cx<R> (&b)[NR]) {
     const FGen g{};
-    constexpr bool Real = F != 3;
-    constexpr int Rot = F == 3 ? 0 : F;
+    constexpr bool Real = F < 3;
+    constexpr int Rot = F == 3 ? 0 : F == 4 ? 3 : F;
+    if constexpr (F == 4) return adj_reg_plain<R, NR, B, false, Gen, 3, kGenX>(m, kGenX, &g, a, b);
     if constexpr (Gen) {
         if (gk == kGenY) return adj_reg_plain<R, NR, B, Real, true, Rot, kGenY>(m, gk, &g, a, b);
         return adj_reg_plain<R, NR, B, Real, true, Rot, kGenX>(m, gk, &g, a, b);
@@ -699,8 +715,9 @@ template <class R, int NR, int L, bool Gen, int F>
 __device__ __forceinline__ double adj_lane_lean(const M2<R> &m, uint32_t gk, int lane, cx<R> (&a)[NR],
                                                 cx<R> (&b)[NR]) {
     const FGen g{};
-    constexpr bool Real = F != 3;
-    constexpr int Rot = F == 3 ? 0 : F;
+    constexpr bool Real = F < 3;
+    constexpr int Rot = F == 3 ? 0 : F == 4 ? 3 : F;
+    if constexpr (F == 4) return adj_lane_plain<R, NR, L, false, Gen, 3, kGenX>(m, kGenX, &g, lane, a, b);
     if constexpr (L >= 4 && Gen) {
         if (gk == kGenY) return adj_lane_plain<R, NR, L, Real, true, Rot, kGenY>(m, gk, &g, lane, a, b);
         return adj_lane_plain<R, NR, L, Real, true, Rot, kGenX>(m, gk, &g, lane, a, b);
@@ -718,16 +735,20 @@ __device__ __forceinline__ void adj_plain_lean(const FOp &op, int lane, cx<R> (&
     const M2<R> m = m2<R>(op);
     const uint32_t gk = f_gkind(op);
     const int rot = f_rot(op), loc = f_loc(op);
-    const int form = rot ? rot : ((Lv == 1 || f_real(op)) ? 0 : 3);
+    // rotation form 3 is F = 4 (level 2, complex128)
+    constexpr int kX = Lv == 2 && sizeof(R) == 8 ? 4 : 0;
+    const int form = kX && rot == 3 ? 4 : rot ? rot : ((Lv == 1 || f_real(op)) ? 0 : 3);
 #define LGH_REG3(B)                                                                                                    \
     (form == 1   ? sink(adj_reg_lean<R, NR, B, Gen, 1>(m, gk, a, b))                                                 \
      : form == 2 ? sink(adj_reg_lean<R, NR, B, Gen, 2>(m, gk, a, b))                                                 \
      : form == 0 ? sink(adj_reg_lean<R, NR, B, Gen, 0>(m, gk, a, b))                                                 \
+     : kX && form == kX ? sink(adj_reg_lean<R, NR, B, Gen, kX>(m, gk, a, b))                                         \
                  : sink(adj_reg_lean<R, NR, B, Gen, Lv == 2 ? 3 : 0>(m, gk, a, b)))
 #define LGH_LANE3(L)                                                                                                   \
     (form == 1   ? sink(adj_lane_lean<R, NR, L, Gen, 1>(m, gk, lane, a, b))                                          \
      : form == 2 ? sink(adj_lane_lean<R, NR, L, Gen, 2>(m, gk, lane, a, b))                                          \
      : form == 0 ? sink(adj_lane_lean<R, NR, L, Gen, 0>(m, gk, lane, a, b))                                          \
+     : kX && form == kX ? sink(adj_lane_lean<R, NR, L, Gen, kX>(m, gk, lane, a, b))                                  \
                  : sink(adj_lane_lean<R, NR, L, Gen, Lv == 2 ? 3 : 0>(m, gk, lane, a, b)))
     if (f_kind(op) == kRegDense) {
         switch (loc) {
@@ -755,7 +776,7 @@ __device__ __forceinline__ void adj_plain_lean(const FOp &op, int lane, cx<R> (&
 // the overlap with a diagonal generator (eigenvalue g_even / g_odd by the
 // parity of the mask bits) and the phase on both states, the lane parity
 // computed once.
-template <class R, int NR, int B, bool Gen>
+template <class R, int NR, int B, bool Gen, bool Unit>
 __device__ __forceinline__ double adj_diag_sym(const FOp &op, double ge, double go, uint64_t base, cx<R> (&a)[NR],
                                                cx<R> (&b)[NR]) {
     const bool lpar = __popcll(base & op.pm_rest) & 1;
@@ -768,8 +789,9 @@ __device__ __forceinline__ double adj_diag_sym(const FOp &op, double ge, double 
     for (int k = 0; k < NR; ++k) {
         const bool odd = B >= 0 && ((k >> B) & 1);
         if constexpr (Gen) acc += (odd ? g1 : g0) * im_cdot2(b[k], a[k]);
-        a[k] = phase_cs(a[k], c, odd ? s1 : s0);
-        b[k] = phase_cs(b[k], c, odd ? s1 : s0);
+        const R sk = odd ? s1 : s0;
+        a[k] = Unit ? ifma(sk, a[k], a[k]) : phase_cs(a[k], c, sk);
+        b[k] = Unit ? ifma(sk, b[k], b[k]) : phase_cs(b[k], c, sk);
     }
     return acc;
 }
@@ -781,17 +803,17 @@ __device__ __forceinline__ bool diag_fast(const FOp &op) {
            (f_slot(op) < 0 || f_gkind(op) == kGenDiag);
 }
 // ge, go: generator eigenvalues for even / odd parity (unused without Gen)
-template <class R, int NR, bool Gen>
+template <class R, int NR, bool Gen, bool Unit = false>
 __device__ __forceinline__ double adj_diag_step(const FOp &op, double ge, double go, uint64_t base, cx<R> (&a)[NR],
                                                 cx<R> (&b)[NR]) {
     switch (f_loc(op)) {
-    case 0: return adj_diag_sym<R, NR, 0, Gen>(op, ge, go, base, a, b);
-    case 1: return adj_diag_sym<R, NR, 1, Gen>(op, ge, go, base, a, b);
-    case 2: return adj_diag_sym<R, NR, 2, Gen>(op, ge, go, base, a, b);
+    case 0: return adj_diag_sym<R, NR, 0, Gen, Unit>(op, ge, go, base, a, b);
+    case 1: return adj_diag_sym<R, NR, 1, Gen, Unit>(op, ge, go, base, a, b);
+    case 2: return adj_diag_sym<R, NR, 2, Gen, Unit>(op, ge, go, base, a, b);
     case 3:
-        if constexpr (NR > 8) return adj_diag_sym<R, NR, 3, Gen>(op, ge, go, base, a, b);
+        if constexpr (NR > 8) return adj_diag_sym<R, NR, 3, Gen, Unit>(op, ge, go, base, a, b);
         return 0.0;
-    default: return adj_diag_sym<R, NR, -1, Gen>(op, ge, go, base, a, b);
+    default: return adj_diag_sym<R, NR, -1, Gen, Unit>(op, ge, go, base, a, b);
     }
 }
 
@@ -908,7 +930,7 @@ inline int lean_level_op(const FOp &f, bool adjoint) {
     }
     const int rot = int((f.meta >> 28) & 3u);
     const bool real = (f.meta >> 21) & 1u;
-    return rot != 0 || real ? 1 : 2;
+    return rot == 1 || rot == 2 || real ? 1 : 2;
 }
 inline bool lean_member(const FOp &m, bool adjoint) {
     const uint32_t mc = (m.meta >> 24) & 3u;
@@ -968,7 +990,19 @@ template <class R, int NR> __device__ __forceinline__ void scale_lean(const FOp 
 #pragma unroll
     for (int k = 0; k < NR; ++k) v[k] = rmul(c, v[k]);
 }
-template <class R, int NR, int Lv>
+template <class R, int NR, bool Unit> __device__ __forceinline__ void diag_lean(const FOp &op, bool lpar, cx<R> (&v)[NR]) {
+    switch (f_loc(op)) {
+    case 0: diag_sym<R, NR, 0, Unit>(op, lpar, v); return;
+    case 1: diag_sym<R, NR, 1, Unit>(op, lpar, v); return;
+    case 2: diag_sym<R, NR, 2, Unit>(op, lpar, v); return;
+    case 3:
+        if constexpr (NR > 8) diag_sym<R, NR, 3, Unit>(op, lpar, v);
+        return;
+    default: diag_sym<R, NR, -1, Unit>(op, lpar, v); return;
+    }
+}
+// Unit: diagonal gates may come in their unit form (batched kernel)
+template <class R, int NR, int Lv, bool Unit = false>
 __device__ __forceinline__ void apply_lean(const FOp &op, int lane, uint64_t base, cx<R> (&v)[NR]) {
     if (f_kind(op) == kDiag) {
         if (Lv == 1 || !f_dsym(op)) {
@@ -976,19 +1010,19 @@ __device__ __forceinline__ void apply_lean(const FOp &op, int lane, uint64_t bas
             return;
         }
         const bool lpar = __popcll(base & op.pm_rest) & 1;
-        switch (f_loc(op)) {
-        case 0: diag_sym<R, NR, 0>(op, lpar, v); return;
-        case 1: diag_sym<R, NR, 1>(op, lpar, v); return;
-        case 2: diag_sym<R, NR, 2>(op, lpar, v); return;
-        case 3:
-            if constexpr (NR > 8) diag_sym<R, NR, 3>(op, lpar, v);
-            return;
-        default: diag_sym<R, NR, -1>(op, lpar, v); return;
+        if constexpr (Unit) {
+            if (f_rot(op)) {
+                diag_lean<R, NR, true>(op, lpar, v);
+                return;
+            }
         }
+        diag_lean<R, NR, false>(op, lpar, v);
+        return;
     }
     const M2<R> m = m2<R>(op);
     const int loc = f_loc(op), rot = f_rot(op);
     const bool real = Lv == 1 || f_real(op);
+    constexpr int kX = Lv == 2 && sizeof(R) == 8 ? 3 : 0; // rotation form 3
     if constexpr (Lv == 2) {
         if (!f_plain(op)) {
             cx_lean<R, NR>(op, m, lane, base, v);
@@ -1001,6 +1035,8 @@ __device__ __forceinline__ void apply_lean(const FOp &op, int lane, uint64_t bas
         reg_plain<R, NR, B, true, 1>(m, v);                                                                            \
     else if (rot == 2)                                                                                                 \
         reg_plain<R, NR, B, true, 2>(m, v);                                                                            \
+    else if (kX && rot == 3)                                                                                           \
+        reg_plain<R, NR, B, false, kX>(m, v);                                                                          \
     else if (real)                                                                                                     \
         reg_plain<R, NR, B, true>(m, v);                                                                               \
     else                                                                                                               \
@@ -1021,6 +1057,8 @@ __device__ __forceinline__ void apply_lean(const FOp &op, int lane, uint64_t bas
         lane_plain<R, NR, L, true, 1>(m, lane, v);                                                                     \
     else if (L >= 4 && rot == 2)                                                                                       \
         lane_plain<R, NR, L, true, 2>(m, lane, v);                                                                     \
+    else if (kX && rot == 3)                                                                                           \
+        lane_plain<R, NR, L, false, kX>(m, lane, v);                                                                   \
     else if (real)                                                                                                     \
         lane_plain<R, NR, L, true>(m, lane, v);                                                                        \
     else                                                                                                               \
