@@ -967,6 +967,20 @@ Built lgh::fz::build_pass(const Pass &p, const std::vector<KOp> &kops, int n, bo
             before[x] = scale;
             if (h.kind == kDiag || h.cm_reg != 0 || h.f.cm_rest != 0) continue;
             const cx<double> *m = h.f.m;
+            // Rotations [[c, is], [is, c]] (RX) likewise become c [[1, iu],
+            // [iu, 1]] with u = s / c: four FMAs per pair for sixteen.  Any
+            // u will do (the scale's floor bounds it); complex64 keeps them
+            // whole, as its values' range is short.
+            if (!single && (h.slot < 0 || h.gkind == kGenX) && m[0].im == 0.0 && m[3].im == 0.0 && m[1].re == 0.0 &&
+                m[2].re == 0.0 && m[1].im != 0.0 && m[3].re == m[0].re && m[2].im == m[1].im &&
+                std::abs(scale * m[0].re) >= scale_floor) {
+                const double c = m[0].re, u = m[1].im / c;
+                h.f.m[0] = h.f.m[3] = cx<double>{1.0, 0.0};
+                h.f.m[1] = h.f.m[2] = cx<double>{0.0, u};
+                h.rot = 3;
+                scale *= c;
+                continue;
+            }
             if (m[0].im != 0.0 || m[1].im != 0.0 || m[2].im != 0.0 || m[3].im != 0.0) continue;
             const double c = m[0].re, s = m[2].re;
             if (m[3].re != c || m[1].re != -s || (c == 0.0 && s == 0.0)) continue;
