@@ -534,6 +534,115 @@ __global__ __launch_bounds__(kBlock) void k_pauli_add(cx<R> *__restrict__ dst, c
 
 // ---------------------------------------------------------------- CSR
 
+// Short rows (see csr_streams): a workgroup takes kBlock / T consecutive rows,
+// whose entries lie together, and stages them in LDS as one stream, every load
+// full and all loads of a step in flight at once.  From there neighbouring
+// lanes walk neighbouring rows, each of the T parts of the workgroup every
+// T-th entry of its row: the columns of neighbouring rows at one place of the
+// row are near each other in an operator on qubits, so a load of x touches
+// few cache lines.  Rows of any length are right; a long one only leaves the
+// other rows' lanes idle while it streams.  T follows the average, so that a
+// workgroup's rows fill about one step.
+// Bound by reading the matrix (70 us of the 89 it takes at the first of these
+// sizes).  <H> of the 21-entry rows of a transverse-field Ising chain on 20
+// qubits, call to call: 150 -> 103 us in complex128 (32-bit indices; with 64
+// the matrix has 528 MB for 440), 119 -> 82 in complex64, against 16 lanes
+// per row, whose loads of x took a cache line per lane and whose second round
+// had 5 of 16 lanes at work.
+constexpr int kCsrItems = 6;
+__global__ __launch_bounds__(kBlock) void k_narrow(int32_t *__restrict__ dst, const int64_t *__restrict__ src,
+                                                   int64_t count) {
+    const int64_t i = int64_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (i < count) dst[i] = int32_t(src[i]);
+}
+
+// Rows of random columns, 2^18 of 30 and 44 entries: 90 and 121 us, with 32
+// lanes per row 92 and 136, in complex128; in complex64 73 and 95, with 32
+// lanes 71 and 89.  Of 18 entries and less the stream is faster in both.
+template <class R> bool csr_streams(double avg) { return avg <= (sizeof(R) == 8 ? 48 : 24); }
+constexpr int kCsrPerCu = 5; // workgroups per CU that the LDS allows
+template <class I, class R, int T>
+__global__ __launch_bounds__(kBlock) void k_csr_stream(const I *__restrict__ indptr, const I *__restrict__ indices,
+                                                       const cx<R> *__restrict__ vals, const cx<R> *__restrict__ x,
+                                                       cx<R> *__restrict__ y, int64_t rows,
+                                                       double *__restrict__ partials) {
+    constexpr int kRows = kBlock / T, kStep = kCsrItems * kBlock, kAhead = 3;
+    __shared__ __align__(16) cx<R> s_val[kStep];
+    __shared__ I s_col[kStep];
+    cx<double> *const s_sum = reinterpret_cast<cx<double> *>(s_val); // after the last step
+    const int tid = threadIdx.x, part = tid / kRows;
+    double acc[2] = {0.0, 0.0};
+    for (int64_t r0 = int64_t(blockIdx.x) * kRows; r0 < rows; r0 += int64_t(gridDim.x) * kRows) {
+        const int64_t row = r0 + tid % kRows;
+        const bool live = row < rows;
+        const int64_t b = live ? int64_t(indptr[row]) : 0, e = live ? int64_t(indptr[row + 1]) : 0;
+        const int64_t kb = indptr[r0], ke = indptr[r0 + kRows < rows ? r0 + kRows : rows];
+        const cx<R> xr = live ? x[row] : cx<R>{R(0), R(0)};
+        double yr = 0.0, yi = 0.0;
+        for (int64_t k0 = kb; k0 < ke; k0 += kStep) {
+            const int n = int(ke - k0 < kStep ? ke - k0 : kStep);
+            cx<R> v[kCsrItems];
+            I col[kCsrItems];
+#pragma unroll
+            for (int q = 0; q < kCsrItems; ++q)
+                if (q * kBlock + tid < n) {
+                    col[q] = __builtin_nontemporal_load(indices + k0 + q * kBlock + tid);
+                    v[q] = ldnt(vals + k0 + q * kBlock + tid);
+                }
+            __syncthreads(); // the step before has been read
+#pragma unroll
+            for (int q = 0; q < kCsrItems; ++q)
+                if (q * kBlock + tid < n) {
+                    s_col[q * kBlock + tid] = col[q];
+                    s_val[q * kBlock + tid] = v[q];
+                }
+            __syncthreads();
+            const int lo = int((b > k0 ? b : k0) - k0), hi = int((e < k0 + n ? e : k0 + n) - k0);
+            for (int k = lo + part; k < hi; k += kAhead * T) {
+                cx<R> xv[kAhead], m[kAhead];
+#pragma unroll
+                for (int q = 0; q < kAhead; ++q) {
+                    const int at = k + q * T < hi ? k + q * T : k;
+                    xv[q] = x[s_col[at]];
+                    m[q] = s_val[at];
+                }
+#pragma unroll
+                for (int q = 0; q < kAhead; ++q)
+                    if (k + q * T < hi) {
+                        yr += double(m[q].re) * xv[q].re - double(m[q].im) * xv[q].im;
+                        yi += double(m[q].re) * xv[q].im + double(m[q].im) * xv[q].re;
+                    }
+            }
+        }
+        if (!y) { // every part on its own: the sum over rows takes them all
+            if (part == 0 || b + part < e) {
+                acc[0] += double(xr.re) * yr + double(xr.im) * yi;
+                acc[1] += double(xr.re) * yi - double(xr.im) * yr;
+            }
+            continue;
+        }
+        if constexpr (T > 1) {
+            __syncthreads();
+            s_sum[tid] = cx<double>{yr, yi};
+            __syncthreads();
+            if (part == 0)
+                for (int q = 1; q < T; ++q) {
+                    yr += s_sum[q * kRows + tid].re;
+                    yi += s_sum[q * kRows + tid].im;
+                }
+        }
+        if (live && part == 0) y[row] = cx<R>{R(yr), R(yi)};
+        __syncthreads();
+    }
+    if (y) return;
+    block_sum<2>(acc);
+    if (tid == 0) {
+        partials[blockIdx.x] = acc[0];
+        partials[gridDim.x + blockIdx.x] = acc[1];
+    }
+}
+
+// Longer rows: L lanes per row.
 template <class I, class R, int L>
 __global__ __launch_bounds__(kBlock) void k_csr(const I *__restrict__ indptr, const I *__restrict__ indices,
                                                 const cx<R> *__restrict__ vals, const cx<R> *__restrict__ x,
@@ -1604,21 +1713,48 @@ void pauli_noalloc_t(const lgh_sv *sv, int64_t nwords, const char *paulis, const
     *result = weighted_total(nwords, coeffs, vals, per_word);
 }
 
+// Host offsets or indices that fit 32 bits, narrowed on the device piece by
+// piece (on the host it took 13 ms of a 45 ms upload of 22 million entries).
+void upload_narrow(int device, int32_t *dst, const int64_t *src, int64_t count) {
+    if (count <= 0) return;
+    constexpr int64_t kPiece = int64_t(1) << 22;
+    const size_t bytes = sizeof(int64_t) * size_t(std::min(count, kPiece));
+    struct Piece {
+        int device;
+        size_t bytes;
+        void *p;
+        ~Piece() {
+            (void)hipStreamSynchronize(nullptr);
+            pool_free(device, p, bytes);
+        }
+    } piece{device, bytes, pool_alloc(device, bytes)};
+    for (int64_t at = 0; at < count; at += kPiece) {
+        const int64_t n = std::min(kPiece, count - at);
+        LGH_HIP(hipMemcpy(piece.p, src + at, sizeof(int64_t) * size_t(n), hipMemcpyHostToDevice));
+        hipLaunchKernelGGL(k_narrow, dim3(unsigned((n + kBlock - 1) / kBlock)), dim3(kBlock), 0, nullptr, dst + at,
+                           static_cast<const int64_t *>(piece.p), n);
+        LGH_LAUNCH_CHECK();
+    }
+}
+
 template <class I, class R>
 void csr_launch(const lgh_csr *csr, const cx<R> *x, cx<R> *y, StreamCtx *ctx, double *partials, unsigned blocks) {
     const I *ip = static_cast<const I *>(csr->indptr);
     const I *ix = static_cast<const I *>(csr->indices);
     const cx<R> *vv = static_cast<const cx<R> *>(csr->values);
     const double avg = csr->avg_row;
+    auto stream = [&](auto t) {
+        hipLaunchKernelGGL((k_csr_stream<I, R, decltype(t)::value>), dim3(blocks), dim3(kBlock), 0, ctx->stream, ip, ix,
+                           vv, x, y, csr->rows, partials);
+    };
     if (avg <= 6)
-        hipLaunchKernelGGL((k_csr<I, R, 4>), dim3(blocks), dim3(kBlock), 0, ctx->stream, ip, ix, vv, x, y, csr->rows,
-                           partials);
+        stream(std::integral_constant<int, 1>{});
     else if (avg <= 12)
-        hipLaunchKernelGGL((k_csr<I, R, 8>), dim3(blocks), dim3(kBlock), 0, ctx->stream, ip, ix, vv, x, y, csr->rows,
-                           partials);
+        stream(std::integral_constant<int, 2>{});
     else if (avg <= 24)
-        hipLaunchKernelGGL((k_csr<I, R, 16>), dim3(blocks), dim3(kBlock), 0, ctx->stream, ip, ix, vv, x, y,
-                           csr->rows, partials);
+        stream(std::integral_constant<int, 4>{});
+    else if (csr_streams<R>(avg))
+        stream(std::integral_constant<int, 8>{});
     else
         hipLaunchKernelGGL((k_csr<I, R, 32>), dim3(blocks), dim3(kBlock), 0, ctx->stream, ip, ix, vv, x, y,
                            csr->rows, partials);
@@ -1627,8 +1763,9 @@ void csr_launch(const lgh_csr *csr, const cx<R> *x, cx<R> *y, StreamCtx *ctx, do
 
 template <class R> void csr_run(const lgh_csr *csr, const lgh_sv *x, lgh_sv *y, double *re, double *im) {
     StreamCtx *ctx = x->ctx;
+    const int per_cu = csr_streams<R>(csr->avg_row) ? kCsrPerCu : 8;
     const unsigned blocks = unsigned(std::max<int64_t>(
-        1, std::min<int64_t>((csr->rows * 16 + kBlock - 1) / kBlock, int64_t(sm_count(x->device)) * 8)));
+        1, std::min<int64_t>((csr->rows * 16 + kBlock - 1) / kBlock, int64_t(sm_count(x->device)) * per_cu)));
     if (y) {
         if (csr->idx64)
             csr_launch<int64_t, R>(csr, cdata<R>(x), mdata<R>(y), ctx, nullptr, blocks);
@@ -1993,7 +2130,8 @@ lgh_status lgh_csr_create(lgh_csr **out, int device, lgh_dtype dtype, int64_t nu
         c->rows = num_rows;
         c->nnz = nnz;
         c->avg_row = double(nnz) / double(num_rows);
-        c->idx64 = dtype == LGH_C128 || num_rows >= (int64_t(1) << 31) || nnz >= (int64_t(1) << 31);
+        // 32-bit indices where they fit: a sixth of a complex128 matrix's bytes
+        c->idx64 = num_rows >= (int64_t(1) << 31) || nnz >= (int64_t(1) << 31);
         DeviceGuard g(device);
         const size_t isz = c->idx64 ? 8 : 4;
         c->b_ptr = isz * size_t(num_rows + 1);
@@ -2006,9 +2144,8 @@ lgh_status lgh_csr_create(lgh_csr **out, int device, lgh_dtype dtype, int64_t nu
             LGH_HIP(hipMemcpy(c->indptr, indptr, c->b_ptr, hipMemcpyHostToDevice));
             if (nnz) LGH_HIP(hipMemcpy(c->indices, indices, 8 * size_t(nnz), hipMemcpyHostToDevice));
         } else {
-            std::vector<int32_t> p(indptr, indptr + num_rows + 1), ix(indices, indices + nnz);
-            LGH_HIP(hipMemcpy(c->indptr, p.data(), c->b_ptr, hipMemcpyHostToDevice));
-            if (nnz) LGH_HIP(hipMemcpy(c->indices, ix.data(), 4 * size_t(nnz), hipMemcpyHostToDevice));
+            upload_narrow(device, static_cast<int32_t *>(c->indptr), indptr, num_rows + 1);
+            upload_narrow(device, static_cast<int32_t *>(c->indices), indices, nnz);
         }
         if (dtype == LGH_C128) {
             if (nnz) LGH_HIP(hipMemcpy(c->values, values, 16 * size_t(nnz), hipMemcpyHostToDevice));

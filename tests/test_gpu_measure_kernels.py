@@ -165,3 +165,43 @@ def test_pauli_words_by_flip_mask(n, dtype):
     # sums of 2^n products of total size 1
     np.testing.assert_allclose(per, ref, atol=2.0 ** (n / 2) * 4e-16, rtol=0)
     np.testing.assert_allclose(total, np.dot(np.arange(len(words)) * 0.01, ref), atol=2.0 ** (n / 2) * 4e-14, rtol=0)
+
+
+@pytest.mark.parametrize("dtype", [np.complex128, np.complex64])
+@pytest.mark.parametrize("n,avg", [(1, 1), (5, 3), (8, 6), (9, 7), (9, 12), (9, 13), (10, 24), (10, 25), (10, 47),
+                                   (11, 60)])
+@pytest.mark.parametrize("shape", ["even", "ragged", "one_long"])
+def test_csr_rows_of_every_length(n, avg, shape, dtype):
+    """<H> and H|x> with rows on both sides of each change of the number of
+    lanes per row: rows of one length, rows of 0 to twice the average, and one
+    row that runs over several steps of its workgroup among empty ones.  Sums
+    in double: relative to the sum of magnitudes, at most 2^16 terms of
+    2^-53 each, 1e-11; H|x> in complex64 is rounded once more (2^-24)."""
+    rng = np.random.default_rng(1000 * n + avg)
+    D = 1 << n
+    if shape == "even":
+        cnt = np.full(D, avg)
+    elif shape == "ragged":
+        cnt = rng.integers(0, 2 * avg + 1, D)
+    else:
+        cnt = np.zeros(D, dtype=np.int64)
+        cnt[D // 3] = avg * D
+    ip = np.zeros(D + 1, dtype=np.int64)
+    np.cumsum(cnt, out=ip[1:])
+    ix = rng.integers(0, D, ip[-1])
+    d = (rng.normal(size=ip[-1]) + 1j * rng.normal(size=ip[-1])).astype(dtype)
+    v = rng.normal(size=D) + 1j * rng.normal(size=D)
+    v = (v / np.linalg.norm(v)).astype(dtype)
+    H, x = N.CSR(ip, ix, d, dtype=dtype), N.State(n, dtype)
+    x.upload(v)
+    row = np.repeat(np.arange(D), cnt)
+    terms = d.astype(np.complex128) * v.astype(np.complex128)[ix]
+    y = np.bincount(row, terms.real, D) + 1j * np.bincount(row, terms.imag, D)
+    mag = np.bincount(row, np.abs(terms), D)
+    e = H.expval(x)
+    ref = np.vdot(v.astype(np.complex128), y)
+    assert abs(e - ref) <= 1e-11 * max(np.sum(np.abs(v) * mag), 1e-300)
+    out = N.State(n, dtype)
+    H.apply(out, x)
+    tol = 1e-11 if dtype == np.complex128 else 1e-11 + 2.0**-23
+    assert np.all(np.abs(out.download() - y) <= tol * np.maximum(mag, 1e-300))
