@@ -311,17 +311,20 @@ constexpr int kDiagNoReg = 7;
 template <class R> __device__ __forceinline__ cx<R> phase_cs(cx<R> x, R c, R s) {
     return cx<R>{c * x.re - s * x.im, c * x.im + s * x.re};
 }
-// Unit: c = 1 (its factor taken out by the host or the preparation kernel)
-template <class R, int NR, int B, bool Unit = false>
+template <class R, int NR, int B>
 __device__ __forceinline__ void diag_sym(const FOp &op, bool lpar, cx<R> (&v)[NR]) {
     const R c = R(op.m[1].re), s = R(op.m[1].im);
     const R s0 = flip(s, lpar ? 0u : kSignBit); // registers with even register parity
     const R s1 = flip(s, lpar ? kSignBit : 0u);
 #pragma unroll
-    for (int k = 0; k < NR; ++k) {
-        const R sk = (B >= 0 && ((k >> B) & 1)) ? s1 : s0;
-        v[k] = Unit ? ifma(sk, v[k], v[k]) : phase_cs(v[k], c, sk);
-    }
+    for (int k = 0; k < NR; ++k) v[k] = phase_cs(v[k], c, (B >= 0 && ((k >> B) & 1)) ? s1 : s0);
+}
+// c = 1: its factor taken out by the preparation kernel
+template <class R, int NR, int B>
+__device__ __forceinline__ void diag_sym_unit(const FOp &op, bool lpar, cx<R> (&v)[NR]) {
+    const R s = R(op.m[1].im), s0 = flip(s, lpar ? 0u : kSignBit), s1 = flip(s, lpar ? kSignBit : 0u);
+#pragma unroll
+    for (int k = 0; k < NR; ++k) v[k] = ifma((B >= 0 && ((k >> B) & 1)) ? s1 : s0, v[k], v[k]);
 }
 
 template <class R, int NR>
@@ -789,9 +792,13 @@ __device__ __forceinline__ double adj_diag_sym(const FOp &op, double ge, double 
     for (int k = 0; k < NR; ++k) {
         const bool odd = B >= 0 && ((k >> B) & 1);
         if constexpr (Gen) acc += (odd ? g1 : g0) * im_cdot2(b[k], a[k]);
-        const R sk = odd ? s1 : s0;
-        a[k] = Unit ? ifma(sk, a[k], a[k]) : phase_cs(a[k], c, sk);
-        b[k] = Unit ? ifma(sk, b[k], b[k]) : phase_cs(b[k], c, sk);
+        if constexpr (Unit) {
+            a[k] = ifma(odd ? s1 : s0, a[k], a[k]);
+            b[k] = ifma(odd ? s1 : s0, b[k], b[k]);
+        } else {
+            a[k] = phase_cs(a[k], c, odd ? s1 : s0);
+            b[k] = phase_cs(b[k], c, odd ? s1 : s0);
+        }
     }
     return acc;
 }
@@ -990,15 +997,15 @@ template <class R, int NR> __device__ __forceinline__ void scale_lean(const FOp 
 #pragma unroll
     for (int k = 0; k < NR; ++k) v[k] = rmul(c, v[k]);
 }
-template <class R, int NR, bool Unit> __device__ __forceinline__ void diag_lean(const FOp &op, bool lpar, cx<R> (&v)[NR]) {
+template <class R, int NR> __device__ __forceinline__ void diag_unit(const FOp &op, bool lpar, cx<R> (&v)[NR]) {
     switch (f_loc(op)) {
-    case 0: diag_sym<R, NR, 0, Unit>(op, lpar, v); return;
-    case 1: diag_sym<R, NR, 1, Unit>(op, lpar, v); return;
-    case 2: diag_sym<R, NR, 2, Unit>(op, lpar, v); return;
+    case 0: diag_sym_unit<R, NR, 0>(op, lpar, v); return;
+    case 1: diag_sym_unit<R, NR, 1>(op, lpar, v); return;
+    case 2: diag_sym_unit<R, NR, 2>(op, lpar, v); return;
     case 3:
-        if constexpr (NR > 8) diag_sym<R, NR, 3, Unit>(op, lpar, v);
+        if constexpr (NR > 8) diag_sym_unit<R, NR, 3>(op, lpar, v);
         return;
-    default: diag_sym<R, NR, -1, Unit>(op, lpar, v); return;
+    default: diag_sym_unit<R, NR, -1>(op, lpar, v); return;
     }
 }
 // Unit: diagonal gates may come in their unit form (batched kernel)
@@ -1012,12 +1019,19 @@ __device__ __forceinline__ void apply_lean(const FOp &op, int lane, uint64_t bas
         const bool lpar = __popcll(base & op.pm_rest) & 1;
         if constexpr (Unit) {
             if (f_rot(op)) {
-                diag_lean<R, NR, true>(op, lpar, v);
+                diag_unit<R, NR>(op, lpar, v);
                 return;
             }
         }
-        diag_lean<R, NR, false>(op, lpar, v);
-        return;
+        switch (f_loc(op)) {
+        case 0: diag_sym<R, NR, 0>(op, lpar, v); return;
+        case 1: diag_sym<R, NR, 1>(op, lpar, v); return;
+        case 2: diag_sym<R, NR, 2>(op, lpar, v); return;
+        case 3:
+            if constexpr (NR > 8) diag_sym<R, NR, 3>(op, lpar, v);
+            return;
+        default: diag_sym<R, NR, -1>(op, lpar, v); return;
+        }
     }
     const M2<R> m = m2<R>(op);
     const int loc = f_loc(op), rot = f_rot(op);
