@@ -641,6 +641,10 @@ __global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 3 : 1) void k
     fused_adj_body<R, 4, Lv>(arrays, ntiles, chunk, pd, ops, gens, partials, partials_stride, from_src, bra_from_lam);
 }
 
+// Slots summed by one store: those of up to eight passes (4 MiB of partial
+// sums per sweep at most).
+constexpr int kStoreSlots = 4 * kMaxSlotsSv4;
+
 // slot sums -> jac[row][col[s]] * factor[s]; blockIdx.y: the sweep
 __global__ __launch_bounds__(kBlock) void k_slot_store(const double *__restrict__ partials_all,
                                                        uint64_t partials_stride, int nparts, int nslots,
@@ -652,15 +656,25 @@ __global__ __launch_bounds__(kBlock) void k_slot_store(const double *__restrict_
     if (s >= nslots) return;
     const double *__restrict__ partials = partials_all + blockIdx.y * partials_stride;
     double *__restrict__ jac = arrays[blockIdx.y].jac_row;
+    const int64_t col = cols[s];
+    const double fac = factors[s];
     double v = 0.0;
-    for (int b = threadIdx.x; b < nparts; b += kBlock) v += partials[size_t(s) * nparts + b];
+    // loads of four rounds in flight, added in order
+    for (int b = threadIdx.x; b < nparts; b += 4 * kBlock) {
+        double t[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) t[q] = b + q * kBlock < nparts ? partials[size_t(s) * nparts + b + q * kBlock] : 0.0;
+#pragma unroll
+        for (int q = 0; q < 4; ++q)
+            if (b + q * kBlock < nparts) v += t[q];
+    }
     v = wave_sum(v);
     if ((threadIdx.x & 63) == 0) sh[threadIdx.x >> 6] = v;
     __syncthreads();
     if (threadIdx.x == 0) {
         double t = 0.0;
         for (int q = 0; q < kWavesPerBlock; ++q) t += sh[q];
-        jac[cols[s]] = factors[s] * t;
+        jac[col] = fac * t;
     }
 }
 
@@ -1226,6 +1240,19 @@ AdjPasses::AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std
         if (bytes) std::memcpy(blob.data() + at, src, bytes);
         return at;
     };
+    // The overlaps of consecutive fused passes are summed and stored together,
+    // as many slots as the partials hold: one store per sweep instead of one
+    // behind every pass, which cost the pass's stream 10 us on 24 qubits.
+    std::vector<int64_t> cols;
+    std::vector<double> facs;
+    auto close = [&](Step &st) { // the store runs after st
+        st.nslots = int(cols.size());
+        st.o_cols = put(cols.data(), cols.size() * 8);
+        st.o_facs = put(facs.data(), facs.size() * 8);
+        cols.clear();
+        facs.clear();
+    };
+    int last_fused = -1; // the step whose store the pending slots wait for
     for (auto it = passes->rbegin(); it != passes->rend(); ++it) {
         Step st;
         if (it->standalone) {
@@ -1234,7 +1261,9 @@ AdjPasses::AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std
                 st.op = i;
             } else {
                 // a run's partial sums, a row of one double per workgroup for
-                // every trainable gate, fit the partials of a fused pass
+                // every trainable gate, fit the partials; the fused passes
+                // before it have been stored
+                if (!cols.empty()) close(steps_[size_t(last_fused)]);
                 size_t room = fused_partials_bytes(n_, device_) / sizeof(double);
                 for (auto next = it; next != passes->rend() && next->standalone; ++next) {
                     const size_t g = size_t(next->ops[0]);
@@ -1250,23 +1279,21 @@ AdjPasses::AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std
                 }
                 if (st.pairs.empty()) st.op = i;
             }
-            std::vector<int64_t> cols;
-            std::vector<double> facs;
-            for (int g : st.pairs)
-                if (slot_col[size_t(g)] >= 0) {
-                    cols.push_back(slot_col[size_t(g)]);
-                    facs.push_back(factor[size_t(g)]);
-                }
-            st.nslots = int(cols.size());
-            st.o_cols = put(cols.data(), cols.size() * 8);
-            st.o_facs = put(facs.data(), facs.size() * 8);
+            if (!st.pairs.empty()) {
+                for (int g : st.pairs)
+                    if (slot_col[size_t(g)] >= 0) {
+                        cols.push_back(slot_col[size_t(g)]);
+                        facs.push_back(factor[size_t(g)]);
+                    }
+                close(st);
+            }
             steps_.push_back(st);
             continue;
         }
         const Built b = build_pass(*it, udag, n_, true, &gens, &slot_col, rb_, true, true, dtype_ == LGH_C64);
         LGH_REQUIRE(b.pd.nslots <= adj_slot_cap(rb_), "fused adjoint pass: more trainable gates than LDS slots");
-        std::vector<int64_t> cols;
-        std::vector<double> facs;
+        if (cols.size() + b.slot_ops.size() > size_t(kStoreSlots)) close(steps_[size_t(last_fused)]);
+        st.row = int(cols.size());
         for (size_t s = 0; s < b.slot_ops.size(); ++s) {
             const int oi = b.slot_ops[s];
             cols.push_back(slot_col[size_t(oi)]);
@@ -1275,12 +1302,11 @@ AdjPasses::AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std
         st.o_desc = put(&b.pd, sizeof(PassDesc));
         st.o_ops = put(b.ops.data(), b.ops.size() * sizeof(FOp));
         st.o_gens = put(b.gens.data(), b.gens.size() * sizeof(FGen));
-        st.o_cols = put(cols.data(), cols.size() * 8);
-        st.o_facs = put(facs.data(), facs.size() * 8);
-        st.nslots = int(cols.size());
         st.level = g_lean.load() ? lean_level(b.ops, true) : 0;
+        last_fused = int(steps_.size());
         steps_.push_back(st);
     }
+    if (!cols.empty()) close(steps_[size_t(last_fused)]);
     if (blob.empty()) return;
     bytes_ = blob.size();
     dev_ = static_cast<unsigned char *>(pool_alloc(device_, bytes_));
@@ -1364,7 +1390,8 @@ void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void 
             hipLaunchKernelGGL(kern, dim3(geo.blocks, unsigned(count)), dim3(kBlock), 0, ctx_->stream, dtab, geo.ntiles,
                                geo.chunk, reinterpret_cast<const PassDesc *>(dev_ + st.o_desc),
                                reinterpret_cast<const FOp *>(dev_ + st.o_ops),
-                               reinterpret_cast<const FGen *>(dev_ + st.o_gens), partials, stride, int(src),
+                               reinterpret_cast<const FGen *>(dev_ + st.o_gens),
+                               partials + uint64_t(st.row) * geo.blocks, stride, int(src),
                                int(from_z));
             from_z = src = false;
             LGH_LAUNCH_CHECK();
@@ -1384,8 +1411,8 @@ void AdjPasses::run(const AdjSweep *sweeps, int count, double *partials, void *t
 size_t fused_partials_bytes(int n, int device) {
     // sized for the smaller tile, which has more workgroups
     if (n < kLaneBits + 3) return 0;
-    // the most slots of any tile height times the most blocks (three register bits)
-    return sizeof(double) * size_t(kMaxSlotsSv4) * geometry(n, device, 3, kMaxWavesPerCUAdjoint).blocks;
+    // the slots of one store times the most blocks (three register bits)
+    return sizeof(double) * size_t(kStoreSlots) * geometry(n, device, 3, kMaxWavesPerCUAdjoint).blocks;
 }
 
 } // namespace lgh

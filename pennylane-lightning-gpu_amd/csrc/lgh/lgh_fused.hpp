@@ -117,7 +117,9 @@ class AdjPasses {
         int op = -1;              // a gate on its own, or -1
         unsigned blocks = 0;      // workgroups of each of the run's trainable gates
         size_t o_ops = 0, o_gens = 0, o_cols = 0, o_facs = 0, o_desc = 0;
-        int nslots = 0, level = 0;
+        int row = 0;              // a fused pass's first row of partials
+        int nslots = 0;           // slots stored after this step, of it and of passes before it
+        int level = 0;
     };
     template <class R>
     void run_t(const AdjSweep *sweeps, int count, double *partials, void *table, const StandaloneStep &s) const;
