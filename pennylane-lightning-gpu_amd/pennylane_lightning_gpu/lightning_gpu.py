@@ -50,16 +50,6 @@ _SHOTS_WARNING = ("Requested adjoint differentiation to be computed with finite 
                   "exact when using the adjoint differentiation method.")
 
 
-def _real_pauli_sum(observable):
-    """Every term a product of Paulis on distinct wires, every coefficient real."""
-    for word in observable.ops:
-        names = word.name if isinstance(word.name, list) else [word.name]
-        wires = list(word.wires)
-        if any(nm not in _name_map for nm in names) or len(names) != len(wires) or len(set(wires)) != len(wires):
-            return False
-    return len(observable.ops) > 0 and not np.iscomplexobj(np.asarray(observable.coeffs))
-
-
 class DeviceError(Exception):
     """Invalid use of the device (mirrors pennylane.DeviceError)."""
 
@@ -238,13 +228,7 @@ class LightningGPU:
                                                     np.asarray(csr.data, dtype=self.C_DTYPE))
         if observable.name == "Hamiltonian":
             device_wires = self.map_wires(observable.wires)
-            # Few wires: the matrix, unless every term is a Pauli word with a
-            # real coefficient, whose kernel reads the state and no matrix.
-            # 8 words on 10, 12 and 13 wires, complex128: 38 ms, 1.0 s and 4.0
-            # s through the matrix (nearly all of it spent on forming it),
-            # 0.13 ms for the whole execution through the words.  complex64 keeps
-            # the matrix, whose entries are rounded after they are summed.
-            if len(device_wires) < 14 and (self.use_csingle or not _real_pauli_sum(observable)):
+            if len(device_wires) < 14:
                 return self._gpu_state.ExpectationValue(device_wires,
                                                         np.asarray(observable.matrix(), self.C_DTYPE).ravel())
             pauli_words, word_wires = [], []

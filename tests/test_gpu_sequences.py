@@ -121,29 +121,3 @@ def test_gates_on_pairs_of_basis_states(n):
         np.testing.assert_allclose(dev.state, psi, atol=1e-13, rtol=0)
         single = LightningGPU(n, c_dtype=np.complex64)
         np.testing.assert_allclose(np.array(single.adjoint_jacobian(tape)), ref, atol=2e-5, rtol=0)
-
-
-@pytest.mark.parametrize("n", [1, 2, 5, 9, 12])
-@pytest.mark.parametrize("terms", ["paulis", "identity", "mixed"])
-def test_hamiltonians_of_few_wires(n, terms):
-    """<H> of at most 13 wires: Pauli words (identities among them) go to the
-    word kernel, sums with any other term to the matrix; both against the
-    dense matrix on the state in 64 bits (sums of at most 2^12 terms of order
-    one: 1e-11)."""
-    from pennylane_lightning_gpu import circuit as qc
-    from pennylane_lightning_gpu.lightning_gpu import LightningGPU
-    rng = np.random.default_rng(n)
-    make = [qc.PauliX, qc.PauliY, qc.PauliZ, qc.Identity]
-    ops = [make[int(rng.integers(3))](w) for w in range(n)]
-    ops.append(qc.Tensor(*[make[int(rng.integers(4))](w) for w in range(n)]) if n > 1 else qc.PauliY(0))
-    if terms == "identity":
-        ops.append(qc.Identity(n - 1))
-    if terms == "mixed":
-        ops.append(qc.Hadamard(0))
-    H = qc.Hamiltonian(rng.normal(size=len(ops)), ops)
-    gates = [qc.Operation(g, [w], [float(rng.uniform(0, 6))]) for w in range(n) for g in ("RX", "RY", "RZ")]
-    dev = LightningGPU(n)
-    got = dev.execute(qc.QuantumTape(gates, [qc.expval(H)]))
-    psi = np.asarray(dev.state).ravel()
-    want = np.vdot(psi, H.matrix() @ psi).real if list(H.wires) == list(range(n)) else None
-    assert want is not None and abs(float(np.squeeze(got)) - want) <= 1e-11 * max(1.0, np.abs(H.coeffs).sum())
