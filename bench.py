@@ -280,7 +280,7 @@ def bench_measurements(N, args):
     timer = StreamTimer(st.stream())
     ms = sorted(timer.time(lambda: csr.expval(st)) for _ in range(5))[2]
     nnz, NN = len(data), 1 << n
-    cbytes = 24 * nnz + 8 * (NN + 1) + 16 * NN
+    cbytes = 20 * nnz + 4 * (NN + 1) + 16 * NN  # 32-bit indices
     out["csr_tfim"] = {"qubits": n, "nnz": nnz, "ms": round(ms, 3), "bytes": cbytes,
                        "GBps": round(cbytes / (ms * 1e-3) / 1e9, 1)}
     del st, csr
