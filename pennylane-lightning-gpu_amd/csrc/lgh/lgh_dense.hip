@@ -244,20 +244,31 @@ template <class R> void dense_apply_t(lgh_sv *sv, const KOp &op) {
     const size_t mbytes = sizeof(cx<double>) * D * D;
     const bool small = mbytes <= kSmallMatrix, whole = op.k <= 6;
     const uint64_t chunk = std::min<uint64_t>(g.ngroups, std::max<uint64_t>(32, kDenseTmp / D));
-    char *ws = nullptr;
-    const size_t o_tmp = small ? 0 : al256(mbytes);
-    if (!small || !whole) ws = static_cast<char *>(ctx->workspace(o_tmp + (whole ? 0 : sizeof(cx<R>) * chunk * D)));
+    // Neither buffer is the workspace, which the adjoint sweep holds while it
+    // applies a gate.  The rows' is bounded (64 MiB) and kept; a large
+    // matrix's is given back once the stream has passed it.
+    struct Matrix {
+        StreamCtx *ctx;
+        size_t bytes;
+        void *p = nullptr;
+        ~Matrix() {
+            if (!p) return;
+            (void)hipStreamSynchronize(ctx->stream);
+            pool_free(ctx->device, p, bytes);
+        }
+    } large{ctx, mbytes};
     const cx<double> *mat;
     if (small) {
         mat = static_cast<const cx<double> *>(ctx->upload(op.mat.data(), mbytes));
     } else {
-        LGH_HIP(hipMemcpyAsync(ws, op.mat.data(), mbytes, hipMemcpyHostToDevice, ctx->stream));
-        mat = reinterpret_cast<const cx<double> *>(ws);
+        large.p = pool_alloc(ctx->device, mbytes);
+        LGH_HIP(hipMemcpyAsync(large.p, op.mat.data(), mbytes, hipMemcpyHostToDevice, ctx->stream));
+        mat = static_cast<const cx<double> *>(large.p);
     }
     if (whole) {
         dense_launch<R, 0>(ctx->stream, data, data, mat, nullptr, g);
     } else {
-        cx<R> *tmp = reinterpret_cast<cx<R> *>(ws + o_tmp);
+        cx<R> *tmp = static_cast<cx<R> *>(ctx->gate_scratch(sizeof(cx<R>) * chunk * D));
         for (uint64_t c = 0; c < g.ngroups; c += chunk) {
             g.col0 = c;
             g.ncols = std::min(chunk, g.ngroups - c);

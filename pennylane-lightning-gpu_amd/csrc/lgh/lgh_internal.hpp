@@ -239,6 +239,8 @@ struct StreamCtx {
 
     void *ws = nullptr;   // device workspace
     size_t ws_bytes = 0;
+    void *gs = nullptr;   // device scratch of a gate
+    size_t gs_bytes = 0;
     void *host = nullptr; // pinned host staging for results
     size_t host_bytes = 0;
 
@@ -248,7 +250,13 @@ struct StreamCtx {
     size_t up_off = 0;
 
     void ring_room(size_t need);
+    // One caller's at a time: what an entry point holds there is lost when
+    // anything it calls asks for the workspace too.
     void *workspace(size_t bytes);
+    // Scratch of one gate (launch_kop), apart from the workspace: the adjoint
+    // sweep keeps its partial sums, Jacobian and pointer tables in that one
+    // while it applies gates.
+    void *gate_scratch(size_t bytes);
     void *host_buffer(size_t bytes);
     // Copies `bytes` from host memory into the device ring (stream ordered)
     // and returns the device address.  Valid until the ring wraps, which

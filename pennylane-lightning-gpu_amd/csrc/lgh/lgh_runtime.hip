@@ -232,11 +232,12 @@ StreamCtx *acquire_ctx(int device, hipStream_t stream) {
 static void free_ctx_buffers(StreamCtx *c) {
     DeviceGuard g(c->device);
     if (c->ws) (void)hipFree(c->ws);
+    if (c->gs) (void)hipFree(c->gs);
     if (c->host) (void)hipHostFree(c->host);
     if (c->up_host) (void)hipHostFree(c->up_host);
     if (c->up_dev) (void)hipFree(c->up_dev);
-    c->ws = c->host = c->up_host = c->up_dev = nullptr;
-    c->ws_bytes = c->host_bytes = c->up_bytes = c->up_off = 0;
+    c->ws = c->gs = c->host = c->up_host = c->up_dev = nullptr;
+    c->ws_bytes = c->gs_bytes = c->host_bytes = c->up_bytes = c->up_off = 0;
 }
 
 void release_ctx(StreamCtx *c) {
@@ -263,6 +264,18 @@ void *StreamCtx::workspace(size_t bytes) {
     LGH_HIP(hipMalloc(&ws, nb));
     ws_bytes = nb;
     return ws;
+}
+
+void *StreamCtx::gate_scratch(size_t bytes) {
+    if (bytes <= gs_bytes) return gs;
+    DeviceGuard g(device);
+    sync();
+    if (gs) LGH_HIP(hipFree(gs));
+    gs = nullptr;
+    gs_bytes = 0;
+    LGH_HIP(hipMalloc(&gs, bytes));
+    gs_bytes = bytes;
+    return gs;
 }
 
 void *StreamCtx::host_buffer(size_t bytes) {
