@@ -532,6 +532,12 @@ __global__ __launch_bounds__(kBlock) void k_pauli_add(cx<R> *__restrict__ dst, c
     dst[i] = cx<R>{R(y.re), R(y.im)};
 }
 
+// The sum without words.  Written, not scaled: dst may hold infinities and NaN.
+template <class R> __global__ __launch_bounds__(kBlock) void k_zero(cx<R> *__restrict__ dst, uint64_t len) {
+    const uint64_t i = uint64_t(blockIdx.x) * kBlock + threadIdx.x;
+    if (i < len) stnt(dst + i, cx<R>{R(0), R(0)});
+}
+
 // ---------------------------------------------------------------- CSR
 
 // Short rows (see csr_streams): a workgroup takes kBlock / T consecutive rows,
@@ -1628,8 +1634,8 @@ void pauli_sum_t(lgh_sv *dst, const lgh_sv *src, int64_t nwords, const char *pau
         add = 1;
     }
     if (!add) { // no words
-        hipLaunchKernelGGL(k_scale<R>, dim3(unsigned((len + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
-                           mdata<R>(dst), len, cx<R>{R(0), R(0)});
+        hipLaunchKernelGGL(k_zero<R>, dim3(unsigned((len + kBlock - 1) / kBlock)), dim3(kBlock), 0, ctx->stream,
+                           mdata<R>(dst), len);
         LGH_LAUNCH_CHECK();
     }
 }
