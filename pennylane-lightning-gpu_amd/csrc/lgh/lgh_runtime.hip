@@ -10,6 +10,7 @@
 #include <cstring>
 #include <map>
 #include <unordered_map>
+#include <utility>
 
 #include <cstdlib>
 
@@ -140,6 +141,26 @@ size_t size_class(size_t bytes) {
     return (bytes + step - 1) / step * step;
 }
 
+// hipMalloc that first gives back what the pool caches when memory is short.
+static void *device_alloc(int device, size_t bytes) {
+    DeviceGuard g(device);
+    void *ptr = nullptr;
+    hipError_t e = hipMalloc(&ptr, bytes);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        Pool &p = pool();
+        std::lock_guard<std::mutex> lk(p.mu);
+        trim_locked(p, device);
+        e = hipMalloc(&ptr, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        throw Error(e == hipErrorOutOfMemory ? LGH_ERR_OUT_OF_MEMORY : LGH_ERR_DEVICE,
+                    "hipMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
+    }
+    return ptr;
+}
+
 void *pool_alloc(int device, size_t bytes) {
     bytes = size_class(bytes);
     Pool &p = pool();
@@ -153,21 +174,7 @@ void *pool_alloc(int device, size_t bytes) {
             return ptr;
         }
     }
-    DeviceGuard g(device);
-    void *ptr = nullptr;
-    hipError_t e = hipMalloc(&ptr, bytes);
-    if (e == hipErrorOutOfMemory) {
-        (void)hipGetLastError();
-        std::lock_guard<std::mutex> lk(p.mu);
-        trim_locked(p, device);
-        e = hipMalloc(&ptr, bytes);
-    }
-    if (e != hipSuccess) {
-        (void)hipGetLastError();
-        throw Error(e == hipErrorOutOfMemory ? LGH_ERR_OUT_OF_MEMORY : LGH_ERR_DEVICE,
-                    "hipMalloc of " + std::to_string(bytes) + " bytes failed: " + hipGetErrorString(e));
-    }
-    return ptr;
+    return device_alloc(device, bytes);
 }
 
 void pool_free(int device, void *ptr, size_t bytes) {
@@ -254,15 +261,26 @@ void release_ctx(StreamCtx *c) {
 
 void StreamCtx::sync() { LGH_HIP(hipStreamSynchronize(stream)); }
 
+// A stream's buffers grow by giving the old one back first.  Their sizes are
+// those of memory that is there: zero from before an allocation that may fail
+// until it has succeeded, so that a smaller request after a failed one
+// allocates again.
 void *StreamCtx::workspace(size_t bytes) {
     if (bytes <= ws_bytes) return ws;
     DeviceGuard g(device);
     sync();
-    if (ws) LGH_HIP(hipFree(ws));
-    ws = nullptr;
-    size_t nb = std::max<size_t>(bytes, std::max<size_t>(ws_bytes * 3 / 2, 1 << 20));
-    LGH_HIP(hipMalloc(&ws, nb));
-    ws_bytes = nb;
+    const size_t nb = std::max<size_t>(bytes, std::max<size_t>(ws_bytes * 3 / 2, 1 << 20));
+    void *old = std::exchange(ws, nullptr);
+    ws_bytes = 0;
+    if (old) LGH_HIP(hipFree(old));
+    try {
+        ws = device_alloc(device, nb);
+        ws_bytes = nb;
+    } catch (const Error &e) {
+        if (nb == bytes || e.code != LGH_ERR_OUT_OF_MEMORY) throw;
+        ws = device_alloc(device, bytes); // without room to grow
+        ws_bytes = bytes;
+    }
     return ws;
 }
 
@@ -270,22 +288,32 @@ void *StreamCtx::gate_scratch(size_t bytes) {
     if (bytes <= gs_bytes) return gs;
     DeviceGuard g(device);
     sync();
-    if (gs) LGH_HIP(hipFree(gs));
-    gs = nullptr;
+    void *old = std::exchange(gs, nullptr);
     gs_bytes = 0;
-    LGH_HIP(hipMalloc(&gs, bytes));
+    if (old) LGH_HIP(hipFree(old));
+    gs = device_alloc(device, bytes);
     gs_bytes = bytes;
     return gs;
+}
+
+// Pinned host memory; a failed call leaves no error behind for the next launch check.
+static void *pinned_alloc(size_t bytes) {
+    void *p = nullptr;
+    const hipError_t e = hipHostMalloc(&p, bytes, hipHostMallocDefault);
+    if (e != hipSuccess) (void)hipGetLastError();
+    LGH_HIP(e);
+    return p;
 }
 
 void *StreamCtx::host_buffer(size_t bytes) {
     if (bytes <= host_bytes) return host;
     DeviceGuard g(device);
     sync();
-    if (host) LGH_HIP(hipHostFree(host));
-    host = nullptr;
-    size_t nb = std::max<size_t>(bytes, 1 << 16);
-    LGH_HIP(hipHostMalloc(&host, nb, hipHostMallocDefault));
+    const size_t nb = std::max<size_t>(bytes, 1 << 16);
+    void *old = std::exchange(host, nullptr);
+    host_bytes = 0;
+    if (old) LGH_HIP(hipHostFree(old));
+    host = pinned_alloc(nb);
     host_bytes = nb;
     return host;
 }
@@ -294,14 +322,19 @@ void *StreamCtx::host_buffer(size_t bytes) {
 void StreamCtx::ring_room(size_t need) {
     if (need > up_bytes) {
         sync();
-        if (up_host) LGH_HIP(hipHostFree(up_host));
-        if (up_dev) LGH_HIP(hipFree(up_dev));
-        up_host = up_dev = nullptr;
-        size_t nb = std::max<size_t>(need, 4 << 20);
-        LGH_HIP(hipHostMalloc(&up_host, nb, hipHostMallocDefault));
-        LGH_HIP(hipMalloc(&up_dev, nb));
+        const size_t nb = std::max<size_t>(need, 4 << 20);
+        void *old_host = std::exchange(up_host, nullptr), *old_dev = std::exchange(up_dev, nullptr);
+        up_bytes = up_off = 0;
+        if (old_host) LGH_HIP(hipHostFree(old_host));
+        if (old_dev) LGH_HIP(hipFree(old_dev));
+        up_host = pinned_alloc(nb);
+        try {
+            up_dev = device_alloc(device, nb);
+        } catch (...) {
+            (void)hipHostFree(std::exchange(up_host, nullptr));
+            throw;
+        }
         up_bytes = nb;
-        up_off = 0;
     }
     if (up_off + need > up_bytes) {
         sync(); // every earlier copy out of the ring has completed
