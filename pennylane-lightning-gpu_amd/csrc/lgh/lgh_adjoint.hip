@@ -27,8 +27,10 @@ namespace {
 constexpr int kBlock = 256;
 constexpr int kWaves = kBlock / 64;
 constexpr int kBras = 8; // observable states per launch
-// bytes of lambda and observable states of the fused sweeps that run side by side
-constexpr size_t kSideBySide = size_t(4) << 30;
+// bytes of lambda and partial sums of the fused sweeps that run side by side
+constexpr size_t kSideBySide = size_t(9) << 28;
+// groups of more than this ask how much memory is free
+constexpr size_t kSideBySideAsk = size_t(64) << 20;
 
 __device__ __forceinline__ double wave_sum(double v) {
 #pragma unroll
@@ -484,12 +486,17 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
         const lgh_sv *like;
         std::vector<void *> ptrs;
         void *take() {
+            ptrs.reserve(ptrs.size() + 1);
             ptrs.push_back(pool_alloc(like->device, like->bytes));
             return ptrs.back();
         }
+        // gives back all but the first `keep`, none of which has been used yet
+        void trim(size_t keep) {
+            for (; ptrs.size() > keep; ptrs.pop_back()) pool_free(like->device, ptrs.back(), like->bytes);
+        }
         ~Buffers() {
             (void)hipStreamSynchronize(like->ctx->stream);
-            for (void *p : ptrs) pool_free(like->device, p, like->bytes);
+            trim(0);
         }
     } buffers{psi_in, {}};
     // The fused sweep reads lambda's starting values from psi itself when no
@@ -513,11 +520,22 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
     // <Z_w> on every wire, complex128, one sweep after another and side by
     // side: 12 qubits 3180 and 570 us (the sweeps of a 4-layer ring circuit),
     // 18 qubits 3329 and 1269, 20 qubits 4677 and 2785, 22 qubits 12.3 and
-    // 10.0 ms, 24 qubits 43 and 40.5 ms.  The limit bounds the memory: a
-    // lambda for each sweep of a group, half of it.
+    // 10.0 ms, 24 qubits 43 and 40.5 ms.  The limit bounds what the call itself
+    // takes for them, a lambda and the partial sums of each; a group that
+    // needs much takes at most half of the memory that is free, so that the
+    // rest is left to the runtime and to other streams.
+    const size_t b_one = fused_path ? fused_partials_bytes(n, psi_in->device) : 0;
+    const size_t per_sweep = psi_in->bytes + b_one + AdjPasses::kTableBytes;
     int group = fused_path ? int(std::max<size_t>(1, std::min<size_t>({size_t(nobs), size_t(65535),
-                                                                             kSideBySide / (2 * psi_in->bytes)})))
+                                                                             kSideBySide / per_sweep})))
                                  : 1;
+    if (size_t(group) * per_sweep > kSideBySideAsk) {
+        size_t free_bytes = 0, total_bytes = 0;
+        if (hipMemGetInfo(&free_bytes, &total_bytes) == hipSuccess)
+            group = int(std::max<size_t>(1, std::min<size_t>(size_t(group), free_bytes / 2 / per_sweep)));
+        else
+            (void)hipGetLastError();
+    }
     // workspace: [jac (nobs*ntp) | bra pointers | partials of the steps | slices | fused partials | sweep table]
     // the widest step shape has one thread per amplitude
     const unsigned max_blocks = unsigned(((1ull << n) + kBlock - 1) / kBlock);
@@ -528,9 +546,24 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
     // the fused path's standalone steps take one observable at a time
     const size_t b_part = al(sizeof(double) * (fused_path ? 1 : size_t(nbatches) * kBras) * max_blocks);
     const size_t b_slices = al(sizeof(double) * kBras * kSlices);
-    const size_t b_fused = al(fused_partials_bytes(n, psi_in->device) * size_t(group));
-    const size_t b_tab = fused_path ? al(AdjPasses::kTableBytes * size_t(group)) : 0;
-    char *ws = static_cast<char *>(ctx->workspace(b_jac + b_ptr + b_part + b_slices + b_fused + b_tab));
+    // lambda per sweep of a group; a single sweep may use up the forward state formed above
+    const bool own = fused_path && apply_ops && nobs == 1;
+    const size_t held = buffers.ptrs.size();
+    size_t b_fused = 0;
+    char *ws = nullptr;
+    for (;;) {
+        b_fused = al(b_one * size_t(group));
+        const size_t b_tab = fused_path ? al(AdjPasses::kTableBytes * size_t(group)) : 0;
+        try {
+            while (fused_path && !own && buffers.ptrs.size() < held + size_t(group)) (void)buffers.take();
+            ws = static_cast<char *>(ctx->workspace(b_jac + b_ptr + b_part + b_slices + b_fused + b_tab));
+            break;
+        } catch (const Error &e) {
+            if (group == 1 || e.code != LGH_ERR_OUT_OF_MEMORY) throw;
+            group /= 2; // what memory is left takes fewer at a time
+            buffers.trim(held + size_t(group));
+        }
+    }
     double *jac_dev = reinterpret_cast<double *>(ws);
     cx<R> **bras_dev = reinterpret_cast<cx<R> **>(ws + b_jac);
     double *partials = reinterpret_cast<double *>(ws + b_jac + b_ptr);
@@ -571,17 +604,8 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
             slot.push_back(col);
         }
         const AdjPasses passes(psi_in, udag, gens, slot, fac);
-        // lambda per sweep of a group; a single sweep may use up the forward state formed above
         std::vector<lgh_sv> lams(size_t(group), *psi_in);
-        const bool own = apply_ops && nobs == 1;
-        for (int j = 0; j < group; ++j) {
-            try {
-                lams[size_t(j)].data = own ? lam.data : buffers.take();
-            } catch (const Error &e) {
-                if (j == 0 || e.code != LGH_ERR_OUT_OF_MEMORY) throw;
-                group = j; // what memory is left takes fewer at a time
-            }
-        }
+        for (int j = 0; j < group; ++j) lams[size_t(j)].data = own ? lam.data : buffers.ptrs[held + size_t(j)];
         auto standalone = [&](const AdjSweep &sw, const KOp &u, const KGen *g, int64_t col, double f) {
             const bool fusedk = u.kind == KOp::DIAG || (u.kind == KOp::DENSE && (u.k == 1 || u.k == 2 || u.k == 4));
             if (!fusedk) {

@@ -641,8 +641,9 @@ __global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 3 : 1) void k
     fused_adj_body<R, 4, Lv>(arrays, ntiles, chunk, pd, ops, gens, partials, partials_stride, from_src, bra_from_lam);
 }
 
-// Slots summed by one store: those of up to eight passes (4 MiB of partial
-// sums per sweep at most).
+// Slots summed by one store: those of up to eight passes.  3 KiB of partial
+// sums per sweep and workgroup of the pass's grid: 12.6 MB on 23 qubits, 100 MB
+// on 26 and more (256 CUs), next to 128 MB and 1 GiB of lambda.
 constexpr int kStoreSlots = 4 * kMaxSlotsSv4;
 
 // slot sums -> jac[row][col[s]] * factor[s]; blockIdx.y: the sweep

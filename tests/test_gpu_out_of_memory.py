@@ -1,5 +1,6 @@
 """A call that asks for more device memory than there is fails with an
-out-of-memory error, and the calls after it work."""
+out-of-memory error, and the calls after it work; sweeps side by side take a
+bounded amount of memory."""
 import numpy as np
 import pytest
 
@@ -29,3 +30,20 @@ def test_calls_after_a_failed_workspace_request():
     assert total == pytest.approx(np.cos(0.4) + 2 * np.cos(0.2), abs=1e-14)
     got = N.adjoint_jacobian(psi, [N.State(n).set_pauli_word_of(psi, "Z", [0])], ops, [0, 1])
     np.testing.assert_allclose(got, [[-np.sin(0.4), 0.0]], atol=1e-14, rtol=0)
+
+
+def test_memory_of_sweeps_side_by_side():
+    """300 observables of 20 qubits: what the call takes, a lambda and partial sums per sweep, stays below 2.25 GiB
+    (and 64 MiB for what does not depend on the number of sweeps)."""
+    n, nobs = 20, 300
+    ops = [("RY", [w], [0.1 * w], False) for w in range(n)]
+    psi = N.State(n, np.complex64).reset().apply(ops)
+    bras = [N.State(n, np.complex64).set_pauli_word_of(psi, "Z", [j % n]) for j in range(nobs)]
+    N.adjoint_jacobian(psi, bras[:1], ops, [0])  # buffers that do not grow with the sweeps
+    free, total = N.C.c_uint64(), N.C.c_uint64()
+    N.check(N.lib().lgh_pool_trim(0))
+    N.check(N.lib().lgh_device_memory(0, N.C.byref(free), N.C.byref(total)))
+    before = free.value
+    N.adjoint_jacobian(psi, bras[1:], ops, list(range(n)))
+    N.check(N.lib().lgh_device_memory(0, N.C.byref(free), N.C.byref(total)))
+    assert before - free.value <= (9 << 28) + (64 << 20)
