@@ -46,6 +46,9 @@ _NO_MATRIX = np.zeros(0, dtype=np.complex128)
 # gates handed to the backend at once: bounds the time its scheduler takes for
 # a circuit that it has not seen (milliseconds per thousand gates)
 _SEQUENCE_MAX = 2048
+# bytes of explicit matrices among them: the sequence holds each until it has
+# been applied, a matrix on 10 wires takes 16 MiB
+_SEQUENCE_MATRIX_BYTES = 16 << 20
 _SHOTS_WARNING = ("Requested adjoint differentiation to be computed with finite shots. The derivative is always "
                   "exact when using the adjoint differentiation method.")
 
@@ -171,7 +174,7 @@ class LightningGPU:
         """lightning_gpu.py:519-555.  A backend state that takes a sequence of
         gates gets them together and applies them in fused passes."""
         sequence = getattr(self._gpu_state, "applySequence", None)
-        pending = []
+        pending, held = [], 0
         for o in operations:
             if o.name == "Identity":
                 continue
@@ -190,9 +193,10 @@ class LightningGPU:
                 params = [float(p) for p in np.ravel(o.parameters)]
             if sequence is not None:
                 pending.append((name, wires, invert, params, mat))
-                if len(pending) == _SEQUENCE_MAX:
+                held += mat.nbytes
+                if len(pending) == _SEQUENCE_MAX or held >= _SEQUENCE_MATRIX_BYTES:
                     sequence(*zip(*pending))
-                    pending = []
+                    pending, held = [], 0
             elif method is None:
                 self._gpu_state.apply(name, wires, False, [], mat)
             else:
