@@ -252,10 +252,12 @@ template <class R> struct PairGen {
     cx<double> g[2][4];
 };
 template <class R, int NP>
-__global__ __launch_bounds__(kBlock) void k_adj_pairs(const AdjArrays *__restrict__ table, PairArgs<R> p, PairGen<R> gen,
-                                                      int with_gen, double *__restrict__ partials, uint64_t stride) {
-    const AdjArrays &ar = table[blockIdx.y];
-    cx<R> *psi = static_cast<cx<R> *>(ar.lam), *bra = static_cast<cx<R> *>(ar.bra);
+__global__ __launch_bounds__(kBlock) void k_adj_pairs(void *lam_one, void *bra_one,
+                                                      const AdjArrays *__restrict__ table, PairArgs<R> p,
+                                                      PairGen<R> gen, int with_gen, double *__restrict__ partials,
+                                                      uint64_t stride) {
+    cx<R> *psi = static_cast<cx<R> *>(table ? table[blockIdx.y].lam : lam_one);
+    cx<R> *bra = static_cast<cx<R> *>(table ? table[blockIdx.y].bra : bra_one);
     double acc[1] = {0.0};
     const uint64_t g = xcd_block() * kBlock + threadIdx.x;
     if (g < p.ngroups) {
@@ -282,8 +284,8 @@ __global__ __launch_bounds__(kBlock) void k_adj_pairs(const AdjArrays *__restric
 }
 
 template <class R>
-void adj_pairs_t(StreamCtx *ctx, int n, const KOp &udag, const KGen *gen, const AdjArrays *table, int count,
-                 double *partials, uint64_t stride) {
+void adj_pairs_t(StreamCtx *ctx, int n, const KOp &udag, const KGen *gen, const AdjArrays &one, const AdjArrays *table,
+                 int count, double *partials, uint64_t stride) {
     const PairArgs<R> p = pair_args<R>(udag, n);
     PairGen<R> pg{};
     const size_t D = size_t(1) << udag.k;
@@ -296,7 +298,7 @@ void adj_pairs_t(StreamCtx *ctx, int n, const KOp &udag, const KGen *gen, const 
     }
     auto kern = udag.npair == 1 ? k_adj_pairs<R, 1> : k_adj_pairs<R, 2>;
     hipLaunchKernelGGL(kern, dim3(unsigned((p.ngroups + kBlock - 1) / kBlock), unsigned(count)), dim3(kBlock), 0,
-                       ctx->stream, table, p, pg, int(gen != nullptr), partials, stride);
+                       ctx->stream, one.lam, one.bra, table, p, pg, int(gen != nullptr), partials, stride);
     LGH_LAUNCH_CHECK();
 }
 
@@ -572,7 +574,14 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
     void *table = ws + b_jac + b_ptr + b_part + b_slices + b_fused;
     std::vector<void *> hp(size_t(nbatches * kBras), nullptr);
     for (int j = 0; j < nobs; ++j) hp[size_t(j)] = bras[j]->data;
-    ctx->copy_in(bras_dev, hp.data(), sizeof(void *) * hp.size());
+    // The pointer table is copied before the first step that reads it.  Most
+    // fused sweeps have none, and a copy as the stream's first command after a
+    // wait cost a lone 12-qubit sweep 17 us.
+    bool bras_there = false;
+    auto need_bras = [&] {
+        if (!bras_there) ctx->copy_in(bras_dev, hp.data(), sizeof(void *) * hp.size());
+        bras_there = true;
+    };
     LGH_HIP(hipMemsetAsync(jac_dev, 0, sizeof(double) * size_t(std::max<int64_t>(1, nobs * ntp)), ctx->stream));
 
     if (fused_path) {
@@ -603,7 +612,7 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
             }
             slot.push_back(col);
         }
-        const AdjPasses passes(psi_in, udag, gens, slot, fac);
+        AdjPasses passes(psi_in, udag, gens, slot, fac, nobs > group);
         std::vector<lgh_sv> lams(size_t(group), *psi_in);
         for (int j = 0; j < group; ++j) lams[size_t(j)].data = own ? lam.data : buffers.ptrs[held + size_t(j)];
         auto standalone = [&](const AdjSweep &sw, const KOp &u, const KGen *g, int64_t col, double f) {
@@ -614,6 +623,7 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
                 return;
             }
             const ptrdiff_t j = (sw.jac_row - jac_dev) / ntp;
+            need_bras();
             fused_step<R>(sw.lam, bras_dev + j, 1, u, g, partials);
             if (g) {
                 const unsigned blocks = step_shape(n, u).blocks;
@@ -647,6 +657,8 @@ void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op
         return;
     }
 
+    need_bras();
+    ctx->sync(); // the first kernels start sooner behind a copy that has been waited for (see above)
     int64_t num_param_ops = 0;
     for (int64_t i = 0; i < nops; ++i)
         if (!is_prep(ops[i]) && ops[i].num_params > 0) ++num_param_ops;
@@ -700,12 +712,12 @@ unsigned adj_pairs_blocks(int n, const KOp &udag) {
     return unsigned((groups + kBlock - 1) / kBlock);
 }
 
-void launch_adj_pairs(StreamCtx *ctx, lgh_dtype dtype, int n, const KOp &udag, const KGen *gen,
+void launch_adj_pairs(StreamCtx *ctx, lgh_dtype dtype, int n, const KOp &udag, const KGen *gen, const AdjArrays &one,
                       const AdjArrays *table, int count, double *partials, uint64_t stride) {
     if (dtype == LGH_C128)
-        adj_pairs_t<double>(ctx, n, udag, gen, table, count, partials, stride);
+        adj_pairs_t<double>(ctx, n, udag, gen, one, table, count, partials, stride);
     else
-        adj_pairs_t<float>(ctx, n, udag, gen, table, count, partials, stride);
+        adj_pairs_t<float>(ctx, n, udag, gen, one, table, count, partials, stride);
 }
 
 } // namespace lgh

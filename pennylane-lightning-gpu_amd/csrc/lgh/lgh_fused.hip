@@ -469,8 +469,13 @@ __global__ __launch_bounds__(kBlock) void k_fused_pass(cx<R> *__restrict__ sv, u
     }
 }
 
-// (blockIdx.y: the sweep)
+// The launch's arrays for sweep blockIdx.y.
 typedef __attribute__((address_space(4))) const AdjArrays CAdjArrays;
+__device__ __forceinline__ AdjArrays sweep_arrays(const AdjArrays &one, const AdjArrays *table) {
+    if (!table) return one;
+    const CAdjArrays *t = (const CAdjArrays *)table + blockIdx.y;
+    return AdjArrays{t->lam_src, t->lam, t->bra, t->zmask, t->jac_row};
+}
 
 // Reverse pass of the adjoint sweep on lambda and one observable state; the
 // sweeps of blockIdx.y run side by side (observables of a state too small to
@@ -486,18 +491,18 @@ typedef __attribute__((address_space(4))) const AdjArrays CAdjArrays;
 // per amplitude), then written like any pass's output: the first reverse pass
 // of a sweep with a Z-word observable needs no separate pass that forms it.
 template <class R, int RB, int Lv>
-__device__ __forceinline__ void fused_adj_body(const AdjArrays *__restrict__ arrays, uint64_t ntiles, uint64_t chunk,
-                                               const PassDesc *__restrict__ pd, const FOp *__restrict__ ops,
+__device__ __forceinline__ void fused_adj_body(const AdjArrays &one, const AdjArrays *__restrict__ table,
+                                               uint64_t ntiles, uint64_t chunk, const PassDesc *__restrict__ pd, const FOp *__restrict__ ops,
                                                const FGen *__restrict__ gens, double *__restrict__ partials_all,
                                                uint64_t partials_stride, int from_src, int bra_from_lam) {
     static_assert(kAccCols * kAccLanes == kBlock, "one accumulator column per lane quad");
     __shared__ double acc[adj_slot_cap(RB)][kAccCols];
     __shared__ double sink[kBlock];
     const AccCols cols{acc, sink};
-    const CAdjArrays *ar = (const CAdjArrays *)arrays + blockIdx.y;
-    cx<R> *lam = static_cast<cx<R> *>(ar->lam), *__restrict__ bra = static_cast<cx<R> *>(ar->bra);
-    const cx<R> *lam_in = from_src ? static_cast<const cx<R> *>(ar->lam_src) : lam;
-    const uint64_t bra_zmask = ar->zmask;
+    const AdjArrays ar = sweep_arrays(one, table);
+    cx<R> *lam = static_cast<cx<R> *>(ar.lam), *__restrict__ bra = static_cast<cx<R> *>(ar.bra);
+    const cx<R> *lam_in = from_src ? static_cast<const cx<R> *>(ar.lam_src) : lam;
+    const uint64_t bra_zmask = ar.zmask;
     double *__restrict__ partials = partials_all + blockIdx.y * partials_stride;
     const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const CFOp *cops = (const CFOp *)ops;
@@ -625,20 +630,22 @@ __device__ __forceinline__ void fused_adj_body(const AdjArrays *__restrict__ arr
 // Lv: lean level of the pass (0: any fusable gate).
 template <class R, int Lv = 0>
 __global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 5 : 3) void k_fused_adj3(
-    const AdjArrays *__restrict__ arrays, uint64_t ntiles, uint64_t chunk, const PassDesc *__restrict__ pd,
-    const FOp *__restrict__ ops, const FGen *__restrict__ gens, double *__restrict__ partials, uint64_t partials_stride,
-    int from_src, int bra_from_lam) {
-    fused_adj_body<R, 3, Lv>(arrays, ntiles, chunk, pd, ops, gens, partials, partials_stride, from_src, bra_from_lam);
+    AdjArrays one, const AdjArrays *__restrict__ table, uint64_t ntiles, uint64_t chunk,
+    const PassDesc *__restrict__ pd, const FOp *__restrict__ ops, const FGen *__restrict__ gens,
+    double *__restrict__ partials, uint64_t partials_stride, int from_src, int bra_from_lam) {
+    fused_adj_body<R, 3, Lv>(one, table, ntiles, chunk, pd, ops, gens, partials, partials_stride, from_src,
+                             bra_from_lam);
 }
 // Four register bits: the complex128 lean kernels are held to 168 VGPRs for
 // three wavefronts per SIMD (39 dwords spilled to scratch at level 1; 4.50
 // against 4.88 ms per 28-qubit pass at two wavefronts).
 template <class R, int Lv = 0>
 __global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 3 : 1) void k_fused_adj4(
-    const AdjArrays *__restrict__ arrays, uint64_t ntiles, uint64_t chunk, const PassDesc *__restrict__ pd,
-    const FOp *__restrict__ ops, const FGen *__restrict__ gens, double *__restrict__ partials, uint64_t partials_stride,
-    int from_src, int bra_from_lam) {
-    fused_adj_body<R, 4, Lv>(arrays, ntiles, chunk, pd, ops, gens, partials, partials_stride, from_src, bra_from_lam);
+    AdjArrays one, const AdjArrays *__restrict__ table, uint64_t ntiles, uint64_t chunk,
+    const PassDesc *__restrict__ pd, const FOp *__restrict__ ops, const FGen *__restrict__ gens,
+    double *__restrict__ partials, uint64_t partials_stride, int from_src, int bra_from_lam) {
+    fused_adj_body<R, 4, Lv>(one, table, ntiles, chunk, pd, ops, gens, partials, partials_stride, from_src,
+                             bra_from_lam);
 }
 
 // Slots summed by one store: those of up to eight passes.  3 KiB of partial
@@ -650,13 +657,13 @@ constexpr int kStoreSlots = 4 * kMaxSlotsSv4;
 __global__ __launch_bounds__(kBlock) void k_slot_store(const double *__restrict__ partials_all,
                                                        uint64_t partials_stride, int nparts, int nslots,
                                                        const int64_t *__restrict__ cols,
-                                                       const double *__restrict__ factors,
-                                                       const AdjArrays *__restrict__ arrays) {
+                                                       const double *__restrict__ factors, AdjArrays one,
+                                                       const AdjArrays *__restrict__ table) {
     __shared__ double sh[kWavesPerBlock];
     const int s = blockIdx.x;
     if (s >= nslots) return;
     const double *__restrict__ partials = partials_all + blockIdx.y * partials_stride;
-    double *__restrict__ jac = arrays[blockIdx.y].jac_row;
+    double *__restrict__ jac = sweep_arrays(one, table).jac_row;
     const int64_t col = cols[s];
     const double fac = factors[s];
     double v = 0.0;
@@ -1225,109 +1232,47 @@ FusionPlan plan_passes(const lgh_op *ops, int64_t num_ops, int n, bool adjoint, 
 
 // The passes are scheduled on the forward order and executed backwards.
 AdjPasses::AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std::vector<KGen> &gens,
-                     const std::vector<int> &slot_col, const std::vector<double> &factor)
+                     const std::vector<int> &slot_col, const std::vector<double> &factor, bool again)
     : udag_(udag), gens_(gens), slot_col_(slot_col), factor_(factor), ctx_(like->ctx), n_(like->n),
-      device_(like->device), dtype_(like->dtype) {
+      device_(like->device), dtype_(like->dtype), again_(again) {
     const FusedCfg cfg = fused_cfg(device_, n_, dtype_, 1);
     rb_ = cfg.rb;
     waves_per_cu_ = cfg.waves_per_cu;
     // the kernel's LDS holds adj_slot_cap(rb) slots
-    const auto passes = schedule_passes_cached(udag, n_, slot_col, rb_, fixed_lanes(dtype_),
-                                               std::min(cfg.slots, adj_slot_cap(rb_)));
-    std::vector<unsigned char> blob;
-    auto put = [&](const void *src, size_t bytes) {
-        const size_t at = blob.size();
-        blob.resize(at + ((bytes + 255) & ~size_t(255)));
-        if (bytes) std::memcpy(blob.data() + at, src, bytes);
-        return at;
-    };
-    // The overlaps of consecutive fused passes are summed and stored together,
-    // as many slots as the partials hold: one store per sweep instead of one
-    // behind every pass, which cost the pass's stream 10 us on 24 qubits.
-    std::vector<int64_t> cols;
-    std::vector<double> facs;
-    auto close = [&](Step &st) { // the store runs after st
-        st.nslots = int(cols.size());
-        st.o_cols = put(cols.data(), cols.size() * 8);
-        st.o_facs = put(facs.data(), facs.size() * 8);
-        cols.clear();
-        facs.clear();
-    };
-    int last_fused = -1; // the step whose store the pending slots wait for
-    for (auto it = passes->rbegin(); it != passes->rend(); ++it) {
-        Step st;
-        if (it->standalone) {
-            const int i = it->ops[0];
-            if (udag[size_t(i)].npair == 0) {
-                st.op = i;
-            } else {
-                // a run's partial sums, a row of one double per workgroup for
-                // every trainable gate, fit the partials; the fused passes
-                // before it have been stored
-                if (!cols.empty()) close(steps_[size_t(last_fused)]);
-                size_t room = fused_partials_bytes(n_, device_) / sizeof(double);
-                for (auto next = it; next != passes->rend() && next->standalone; ++next) {
-                    const size_t g = size_t(next->ops[0]);
-                    if (udag[g].npair == 0) break;
-                    if (slot_col[g] >= 0) {
-                        const unsigned blocks = adj_pairs_blocks(n_, udag[g]);
-                        if (blocks > room || (st.blocks && blocks != st.blocks)) break;
-                        st.blocks = blocks;
-                        room -= blocks;
-                    }
-                    st.pairs.push_back(int(g));
-                    it = next;
-                }
-                if (st.pairs.empty()) st.op = i;
-            }
-            if (!st.pairs.empty()) {
-                for (int g : st.pairs)
-                    if (slot_col[size_t(g)] >= 0) {
-                        cols.push_back(slot_col[size_t(g)]);
-                        facs.push_back(factor[size_t(g)]);
-                    }
-                close(st);
-            }
-            steps_.push_back(st);
-            continue;
-        }
-        const Built b = build_pass(*it, udag, n_, true, &gens, &slot_col, rb_, true, true, dtype_ == LGH_C64);
-        LGH_REQUIRE(b.pd.nslots <= adj_slot_cap(rb_), "fused adjoint pass: more trainable gates than LDS slots");
-        if (cols.size() + b.slot_ops.size() > size_t(kStoreSlots)) close(steps_[size_t(last_fused)]);
-        st.row = int(cols.size());
-        for (size_t s = 0; s < b.slot_ops.size(); ++s) {
-            const int oi = b.slot_ops[s];
-            cols.push_back(slot_col[size_t(oi)]);
-            facs.push_back(factor[size_t(oi)] * b.slot_scale[s]);
-        }
-        st.o_desc = put(&b.pd, sizeof(PassDesc));
-        st.o_ops = put(b.ops.data(), b.ops.size() * sizeof(FOp));
-        st.o_gens = put(b.gens.data(), b.gens.size() * sizeof(FGen));
-        st.level = g_lean.load() ? lean_level(b.ops, true) : 0;
-        last_fused = int(steps_.size());
-        steps_.push_back(st);
-    }
-    if (!cols.empty()) close(steps_[size_t(last_fused)]);
-    if (blob.empty()) return;
-    bytes_ = blob.size();
-    dev_ = static_cast<unsigned char *>(pool_alloc(device_, bytes_));
-    try {
-        ctx_->copy_in(dev_, blob.data(), bytes_);
-    } catch (...) {
-        pool_free(device_, dev_, bytes_);
-        throw;
-    }
+    passes_ = schedule_passes_cached(udag, n_, slot_col, rb_, fixed_lanes(dtype_),
+                                     std::min(cfg.slots, adj_slot_cap(rb_)));
 }
 
 AdjPasses::~AdjPasses() {
-    if (!dev_) return;
+    if (kept_.empty()) return;
     (void)hipStreamSynchronize(ctx_->stream);
-    pool_free(device_, dev_, bytes_);
+    for (const auto &k : kept_) pool_free(device_, k.first, k.second);
+}
+
+struct AdjPasses::Blob {
+    std::vector<unsigned char> bytes;
+    size_t put(const void *src, size_t count) {
+        const size_t at = bytes.size();
+        bytes.resize(at + ((count + 255) & ~size_t(255)));
+        if (count) std::memcpy(bytes.data() + at, src, count);
+        return at;
+    }
+};
+
+// Through the upload ring where no run follows: a step's descriptors are read
+// by the launches right after their copy, before anything else is uploaded.
+const unsigned char *AdjPasses::to_device(const Blob &blob) {
+    if (!again_) return static_cast<const unsigned char *>(ctx_->upload(blob.bytes.data(), blob.bytes.size()));
+    kept_.reserve(kept_.size() + 1);
+    void *d = pool_alloc(device_, blob.bytes.size());
+    kept_.emplace_back(d, blob.bytes.size());
+    ctx_->copy_in(d, blob.bytes.data(), blob.bytes.size());
+    return static_cast<const unsigned char *>(d);
 }
 
 template <class R>
 void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void *table,
-                      const StandaloneStep &standalone) const {
+                      const StandaloneStep &standalone) {
     static_assert(sizeof(AdjArrays) <= kTableBytes, "a table entry per sweep");
     const Geometry geo = geometry(n_, device_, rb_, waves_per_cu_, g_waves_adj.load());
     const uint64_t stride = fused_partials_bytes(n_, device_) / sizeof(double);
@@ -1340,16 +1285,11 @@ void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void 
         LGH_REQUIRE(j == 0 || s.bra_from_z == from_z, "adjoint sweeps side by side must be of one kind");
         from_z = s.bra_from_z;
     }
-    ctx_->copy_in(table, tab.data(), tab.size() * sizeof(AdjArrays));
-    const AdjArrays *dtab = static_cast<const AdjArrays *>(table);
-    auto store = [&](const Step &st, unsigned blocks) {
-        if (st.nslots == 0) return;
-        hipLaunchKernelGGL(k_slot_store, dim3(unsigned(st.nslots), unsigned(count)), dim3(kBlock), 0, ctx_->stream,
-                           partials, stride, int(blocks), st.nslots,
-                           reinterpret_cast<const int64_t *>(dev_ + st.o_cols),
-                           reinterpret_cast<const double *>(dev_ + st.o_facs), dtab);
-        LGH_LAUNCH_CHECK();
-    };
+    const AdjArrays one = tab[0], *dtab = nullptr;
+    if (count > 1) {
+        ctx_->copy_in(table, tab.data(), tab.size() * sizeof(AdjArrays));
+        dtab = static_cast<const AdjArrays *>(table);
+    }
     // the sweeps' own lambda and observable states, where a pass would read them elsewhere or form them
     auto settle = [&] {
         for (int j = 0; j < count; ++j) {
@@ -1360,49 +1300,143 @@ void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void 
         }
         from_z = src = false;
     };
-    for (const Step &st : steps_) {
+    auto launch = [&](const Step &st) {
         if (!st.pairs.empty()) {
             settle();
             uint64_t row = 0;
             for (int i : st.pairs) {
                 const bool train = slot_col_[size_t(i)] >= 0;
-                launch_adj_pairs(ctx_, dtype_, n_, udag_[size_t(i)], train ? &gens_[size_t(i)] : nullptr, dtab, count,
-                                 partials + row, stride);
+                launch_adj_pairs(ctx_, dtype_, n_, udag_[size_t(i)], train ? &gens_[size_t(i)] : nullptr, one, dtab,
+                                 count, partials + row, stride);
                 if (train) row += st.blocks;
             }
-            store(st, st.blocks);
-            continue;
+            return;
         }
         if (st.op >= 0) {
             settle();
             const size_t i = size_t(st.op);
             for (int j = 0; j < count; ++j)
                 standalone(sweeps[j], udag_[i], slot_col_[i] >= 0 ? &gens_[i] : nullptr, slot_col_[i], factor_[i]);
+            return;
+        }
+        ProfScope prof(kProfFusedAdj, ctx_->stream);
+        auto kern = rb_ == 4 ? (st.level == 1   ? k_fused_adj4<R, 1>
+                                : st.level == 2 ? k_fused_adj4<R, 2>
+                                                : k_fused_adj4<R>)
+                             : (st.level == 1   ? k_fused_adj3<R, 1>
+                                : st.level == 2 ? k_fused_adj3<R, 2>
+                                                : k_fused_adj3<R>);
+        hipLaunchKernelGGL(kern, dim3(geo.blocks, unsigned(count)), dim3(kBlock), 0, ctx_->stream, one, dtab,
+                           geo.ntiles, geo.chunk, reinterpret_cast<const PassDesc *>(st.dev),
+                           reinterpret_cast<const FOp *>(st.dev + st.o_ops),
+                           reinterpret_cast<const FGen *>(st.dev + st.o_gens),
+                           partials + uint64_t(st.row) * geo.blocks, stride, int(src), int(from_z));
+        from_z = src = false;
+        LGH_LAUNCH_CHECK();
+    };
+    auto store = [&](const Step &st) {
+        if (!st.store || st.pending == 0) return;
+        hipLaunchKernelGGL(k_slot_store, dim3(unsigned(st.pending), unsigned(count)), dim3(kBlock), 0, ctx_->stream,
+                           partials, stride, int(st.pairs.empty() ? geo.blocks : st.blocks), st.pending,
+                           reinterpret_cast<const int64_t *>(st.dev + st.o_cols),
+                           reinterpret_cast<const double *>(st.dev + st.o_facs), one, dtab);
+        LGH_LAUNCH_CHECK();
+    };
+    if (built_) {
+        for (const Step &st : steps_) {
+            launch(st);
+            store(st);
+        }
+        return;
+    }
+
+    // The overlaps of consecutive fused passes are summed and stored together,
+    // as many slots as the partials hold: one store per sweep instead of one
+    // behind every pass, which cost the pass's stream 10 us on 24 qubits.  The
+    // columns and factors of the slots still to be stored travel with every
+    // pass, so that the store behind it needs no copy of its own.
+    std::vector<int64_t> cols;
+    std::vector<double> facs;
+    int last = -1; // the fused pass whose store the pending slots wait for
+    auto close = [&] {
+        if (cols.empty()) return;
+        Step &st = steps_[size_t(last)];
+        st.store = true;
+        store(st);
+        cols.clear();
+        facs.clear();
+    };
+    auto put_slots = [&](Step &st, Blob &blob) {
+        st.pending = int(cols.size());
+        st.o_cols = blob.put(cols.data(), cols.size() * 8);
+        st.o_facs = blob.put(facs.data(), facs.size() * 8);
+    };
+    for (auto it = passes_->rbegin(); it != passes_->rend(); ++it) {
+        Step st;
+        if (it->standalone) {
+            close(); // before what the gate uploads
+            const int i = it->ops[0];
+            if (udag_[size_t(i)].npair > 0) {
+                // a run's partial sums, a row of one double per workgroup for
+                // every trainable gate, fit the partials
+                size_t room = stride;
+                for (auto next = it; next != passes_->rend() && next->standalone; ++next) {
+                    const size_t g = size_t(next->ops[0]);
+                    if (udag_[g].npair == 0) break;
+                    if (slot_col_[g] >= 0) {
+                        const unsigned blocks = adj_pairs_blocks(n_, udag_[g]);
+                        if (blocks > room || (st.blocks && blocks != st.blocks)) break;
+                        st.blocks = blocks;
+                        room -= blocks;
+                        cols.push_back(slot_col_[g]);
+                        facs.push_back(factor_[g]);
+                    }
+                    st.pairs.push_back(int(g));
+                    it = next;
+                }
+            }
+            if (st.pairs.empty()) {
+                st.op = i;
+            } else if (!cols.empty()) {
+                Blob blob;
+                put_slots(st, blob);
+                st.store = true;
+                st.dev = to_device(blob);
+                cols.clear();
+                facs.clear();
+            }
+            steps_.push_back(std::move(st));
+            launch(steps_.back());
+            store(steps_.back());
             continue;
         }
-        {
-            ProfScope prof(kProfFusedAdj, ctx_->stream);
-            auto kern = rb_ == 4 ? (st.level == 1   ? k_fused_adj4<R, 1>
-                                    : st.level == 2 ? k_fused_adj4<R, 2>
-                                                    : k_fused_adj4<R>)
-                                 : (st.level == 1   ? k_fused_adj3<R, 1>
-                                    : st.level == 2 ? k_fused_adj3<R, 2>
-                                                    : k_fused_adj3<R>);
-            hipLaunchKernelGGL(kern, dim3(geo.blocks, unsigned(count)), dim3(kBlock), 0, ctx_->stream, dtab, geo.ntiles,
-                               geo.chunk, reinterpret_cast<const PassDesc *>(dev_ + st.o_desc),
-                               reinterpret_cast<const FOp *>(dev_ + st.o_ops),
-                               reinterpret_cast<const FGen *>(dev_ + st.o_gens),
-                               partials + uint64_t(st.row) * geo.blocks, stride, int(src),
-                               int(from_z));
-            from_z = src = false;
-            LGH_LAUNCH_CHECK();
+        const Built b = build_pass(*it, udag_, n_, true, &gens_, &slot_col_, rb_, true, true, dtype_ == LGH_C64);
+        LGH_REQUIRE(b.pd.nslots <= adj_slot_cap(rb_), "fused adjoint pass: more trainable gates than LDS slots");
+        if (cols.size() + b.slot_ops.size() > size_t(kStoreSlots)) close();
+        st.row = int(cols.size());
+        for (size_t s = 0; s < b.slot_ops.size(); ++s) {
+            const int oi = b.slot_ops[s];
+            cols.push_back(slot_col_[size_t(oi)]);
+            facs.push_back(factor_[size_t(oi)] * b.slot_scale[s]);
         }
-        store(st, geo.blocks);
+        Blob blob;
+        blob.put(&b.pd, sizeof(PassDesc));
+        st.o_ops = blob.put(b.ops.data(), b.ops.size() * sizeof(FOp));
+        st.o_gens = blob.put(b.gens.data(), b.gens.size() * sizeof(FGen));
+        put_slots(st, blob);
+        st.level = g_lean.load() ? lean_level(b.ops, true) : 0;
+        st.dev = to_device(blob);
+        last = int(steps_.size());
+        steps_.push_back(std::move(st));
+        launch(steps_.back());
     }
+    close();
+    built_ = true;
 }
 
 void AdjPasses::run(const AdjSweep *sweeps, int count, double *partials, void *table,
-                    const StandaloneStep &standalone) const {
+                    const StandaloneStep &standalone) {
+    LGH_REQUIRE(!built_ || again_, "adjoint passes built for one run");
     if (dtype_ == LGH_C128)
         run_t<double>(sweeps, count, partials, table, standalone);
     else

@@ -72,7 +72,10 @@ struct AdjSweep {
     std::function<void()> materialize;
 };
 
-// One sweep's arrays (device table, one entry per sweep of a launch).
+// One sweep's arrays.  A launch of several sweeps reads them from a device
+// table, one entry per sweep; a launch of one has them as kernel arguments (a
+// table pointer of null), which saves a copy per call and a chain of two reads
+// from memory at the start of every kernel.
 struct AdjArrays {
     const void *lam_src; // lambda's starting values
     void *lam, *bra;
@@ -85,7 +88,7 @@ struct AdjArrays {
 // generator, workgroup b of sweep y leaves its share of Im<bra|G lambda> in
 // partials[y * stride + b].
 unsigned adj_pairs_blocks(int n, const KOp &udag);
-void launch_adj_pairs(StreamCtx *ctx, lgh_dtype dtype, int n, const KOp &udag, const KGen *gen,
+void launch_adj_pairs(StreamCtx *ctx, lgh_dtype dtype, int n, const KOp &udag, const KGen *gen, const AdjArrays &one,
                       const AdjArrays *table, int count, double *partials, uint64_t stride);
 
 // Applies U^dagger of one non-fusable gate to a sweep's lambda and observable
@@ -93,21 +96,23 @@ void launch_adj_pairs(StreamCtx *ctx, lgh_dtype dtype, int n, const KOp &udag, c
 using StandaloneStep =
     std::function<void(const AdjSweep &sweep, const KOp &udag, const KGen *gen, int64_t col, double factor)>;
 
-// The fused reverse passes of a circuit: scheduled, built and uploaded once,
-// run for any number of sweeps.  udag: the ops in forward order compiled as
-// U^dagger; slot_col[i]: Jacobian column of a trainable gate or -1;
-// factor[i] = -2 s (inverse ? -1 : 1).
+// The fused reverse passes of a circuit, scheduled once.  A pass is built and
+// uploaded in the first run, just before its launch, so that the host works on
+// it while the device runs the pass before.  again: more than one run follows;
+// the descriptors are then kept on the device.  udag: the ops in forward order
+// compiled as U^dagger; slot_col[i]: Jacobian column of a trainable gate or
+// -1; factor[i] = -2 s (inverse ? -1 : 1).
 class AdjPasses {
   public:
     AdjPasses(const lgh_sv *like, const std::vector<KOp> &udag, const std::vector<KGen> &gens,
-              const std::vector<int> &slot_col, const std::vector<double> &factor);
+              const std::vector<int> &slot_col, const std::vector<double> &factor, bool again);
     ~AdjPasses();
     AdjPasses(const AdjPasses &) = delete;
     // Runs the sweeps side by side, one launch per pass for all of them.
     // partials: count * fused_partials_bytes() bytes; table: count *
     // kTableBytes bytes, both on the device and the call's own.
     static constexpr size_t kTableBytes = 64;
-    void run(const AdjSweep *sweeps, int count, double *partials, void *table, const StandaloneStep &standalone) const;
+    void run(const AdjSweep *sweeps, int count, double *partials, void *table, const StandaloneStep &standalone);
 
   private:
     // A fused pass, a gate on its own, or a run of gates that mix pairs of
@@ -116,13 +121,17 @@ class AdjPasses {
         std::vector<int> pairs;   // that run's gates, in execution order
         int op = -1;              // a gate on its own, or -1
         unsigned blocks = 0;      // workgroups of each of the run's trainable gates
-        size_t o_ops = 0, o_gens = 0, o_cols = 0, o_facs = 0, o_desc = 0;
+        const unsigned char *dev = nullptr; // descriptors; offsets into them:
+        size_t o_ops = 0, o_gens = 0, o_cols = 0, o_facs = 0;
         int row = 0;              // a fused pass's first row of partials
-        int nslots = 0;           // slots stored after this step, of it and of passes before it
+        int pending = 0;          // slots whose columns and factors are in dev: its own and those of passes before it
+        bool store = false;       // they are stored after this step
         int level = 0;
     };
+    struct Blob; // host copy of a step's descriptors
     template <class R>
-    void run_t(const AdjSweep *sweeps, int count, double *partials, void *table, const StandaloneStep &s) const;
+    void run_t(const AdjSweep *sweeps, int count, double *partials, void *table, const StandaloneStep &s);
+    const unsigned char *to_device(const Blob &blob);
     const std::vector<KOp> &udag_;
     const std::vector<KGen> &gens_;
     const std::vector<int> &slot_col_;
@@ -130,9 +139,10 @@ class AdjPasses {
     StreamCtx *ctx_;
     int n_, device_, rb_, waves_per_cu_;
     lgh_dtype dtype_;
-    std::vector<Step> steps_;     // in execution order
-    unsigned char *dev_ = nullptr; // descriptors of every pass
-    size_t bytes_ = 0;
+    bool again_, built_ = false;
+    std::shared_ptr<const std::vector<Pass>> passes_;
+    std::vector<Step> steps_;                    // in execution order
+    std::vector<std::pair<void *, size_t>> kept_; // descriptors of every step, where runs follow the first
 };
 size_t fused_partials_bytes(int n, int device);
 

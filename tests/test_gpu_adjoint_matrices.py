@@ -11,6 +11,7 @@ pytestmark = pytest.mark.gpu
 N = pytest.importorskip("pennylane_lightning_gpu._native")
 
 from oracle import pyoracle as po  # noqa: E402
+from pennylane_lightning_gpu.workloads import layered_ring  # noqa: E402
 
 
 def circuit(n, seed):
@@ -57,3 +58,22 @@ def test_adjoint_over_wide_matrices(n, dtype, fusion):
     np.testing.assert_allclose(one, ref[:1], atol=tol, rtol=0)
     np.testing.assert_allclose(many, ref, atol=tol, rtol=0)
     np.testing.assert_allclose(z, ref[[2, 2]], atol=tol, rtol=0)
+
+
+@pytest.mark.parametrize("nobs", [1, 3])
+def test_more_trainable_gates_than_one_store(nobs):
+    """450 trainable gates on 10 qubits, more than the partial sums of one store hold, with a gate that runs on its
+    own in between: against the unfused sweep."""
+    n = 10
+    u, _ = np.linalg.qr(np.random.default_rng(1).normal(size=(8, 8)))
+    ops = layered_ring(n, 9, seed=4) + [("QubitUnitary", [0, 4, 9], [], False, u)] + layered_ring(n, 6, seed=5)
+    psi = N.State(n).reset().apply(ops)
+    tp = list(range(sum(1 for o in ops if o[2])))
+    fused = N.adjoint_jacobian_zwords(psi, [[w] for w in range(nobs)], ops, tp)
+    N.set_fusion(False)
+    try:
+        plain = N.adjoint_jacobian_zwords(psi, [[w] for w in range(nobs)], ops, tp)
+    finally:
+        N.set_fusion(True)
+    # 600 gates of some 8 roundings each on two states
+    np.testing.assert_allclose(fused, plain, atol=2 * 8 * 600 * 2.3e-16, rtol=0)

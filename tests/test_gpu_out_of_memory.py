@@ -44,6 +44,13 @@ def test_memory_of_sweeps_side_by_side():
     N.check(N.lib().lgh_pool_trim(0))
     N.check(N.lib().lgh_device_memory(0, N.C.byref(free), N.C.byref(total)))
     before = free.value
-    N.adjoint_jacobian(psi, bras[1:], ops, list(range(n)))
+    jac = N.adjoint_jacobian(psi, bras[1:], ops, list(range(n)))
     N.check(N.lib().lgh_device_memory(0, N.C.byref(free), N.C.byref(total)))
     assert before - free.value <= (9 << 28) + (64 << 20)
+    # observables repeat every 20 rows, within a group of sweeps and from one group to the next
+    np.testing.assert_array_equal(jac[n:], jac[:-n])
+    # row j: d<Z_w> / d theta_w = -sin theta_w for w = (j + 1) % 20, in single precision
+    w = np.arange(1, nobs) % n
+    ref = np.zeros((nobs - 1, n))
+    ref[np.arange(nobs - 1), w] = -np.sin(0.1 * w)
+    np.testing.assert_allclose(jac, ref, atol=20 * 1.2e-7 * 4, rtol=0)
