@@ -262,20 +262,28 @@ __global__ __launch_bounds__(kBlock) void k_adj_pairs(void *lam_one, void *bra_o
     const uint64_t g = xcd_block() * kBlock + threadIdx.x;
     if (g < p.ngroups) {
         const uint64_t base = expand(g, p.fx) | p.cmask;
+        cx<R> a0[NP], a1[NP], b0[NP], b1[NP];
 #pragma unroll
         for (int q = 0; q < NP; ++q) {
             const uint64_t i = base | p.lo[q], j = base | p.hi[q];
-            const cx<R> a0 = ldnt(psi + i), a1 = ldnt(psi + j), b0 = ldnt(bra + i), b1 = ldnt(bra + j);
+            a0[q] = ldnt(psi + i);
+            a1[q] = ldnt(psi + j);
+            b0[q] = ldnt(bra + i);
+            b1[q] = ldnt(bra + j);
+        }
+#pragma unroll
+        for (int q = 0; q < NP; ++q) {
+            const uint64_t i = base | p.lo[q], j = base | p.hi[q];
             const cx<R> *m = p.m[q];
             if (with_gen) {
                 const cx<double> *gm = gen.g[q];
-                acc[0] += im_dot(b0, cfma(gm[1], up(a1), cmul(gm[0], up(a0))));
-                acc[0] += im_dot(b1, cfma(gm[3], up(a1), cmul(gm[2], up(a0))));
+                acc[0] += im_dot(b0[q], cfma(gm[1], up(a1[q]), cmul(gm[0], up(a0[q]))));
+                acc[0] += im_dot(b1[q], cfma(gm[3], up(a1[q]), cmul(gm[2], up(a0[q]))));
             }
-            stnt(bra + i, cfma(m[1], b1, cmul(m[0], b0)));
-            stnt(bra + j, cfma(m[3], b1, cmul(m[2], b0)));
-            stnt(psi + i, cfma(m[1], a1, cmul(m[0], a0)));
-            stnt(psi + j, cfma(m[3], a1, cmul(m[2], a0)));
+            stnt(bra + i, cfma(m[1], b1[q], cmul(m[0], b0[q])));
+            stnt(bra + j, cfma(m[3], b1[q], cmul(m[2], b0[q])));
+            stnt(psi + i, cfma(m[1], a1[q], cmul(m[0], a0[q])));
+            stnt(psi + j, cfma(m[3], a1[q], cmul(m[2], a0[q])));
         }
     }
     if (!with_gen) return;

@@ -404,17 +404,24 @@ __global__ __launch_bounds__(kBlock) void k_denseK(cx<R> *__restrict__ sv, uint6
 // writes those amplitudes (an eighth of the state for a double excitation, half
 // for a single excitation or a swap), in the order of operations of the dense
 // kernel.  Bound by the launch up to about 20 qubits: a double excitation on
-// 18 qubits 3.4 us against 9.9 us as a dense 16 x 16 matrix.
+// 18 qubits 3.4 us against 9.9 us as a dense 16 x 16 matrix.  All loads come
+// before the first store: with a pair at a time two pairs took 1.7 to 2.2 times
+// as long on 24 and 26 qubits.
 template <class R, int NP>
 __global__ __launch_bounds__(kBlock) void k_pairs(cx<R> *__restrict__ sv, PairArgs<R> p) {
     const uint64_t g = xcd_block() * kBlock + threadIdx.x;
     if (g >= p.ngroups) return;
     const uint64_t base = expand(g, p.fx) | p.cmask;
+    cx<R> a[NP], b[NP];
 #pragma unroll
     for (int q = 0; q < NP; ++q) {
-        const cx<R> a = ldnt(sv + (base | p.lo[q])), b = ldnt(sv + (base | p.hi[q]));
-        stnt(sv + (base | p.lo[q]), cfma(p.m[q][1], b, cmul(p.m[q][0], a)));
-        stnt(sv + (base | p.hi[q]), cfma(p.m[q][3], b, cmul(p.m[q][2], a)));
+        a[q] = ldnt(sv + (base | p.lo[q]));
+        b[q] = ldnt(sv + (base | p.hi[q]));
+    }
+#pragma unroll
+    for (int q = 0; q < NP; ++q) {
+        stnt(sv + (base | p.lo[q]), cfma(p.m[q][1], b[q], cmul(p.m[q][0], a[q])));
+        stnt(sv + (base | p.hi[q]), cfma(p.m[q][3], b[q], cmul(p.m[q][2], a[q])));
     }
 }
 
@@ -466,7 +473,7 @@ template <class R> void launch_kop_t(lgh_sv *sv, const KOp &op) {
         LGH_LAUNCH_CHECK();
         return;
     }
-    if (op.npair > 0) {
+    if (pairs_pay(op, n, sv->dtype, false)) {
         const PairArgs<R> p = pair_args<R>(op, n);
         auto kern = op.npair == 1 ? k_pairs<R, 1> : k_pairs<R, 2>;
         hipLaunchKernelGGL(kern, dim3(unsigned((p.ngroups + kBlock - 1) / kBlock)), dim3(kBlock), 0, st, data, p);

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <complex>
 #include <cstdint>
 #include <memory>
@@ -362,6 +363,36 @@ struct KOp {
     int pair_row[2] = {0, 0};
     int pair_flip = 0;
 };
+
+// Whether a gate of pairs runs in the kernels that touch the pairs only, or as
+// the 4 x 4 matrix it is.  Small states are bound by launches and caches and
+// gain in any case; large ones by memory, which moves whole lines: a low
+// target bit leaves the pairs in pieces of lines, and the matrix kernels, which
+// read and write every amplitude in order, move no more.  The times of the
+// pairs over the matrix, measured for target bits 0 to 4 with the other one next
+// to it and at the top, 16 to 27 qubits (25 in the adjoint sweep):
+//  one pair, forward: whole lines 0.51-0.87; pieces in complex64 0.87-0.98 up to
+//   32 MiB, 0.96-1.13 at 64, up to 1.44 at 1 GiB; in complex128 0.73-0.91 with
+//   both bits inside a line, with one inside 0.80-1.00 up to 256 MiB, 1.06 above;
+//  two pairs, forward: 0.63-1.01 in complex128, in complex64 0.86-0.98 up to
+//   128 MiB, runs shorter than 128 bytes 1.00-1.05 above;
+//  one pair, adjoint: 0.59-0.93 in complex128, whole lines 0.60-0.94 and both
+//   bits inside a line 0.71-0.98 in complex64, one inside 0.77-0.98 below 32 MiB,
+//   1.05-1.17 from there;
+//  two pairs, adjoint: runs of 128 bytes 0.68-1.03, shorter ones 0.67-0.98 below
+//   32 MiB, up to 1.56 from there.
+// Four targets (a double excitation: an eighth of the state) always pay.
+inline bool pairs_pay(const KOp &op, int n, lgh_dtype dtype, bool adjoint) {
+    if (op.npair == 0) return false;
+    if (op.k != 2) return true;
+    const bool single = dtype == LGH_C64;
+    const size_t amp = single ? 8 : 16, state = amp << n, MiB = size_t(1) << 20;
+    const size_t low = amp << std::min(op.tbits[0], op.tbits[1]), high = amp << std::max(op.tbits[0], op.tbits[1]);
+    if (op.npair == 2) return low >= 128 || (adjoint ? state < 32 * MiB : !single || state < 256 * MiB);
+    if (low >= 64) return true;
+    if (adjoint) return !single || high < 64 || state < 32 * MiB;
+    return single ? state < 64 * MiB : high < 64 || state < 512 * MiB;
+}
 
 // The pairs of a KOp as kernel arguments: 2x2 matrices on the amplitudes at
 // base | lo[q] and base | hi[q].
