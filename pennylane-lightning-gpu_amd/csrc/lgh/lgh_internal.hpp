@@ -336,6 +336,7 @@ struct lgh_csr {
     void *values = nullptr;  // cx<R>, nnz
     size_t b_ptr = 0, b_idx = 0, b_val = 0;
     double avg_row = 0;
+    int64_t longest_row = 0;
 };
 
 namespace lgh {

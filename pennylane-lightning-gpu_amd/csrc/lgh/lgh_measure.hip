@@ -565,7 +565,23 @@ __global__ __launch_bounds__(kBlock) void k_narrow(int32_t *__restrict__ dst, co
 // Rows of random columns, 2^18 of 30 and 44 entries: 90 and 121 us, with 32
 // lanes per row 92 and 136, in complex128; in complex64 73 and 95, with 32
 // lanes 71 and 89.  Of 18 entries and less the stream is faster in both.
-template <class R> bool csr_streams(double avg) { return avg <= (sizeof(R) == 8 ? 48 : 24); }
+//
+// A long row among short ones is walked by T lanes of its workgroup, or by the
+// 32 of a row: 90 and 140 ns an entry and lane.  The rest of the matrix takes
+// the time of reading it as a stream, and with 32 lanes per row 2 us for every
+// 16384 rows, the grid's, in each of which the same workgroup may get a long
+// one.  One dense row above a diagonal, complex128: 1050 us as a stream, 115 with
+// 32 lanes on 2^14 rows, 20 and 3.7 ms on 2^18; every 256th row of 2000 entries, the
+// others of one: 111 and 40 us on 2^14 rows, 280 and 590 on 2^18.
+inline int csr_parts(double avg) { return avg <= 6 ? 1 : avg <= 12 ? 2 : avg <= 24 ? 4 : 8; }
+template <class R> bool csr_streams(const lgh_csr *csr) {
+    const double avg = csr->avg_row, longest = double(csr->longest_row);
+    if (avg > (sizeof(R) == 8 ? 48 : 24)) return false;
+    if (longest <= 4 * avg + 16) return true;
+    const double stream = 2.2e-4 * double(csr->b_val + csr->b_idx) + 90.0 * longest / csr_parts(avg);
+    const double lanes = (2000.0 + 140.0 * longest / 32) * std::max(1.0, double(csr->rows) / 16384);
+    return stream <= lanes;
+}
 constexpr int kCsrPerCu = 5; // workgroups per CU that the LDS allows
 template <class I, class R, int T>
 __global__ __launch_bounds__(kBlock) void k_csr_stream(const I *__restrict__ indptr, const I *__restrict__ indices,
@@ -1720,10 +1736,17 @@ void pauli_noalloc_t(const lgh_sv *sv, int64_t nwords, const char *paulis, const
 }
 
 // Host offsets or indices that fit 32 bits, narrowed on the device piece by
-// piece (on the host it took 13 ms of a 45 ms upload of 22 million entries).
+// piece (on the host it took 13 ms of a 45 ms upload of 22 million entries);
+// a single piece on the host, where the staging costs more (2^12 rows of 13
+// entries: 105 us to create the matrix, 86 without).
 void upload_narrow(int device, int32_t *dst, const int64_t *src, int64_t count) {
     if (count <= 0) return;
     constexpr int64_t kPiece = int64_t(1) << 22;
+    if (count <= kPiece) {
+        const std::vector<int32_t> v(src, src + count);
+        LGH_HIP(hipMemcpy(dst, v.data(), sizeof(int32_t) * size_t(count), hipMemcpyHostToDevice));
+        return;
+    }
     const size_t bytes = sizeof(int64_t) * size_t(std::min(count, kPiece));
     struct Piece {
         int device;
@@ -1748,28 +1771,25 @@ void csr_launch(const lgh_csr *csr, const cx<R> *x, cx<R> *y, StreamCtx *ctx, do
     const I *ip = static_cast<const I *>(csr->indptr);
     const I *ix = static_cast<const I *>(csr->indices);
     const cx<R> *vv = static_cast<const cx<R> *>(csr->values);
-    const double avg = csr->avg_row;
     auto stream = [&](auto t) {
         hipLaunchKernelGGL((k_csr_stream<I, R, decltype(t)::value>), dim3(blocks), dim3(kBlock), 0, ctx->stream, ip, ix,
                            vv, x, y, csr->rows, partials);
     };
-    if (avg <= 6)
-        stream(std::integral_constant<int, 1>{});
-    else if (avg <= 12)
-        stream(std::integral_constant<int, 2>{});
-    else if (avg <= 24)
-        stream(std::integral_constant<int, 4>{});
-    else if (csr_streams<R>(avg))
-        stream(std::integral_constant<int, 8>{});
-    else
-        hipLaunchKernelGGL((k_csr<I, R, 32>), dim3(blocks), dim3(kBlock), 0, ctx->stream, ip, ix, vv, x, y,
-                           csr->rows, partials);
+    switch (csr_streams<R>(csr) ? csr_parts(csr->avg_row) : 0) {
+    case 1: stream(std::integral_constant<int, 1>{}); break;
+    case 2: stream(std::integral_constant<int, 2>{}); break;
+    case 4: stream(std::integral_constant<int, 4>{}); break;
+    case 8: stream(std::integral_constant<int, 8>{}); break;
+    default:
+        hipLaunchKernelGGL((k_csr<I, R, 32>), dim3(blocks), dim3(kBlock), 0, ctx->stream, ip, ix, vv, x, y, csr->rows,
+                           partials);
+    }
     LGH_LAUNCH_CHECK();
 }
 
 template <class R> void csr_run(const lgh_csr *csr, const lgh_sv *x, lgh_sv *y, double *re, double *im) {
     StreamCtx *ctx = x->ctx;
-    const int per_cu = csr_streams<R>(csr->avg_row) ? kCsrPerCu : 8;
+    const int per_cu = csr_streams<R>(csr) ? kCsrPerCu : 8;
     const unsigned blocks = unsigned(std::max<int64_t>(
         1, std::min<int64_t>((csr->rows * 16 + kBlock - 1) / kBlock, int64_t(sm_count(x->device)) * per_cu)));
     if (y) {
@@ -2127,7 +2147,13 @@ lgh_status lgh_csr_create(lgh_csr **out, int device, lgh_dtype dtype, int64_t nu
         LGH_REQUIRE(out && indptr && (nnz == 0 || (indices && values)), "null pointer");
         LGH_REQUIRE(num_rows >= 1, "CSR matrix needs at least one row");
         LGH_REQUIRE(indptr[0] == 0 && indptr[num_rows] == nnz, "CSR offsets do not match nnz");
-        for (int64_t r = 0; r < num_rows; ++r) LGH_REQUIRE(indptr[r + 1] >= indptr[r], "CSR offsets must not decrease");
+        int64_t shortest = 0, longest = 0;
+        for (int64_t r = 0; r < num_rows; ++r) {
+            const int64_t len = indptr[r + 1] - indptr[r];
+            shortest = std::min(shortest, len);
+            longest = std::max(longest, len);
+        }
+        LGH_REQUIRE(shortest >= 0, "CSR offsets must not decrease");
         for (int64_t k = 0; k < nnz; ++k)
             LGH_REQUIRE(indices[k] >= 0 && indices[k] < num_rows, "CSR column index out of range");
         auto c = std::make_unique<lgh_csr>();
@@ -2136,6 +2162,7 @@ lgh_status lgh_csr_create(lgh_csr **out, int device, lgh_dtype dtype, int64_t nu
         c->rows = num_rows;
         c->nnz = nnz;
         c->avg_row = double(nnz) / double(num_rows);
+        c->longest_row = longest;
         // 32-bit indices where they fit: a sixth of a complex128 matrix's bytes
         c->idx64 = num_rows >= (int64_t(1) << 31) || nnz >= (int64_t(1) << 31);
         DeviceGuard g(device);
