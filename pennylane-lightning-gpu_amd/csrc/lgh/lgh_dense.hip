@@ -214,16 +214,24 @@ DenseArgs dense_args(int n, const int *tbits, int k, const std::vector<int> &cbi
 }
 
 // workgroups of a launch over g.ncols columns
+// Five and six target bits with few columns: the time is one tile's chain of
+// matrix instructions, and tiles of half the size with half the chain (H = 1)
+// run on CUs that would be idle. A 6-wire unitary on 12 qubits, complex128: 40.3
+// us a call with the large tiles, 38.4 here (44.8 with a thread per row of M);
+// 2^18 amplitudes 43.4 and 39.6, 2^19 42.9 and 45.4.
+constexpr uint64_t kDenseNarrow = 1 << 18; // amplitudes
+bool dense_narrow(const DenseArgs &g) { return g.tb.k <= 6 && (g.ncols << g.tb.k) <= kDenseNarrow; }
 unsigned dense_blocks(const DenseArgs &g) {
-    const uint64_t mt = std::min(64, 1 << g.tb.k), nt = g.tb.k <= 5 ? 64 : 32;
+    const uint64_t mt = std::min(64, 1 << g.tb.k);
+    const uint64_t nt = dense_narrow(g) && g.tb.k > 4 ? (g.tb.k == 5 ? 32 : 16) : g.tb.k <= 5 ? 64 : 32;
     return unsigned(((1ull << g.tb.k) / mt) * ((g.ncols + nt - 1) / nt));
 }
 template <class R, int Mode>
 void dense_launch(hipStream_t st, const cx<R> *sv, cx<R> *dst, const cx<double> *mat, double *partials,
                   const DenseArgs &g) {
     auto kern = g.tb.k == 4   ? k_dense_mm<R, 1, 1, 4, Mode>
-                : g.tb.k == 5 ? k_dense_mm<R, 2, 1, 4, Mode>
-                              : k_dense_mm<R, 2, 2, 2, Mode>;
+                : g.tb.k == 5 ? (dense_narrow(g) ? k_dense_mm<R, 1, 2, 2, Mode> : k_dense_mm<R, 2, 1, 4, Mode>)
+                              : (dense_narrow(g) ? k_dense_mm<R, 1, 4, 1, Mode> : k_dense_mm<R, 2, 2, 2, Mode>);
     hipLaunchKernelGGL(kern, dim3(dense_blocks(g)), dim3(kBlock), 0, st, sv, dst, mat, partials, g);
     LGH_LAUNCH_CHECK();
 }

@@ -249,12 +249,12 @@ KOp compile_op(const lgh_op &op, int n, bool dagger) {
     const int dt = 1 << kt;
     Mat t;
     if (op.gate == LGH_GATE_MATRIX) {
-        t.resize(size_t(dt) * dt);
-        for (size_t i = 0; i < t.size(); ++i) t[i] = C(op.matrix[2 * i], op.matrix[2 * i + 1]);
+        const C *m = reinterpret_cast<const C *>(op.matrix); // interleaved, as std::complex is laid out
+        t.assign(m, m + size_t(dt) * dt);
     } else {
         t = target_matrix(op.gate, op.params, kt);
     }
-    k.mat = inv ? dagger_of(t, dt) : t;
+    k.mat = inv ? dagger_of(t, dt) : std::move(t);
     auto pairs = [&](int flip, int row0, int row1 = -1) {
         k.pair_flip = flip;
         k.pair_row[k.npair++] = row0;
