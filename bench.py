@@ -319,6 +319,14 @@ PUBLISHED_A100_S = {(21, 1): 2.7, (21, 2): 4.5, (23, 1): 5.6, (23, 2): 8.0,
                     (25, 1): 16.0, (25, 2): 19.0, (27, 1): 57.0, (27, 2): 72.0}
 
 
+def adjoint_bytes_per_launch(passes, sweeps, launches, state_bytes):
+    """Mean bytes of a launch when `sweeps` reverse sweeps of `passes` fused
+    passes each ran in `launches` launches.  A sweep's first pass forms its
+    observable state: it reads lambda and writes both states, every other pass
+    reads and writes both.  Sweeps side by side share launches, not traffic."""
+    return sweeps * (4 * passes - 1) * state_bytes / max(1, launches)
+
+
 def bench_published(N, ops_mod, args):
     """The reference's published workload shape on this build, through the
     pybind11 API as the device drives it: reset, the StronglyEntanglingLayers
@@ -326,7 +334,7 @@ def bench_published(N, ops_mod, args):
     observables.  One warm-up, median of 3.  The fused adjoint passes of the
     timed runs are timed with HIP events: each observable's sweep forms its
     observable state inside its first pass (3 state bytes) and moves 4 state
-    bytes in every other pass."""
+    bytes in every other pass; a launch holds a pass of several sweeps."""
     import numpy as np
 
     from pennylane_lightning_gpu.workloads import strongly_entangling
@@ -366,7 +374,8 @@ def bench_published(N, ops_mod, args):
             f_n, f_ms = N.profile_read("fused_pass")
             N.profile_enable(False)
             sec = sorted(ts)[1]
-            a_bytes = (4 * a_n - 3 * n) * S / max(1, a_n)  # per launch, averaged over 3 runs
+            passes = N.fusion_plan(n, ops, adjoint=True)["passes"]
+            a_bytes = adjoint_bytes_per_launch(passes, 3 * n, a_n, S)  # 3 runs
             pub = PUBLISHED_A100_S.get((n, layers))
             rows.append({
                 "wires": n, "layers": layers, "params": n_par, "observables": n, "s": round(sec, 4),
