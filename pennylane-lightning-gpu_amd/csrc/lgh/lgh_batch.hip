@@ -412,8 +412,8 @@ __device__ __forceinline__ void rev_pass(const CTPass *tp, const CFOp *fops, con
                         } else {
                             adj_diag_step<R, NR, false>(cur, 0.0, 0.0, base, a, b);
                         }
-                    } else if (Lv == 2 && !f_plain(cur)) { // a controlled X, not trainable
-                        if constexpr (Lv == 2) {
+                    } else if (Lv >= 2 && !f_plain(cur)) { // a controlled X, not trainable
+                        if constexpr (Lv >= 2) {
                             const M2<R> m = m2<R>(cur);
                             cx_lean<R, NR>(cur, m, lane, base, a);
                             cx_lean<R, NR>(cur, m, lane, base, b);
@@ -776,7 +776,9 @@ unsigned batch_grid(int dev, int32_t ncirc, int per_cu) {
 
 typedef void (*BatchKernel)(const CircDev *, int, uint32_t *, int);
 template <class R> BatchKernel batch_kernel(int lean) {
-    return lean == 1 ? k_batch<R, 1> : lean == 2 ? k_batch<R, 2> : k_batch<R, 0>;
+    // level 2 in complex128: RX comes with its cosine taken out (see Scales)
+    constexpr int kLevel2 = sizeof(R) == 8 ? 3 : 2;
+    return lean == 1 ? k_batch<R, 1> : lean == 2 ? k_batch<R, kLevel2> : k_batch<R, 0>;
 }
 
 template <class R>

@@ -417,7 +417,7 @@ using namespace lgh;
 namespace {
 
 // Forward pass: every wavefront processes tiles [w*chunk, (w+1)*chunk).
-// Lv 1, 2: the pass holds only the gate forms of that lean level
+// Lv 1, 2, 3: the pass holds only the gate forms of that lean level
 // (lean_level); 0: any fusable gate.
 template <class R, int RB, int Lv = 0>
 __global__ __launch_bounds__(kBlock) void k_fused_pass(cx<R> *__restrict__ sv, uint64_t ntiles, uint64_t chunk,
@@ -562,14 +562,14 @@ __device__ __forceinline__ void fused_adj_body(const AdjArrays &one, const AdjAr
                     if (Lv == 1 || !f_dsym(cur)) { // the pass's closing scale
                         scale_lean<R, NR>(cur, a);
                         scale_lean<R, NR>(cur, b);
-                    } else if constexpr (Lv == 2) {
+                    } else if constexpr (Lv >= 2) {
                         if (slot >= 0)
                             acc_add(cols, slot, adj_diag_step<R, NR, true>(cur, cur.m[2].re, cur.m[3].re, base, a, b));
                         else
                             adj_diag_step<R, NR, false>(cur, 0.0, 0.0, base, a, b);
                     }
-                } else if (Lv == 2 && !f_plain(cur)) { // a controlled X, not trainable
-                    if constexpr (Lv == 2) {
+                } else if (Lv >= 2 && !f_plain(cur)) { // a controlled X, not trainable
+                    if constexpr (Lv >= 2) {
                         const M2<R> m = m2<R>(cur);
                         cx_lean<R, NR>(cur, m, lane, base, a);
                         cx_lean<R, NR>(cur, m, lane, base, b);
@@ -1162,6 +1162,8 @@ void run_forward(lgh_sv *sv, const std::vector<KOp> &kops, const std::vector<Pas
         const int lv = g_lean.load() ? lean_level(b.ops, false) : 0;
         auto kern = rb == 4 ? (lv == 1 ? k_fused_pass<R, 4, 1> : lv == 2 ? k_fused_pass<R, 4, 2> : k_fused_pass<R, 4>)
                             : (lv == 1 ? k_fused_pass<R, 3, 1> : lv == 2 ? k_fused_pass<R, 3, 2> : k_fused_pass<R, 3>);
+        if constexpr (sizeof(R) == 8)
+            if (lv == 3) kern = rb == 4 ? k_fused_pass<R, 4, 3> : k_fused_pass<R, 3, 3>;
         hipLaunchKernelGGL(kern, dim3(geo.blocks), dim3(kBlock), 0, ctx->stream, static_cast<cx<R> *>(sv->data),
                            geo.ntiles, geo.chunk, reinterpret_cast<const PassDesc *>(d),
                            reinterpret_cast<const FOp *>(d + pb));
@@ -1326,6 +1328,8 @@ void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void 
                              : (st.level == 1   ? k_fused_adj3<R, 1>
                                 : st.level == 2 ? k_fused_adj3<R, 2>
                                                 : k_fused_adj3<R>);
+        if constexpr (sizeof(R) == 8)
+            if (st.level == 3) kern = rb_ == 4 ? k_fused_adj4<R, 3> : k_fused_adj3<R, 3>;
         hipLaunchKernelGGL(kern, dim3(geo.blocks, unsigned(count)), dim3(kBlock), 0, ctx_->stream, one, dtab,
                            geo.ntiles, geo.chunk, reinterpret_cast<const PassDesc *>(st.dev),
                            reinterpret_cast<const FOp *>(st.dev + st.o_ops),

@@ -738,21 +738,21 @@ __device__ __forceinline__ void adj_plain_lean(const FOp &op, int lane, cx<R> (&
     const M2<R> m = m2<R>(op);
     const uint32_t gk = f_gkind(op);
     const int rot = f_rot(op), loc = f_loc(op);
-    // rotation form 3 is F = 4 (level 2, complex128)
-    constexpr int kX = Lv == 2 && sizeof(R) == 8 ? 4 : 0;
+    // rotation form 3 is F = 4 (level 3)
+    constexpr int kX = Lv == 3 ? 4 : 0;
     const int form = kX && rot == 3 ? 4 : rot ? rot : ((Lv == 1 || f_real(op)) ? 0 : 3);
 #define LGH_REG3(B)                                                                                                    \
     (form == 1   ? sink(adj_reg_lean<R, NR, B, Gen, 1>(m, gk, a, b))                                                 \
      : form == 2 ? sink(adj_reg_lean<R, NR, B, Gen, 2>(m, gk, a, b))                                                 \
      : form == 0 ? sink(adj_reg_lean<R, NR, B, Gen, 0>(m, gk, a, b))                                                 \
      : kX && form == kX ? sink(adj_reg_lean<R, NR, B, Gen, kX>(m, gk, a, b))                                         \
-                 : sink(adj_reg_lean<R, NR, B, Gen, Lv == 2 ? 3 : 0>(m, gk, a, b)))
+                 : sink(adj_reg_lean<R, NR, B, Gen, Lv >= 2 ? 3 : 0>(m, gk, a, b)))
 #define LGH_LANE3(L)                                                                                                   \
     (form == 1   ? sink(adj_lane_lean<R, NR, L, Gen, 1>(m, gk, lane, a, b))                                          \
      : form == 2 ? sink(adj_lane_lean<R, NR, L, Gen, 2>(m, gk, lane, a, b))                                          \
      : form == 0 ? sink(adj_lane_lean<R, NR, L, Gen, 0>(m, gk, lane, a, b))                                          \
      : kX && form == kX ? sink(adj_lane_lean<R, NR, L, Gen, kX>(m, gk, lane, a, b))                                  \
-                 : sink(adj_lane_lean<R, NR, L, Gen, Lv == 2 ? 3 : 0>(m, gk, lane, a, b)))
+                 : sink(adj_lane_lean<R, NR, L, Gen, Lv >= 2 ? 3 : 0>(m, gk, lane, a, b)))
     if (f_kind(op) == kRegDense) {
         switch (loc) {
         case 0: LGH_REG3(0); return;
@@ -913,9 +913,12 @@ inline bool pure_scale(const FOp &f) {
 // real 2x2 gates, diagonal runs, a pass's closing real scale), 2 for the
 // further forms of level-2 kernels (uncontrolled complex 2x2 gates,
 // controlled X gates, phases symmetric under conjugation on at most one
-// register bit), 0 for anything else.  Trainable dense gates need an X or Y
+// register bit), 3 for RX with its cosine taken out as well (rotation form 3,
+// complex128), 0 for anything else.  Trainable dense gates need an X or Y
 // generator, trainable phases a diagonal one.  Each level is a kernel of its
-// own: the level-2 cases cost the level-1 passes a little.
+// own: the level-2 cases cost the level-1 passes a little, and the RX form in
+// level 2 doubled the spilled registers of every pass with a CNOT (adjoint, three
+// register bits 17 -> 35, four 40 -> 76).
 inline int lean_level_op(const FOp &f, bool adjoint) {
     const uint32_t kind = f.meta & 15u;
     const bool trainable = adjoint && int((f.meta >> 8) & 255u) > 0;
@@ -937,7 +940,7 @@ inline int lean_level_op(const FOp &f, bool adjoint) {
     }
     const int rot = int((f.meta >> 28) & 3u);
     const bool real = (f.meta >> 21) & 1u;
-    return rot == 1 || rot == 2 || real ? 1 : 2;
+    return rot == 3 ? 3 : rot != 0 || real ? 1 : 2;
 }
 inline bool lean_member(const FOp &m, bool adjoint) {
     const uint32_t mc = (m.meta >> 24) & 3u;
@@ -1036,8 +1039,8 @@ __device__ __forceinline__ void apply_lean(const FOp &op, int lane, uint64_t bas
     const M2<R> m = m2<R>(op);
     const int loc = f_loc(op), rot = f_rot(op);
     const bool real = Lv == 1 || f_real(op);
-    constexpr int kX = Lv == 2 && sizeof(R) == 8 ? 3 : 0; // rotation form 3
-    if constexpr (Lv == 2) {
+    constexpr int kX = Lv == 3 ? 3 : 0; // rotation form 3
+    if constexpr (Lv >= 2) {
         if (!f_plain(op)) {
             cx_lean<R, NR>(op, m, lane, base, v);
             return;
