@@ -272,6 +272,16 @@ struct PTile {
     int bit[kPTileBits];
 };
 
+// Half of a launch's words as kernel arguments, and the kernel that writes them
+// to device memory: for callers that may neither allocate nor wait.
+struct PHalf {
+    uint32_t w[sizeof(PLaunch) / 8];
+};
+static_assert(sizeof(PLaunch) % 8 == 0 && sizeof(PHalf) <= 3072, "two halves, each within the kernel arguments");
+__global__ __launch_bounds__(256) void k_pauli_put(uint32_t *__restrict__ dst, PHalf h) {
+    for (unsigned i = threadIdx.x; i < sizeof(PHalf) / 4; i += 256) dst[i] = h.w[i];
+}
+
 // The products of a flip mask, 32 pairs per lane.
 template <class R, uint32_t Kind>
 __device__ __forceinline__ void pair_products(const char *tile, uint32_t pivot, uint32_t flip, int lane,
@@ -1717,9 +1727,13 @@ void pauli_noalloc_t(const lgh_sv *sv, int64_t nwords, const char *paulis, const
                                                   std::to_string(kNoAllocScratchBytes) + " available");
     PauliBufs bufs{reinterpret_cast<double *>(base), pcap, reinterpret_cast<double *>(base) + pcap,
                    [](StreamCtx *c, const PLaunch &l, void *dst) {
-                       // pageable memory of the calling thread: wait until it has been read
-                       LGH_HIP(hipMemcpyAsync(dst, &l, sizeof(l), hipMemcpyHostToDevice, c->stream));
-                       c->sync();
+                       for (int q = 0; q < 2; ++q) {
+                           PHalf h;
+                           std::memcpy(&h, reinterpret_cast<const char *>(&l) + q * sizeof(h), sizeof(h));
+                           hipLaunchKernelGGL(k_pauli_put, dim3(1), dim3(256), 0, c->stream,
+                                              static_cast<uint32_t *>(dst) + q * (sizeof(h) / 4), h);
+                           LGH_LAUNCH_CHECK();
+                       }
                        return static_cast<const PLaunch *>(dst);
                    },
                    base + o_words};
