@@ -693,6 +693,9 @@ struct HOp {
     int loc = 0, slot = -1;
     uint64_t cm_reg = 0, pm_reg = 0; // control / parity bits among the register bits
     FOp f{};
+    // a product of merged gates before it was rounded to f.m (complex128)
+    bool merged = false;
+    cx<long double> m[4] = {};
 };
 
 FOp pack(const HOp &h, const uint64_t (&reg_off)[kMaxNR], int nr) {
@@ -918,22 +921,51 @@ Built lgh::fz::build_pass(const Pass &p, const std::vector<KOp> &kops, int n, bo
             !keep_apart(h, hops[size_t(last_single[size_t(single_bit)])])) {
             // fold into the earlier gate on the same bit: M <- M_new * M_old
             HOp &prev = hops[size_t(last_single[size_t(single_bit)])];
-            const cx<double> zero{0, 0};
-            cx<double> mn[4], mo[4];
-            if (h.kind == kDiag) {
-                mn[0] = f.m[0]; mn[1] = zero; mn[2] = zero; mn[3] = f.m[1];
+            // Complex128: the product in extended precision, scaled to a
+            // determinant of modulus one where it is unitary, and rounded once.
+            // Its factors are rounded, and so were the products: the norm
+            // drifted by 0.85e-16 per merged gate.
+            auto product = [](const auto (&x)[4], const auto (&y)[4], auto (&z)[4]) {
+                auto mul = [](auto p, auto q) { return decltype(p){p.re * q.re - p.im * q.im, p.re * q.im + p.im * q.re}; };
+                auto add = [](auto p, auto q) { return decltype(p){p.re + q.re, p.im + q.im}; };
+                for (int i = 0; i < 2; ++i)
+                    for (int j = 0; j < 2; ++j)
+                        z[2 * i + j] = add(mul(x[2 * i], y[j]), mul(x[2 * i + 1], y[2 + j]));
+            };
+            auto entries = [](const HOp &x, auto (&z)[4]) {
+                using T = decltype(z[0].re);
+                const cx<double> *m = x.f.m;
+                for (int q = 0; q < 4; ++q) z[q] = {T(m[q].re), T(m[q].im)};
+                if (x.kind == kDiag) {
+                    z[3] = z[1];
+                    z[1] = z[2] = {T(0), T(0)};
+                }
+            };
+            cx<double> r[4];
+            cx<long double> exact[4] = {};
+            if (single) {
+                cx<double> mn[4], mo[4];
+                entries(h, mn);
+                entries(prev, mo);
+                product(mn, mo, r);
             } else {
-                for (int q = 0; q < 4; ++q) mn[q] = f.m[q];
+                cx<long double> mn[4], mo[4];
+                entries(h, mn);
+                entries(prev, mo);
+                if (prev.merged) std::copy(prev.m, prev.m + 4, mo);
+                product(mn, mo, exact);
+                const cx<long double> *e = exact;
+                auto norm = [](cx<long double> x) { return x.re * x.re + x.im * x.im; };
+                const long double row0 = norm(e[0]) + norm(e[1]) - 1, row1 = norm(e[2]) + norm(e[3]) - 1;
+                const long double det =
+                    norm({e[0].re * e[3].re - e[0].im * e[3].im - e[1].re * e[2].re + e[1].im * e[2].im,
+                          e[0].re * e[3].im + e[0].im * e[3].re - e[1].re * e[2].im - e[1].im * e[2].re}) - 1;
+                if (std::abs(row0) < 1e-14L && std::abs(row1) < 1e-14L && std::abs(det) < 2e-14L) {
+                    const long double f = 1 - det / 4; // (1 + det)^-1/4, det being |det|^2 - 1
+                    for (auto &x : exact) x = {f * x.re, f * x.im};
+                }
+                for (int q = 0; q < 4; ++q) r[q] = {double(exact[q].re), double(exact[q].im)};
             }
-            if (prev.kind == kDiag) {
-                mo[0] = prev.f.m[0]; mo[1] = zero; mo[2] = zero; mo[3] = prev.f.m[1];
-            } else {
-                for (int q = 0; q < 4; ++q) mo[q] = prev.f.m[q];
-            }
-            auto mul = [](cx<double> x, cx<double> y) { return cx<double>{x.re * y.re - x.im * y.im, x.re * y.im + x.im * y.re}; };
-            auto add = [](cx<double> x, cx<double> y) { return cx<double>{x.re + y.re, x.im + y.im}; };
-            const cx<double> r[4] = {add(mul(mn[0], mo[0]), mul(mn[1], mo[2])), add(mul(mn[0], mo[1]), mul(mn[1], mo[3])),
-                                     add(mul(mn[2], mo[0]), mul(mn[3], mo[2])), add(mul(mn[2], mo[1]), mul(mn[3], mo[3]))};
             const int bit = single_bit;
             prev = HOp{};
             if (lane_loc(bit) >= 0) {
@@ -944,6 +976,8 @@ Built lgh::fz::build_pass(const Pass &p, const std::vector<KOp> &kops, int n, bo
                 prev.loc = reg_loc(bit);
             }
             for (int q = 0; q < 4; ++q) prev.f.m[q] = r[q];
+            prev.merged = !single;
+            std::copy(exact, exact + 4, prev.m);
             continue;
         }
         for (int bit = 0; bit < 64; ++bit)
@@ -977,7 +1011,23 @@ Built lgh::fz::build_pass(const Pass &p, const std::vector<KOp> &kops, int n, bo
     };
     size_t scale_hop = hops.size() + 1;           // index of a closing scale gate, if any
     size_t fold_i = hops.size() + 1, fold_j = 0;  // the run that applies the scale, if any
-    double scale = 1.0;
+    // The scale of complex128 passes is kept in extended precision and rounded
+    // once, and the factor of a rotation is the one that makes it unitary with the
+    // ratio as it was rounded, 1 / sqrt(1 + ratio^2): the cosine and the
+    // ratio each rounded would let the norm drift by both roundings a gate
+    // (576 random rotations: 1.4e-15 rms; 0.75e-15 with the whole matrices;
+    // 0.14e-15 so).  A matrix that is no rotation keeps its own factor.
+    long double scale_l = 1.0L;
+    auto take_out = [&](double factor, double ratio) {
+        if (single) {
+            scale_l = double(scale_l) * factor;
+            return;
+        }
+        // c (1 + d / 2) with d = 1 - c^2 (1 + ratio^2) is that factor to d^2
+        const long double c = factor, r = ratio, d = 1 - c * c * (1 + r * r);
+        scale_l *= std::abs(d) < 4e-15L ? c + c * d / 2 : c;
+    };
+    double scale = 1.0; // scale_l, rounded
     // smallest running product: 2^-20 for complex64 registers (values up to
     // 2^20 times the amplitudes, far inside float range), 2^-100 for
     // complex128 (the squared ratios of the Jacobian factors stay normal)
@@ -1000,7 +1050,8 @@ Built lgh::fz::build_pass(const Pass &p, const std::vector<KOp> &kops, int n, bo
                 h.f.m[0] = h.f.m[3] = cx<double>{1.0, 0.0};
                 h.f.m[1] = h.f.m[2] = cx<double>{0.0, u};
                 h.rot = 3;
-                scale *= c;
+                take_out(c, u);
+                scale = double(scale_l);
                 continue;
             }
             if (m[0].im != 0.0 || m[1].im != 0.0 || m[2].im != 0.0 || m[3].im != 0.0) continue;
@@ -1019,7 +1070,7 @@ Built lgh::fz::build_pass(const Pass &p, const std::vector<KOp> &kops, int n, bo
                 h.f.m[2] = cx<double>{t, 0.0};
                 h.f.m[3] = cx<double>{1.0, 0.0};
                 h.rot = 1;
-                scale *= c;
+                take_out(c, t);
             } else { // s [[c/s, -1], [1, c/s]]
                 const double t = c / s;
                 h.f.m[0] = cx<double>{t, 0.0};
@@ -1027,8 +1078,9 @@ Built lgh::fz::build_pass(const Pass &p, const std::vector<KOp> &kops, int n, bo
                 h.f.m[2] = cx<double>{1.0, 0.0};
                 h.f.m[3] = cx<double>{t, 0.0};
                 h.rot = 2;
-                scale *= s;
+                take_out(s, t);
             }
+            scale = double(scale_l);
         }
         if (scale != 1.0) {
             // The scale is a global factor, so any point of the pass may
