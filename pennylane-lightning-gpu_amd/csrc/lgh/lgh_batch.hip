@@ -110,7 +110,10 @@ struct CircDev {
 // out at most 2^-100 (past it, its gates stay whole), and every fourth pass
 // multiplies the product of the four before it back in where it loads its
 // tiles, so the values stay within 2^400 of the state's.  A tile of 8 registers
-// spends 48 FMAs per state on RX, RY, RZ instead of 128.
+// spends 48 FMAs per state on RX, RY, RZ instead of 128.  The factor that makes
+// a gate of the rounded ratio unitary differs from the rounded cosine by up to
+// an ulp; the differences are summed beside the product (see unit_residual),
+// as the norm would drift by them gate after gate.
 constexpr int kScaleGroup = 4;
 constexpr double kScaleFloor = 0x1p-100;
 struct Scales { // a circuit's scale array, by pass (forward, then reverse)
@@ -169,6 +172,25 @@ __device__ __forceinline__ void set_gate(FOp &f, int form, double c, double s, d
     if (unit) f.meta |= (form == kRX ? 3u : 1u) << 28;
 }
 
+// A product of factors and what it is off by, relative: the true one is v (1 + off).
+struct Product {
+    double v = 1.0, off = 0.0;
+    __device__ __forceinline__ double rounded() const { return fma(v, off, v); }
+};
+__device__ __forceinline__ Product operator*(const Product &a, const Product &b) {
+    const double v = a.v * b.v, low = fma(a.v, b.v, -v);
+    return Product{v, a.off + b.off + (low != 0.0 ? low / v : 0.0)};
+}
+
+// (f - c) / c for the factor f = 1 / sqrt(1 + u^2) of the rounded ratio u of sine
+// and cosine c: half of 1 - c^2 (1 + u^2), whose terms are formed exactly.
+__device__ __forceinline__ double unit_residual(double c, double u) {
+    const double q = __dmul_rn(c, u), ql = fma(c, u, -q);
+    const double ch = __dmul_rn(c, c), cl = fma(c, c, -ch), sh = __dmul_rn(q, q), sl = fma(q, q, -sh) + 2.0 * q * ql;
+    const double most = ch >= 0.5 ? __dadd_rn(__dadd_rn(ch, -1.0), sh) : __dadd_rn(__dadd_rn(sh, -1.0), ch);
+    return -0.5 * (most + (cl + sl));
+}
+
 __global__ __launch_bounds__(kBlock) void k_batch_prep(const CircDev *__restrict__ circs, uint32_t *counter) {
     if (blockIdx.x == 0 && threadIdx.x == 0) *counter = 0u;
     const CircDev &cd = circs[blockIdx.x];
@@ -193,7 +215,7 @@ __global__ __launch_bounds__(kBlock) void k_batch_prep(const CircDev *__restrict
     double *pend = cd.scales, *load = pend + np, *slots = load + np + 1;
     for (int p = w; p <= np; p += kWaves) {
         const TPass &tp = p < nf ? t->fwd[p] : p < np ? t->rev[p - nf] : *t->obs;
-        double run = 1.0;
+        Product run;
         for (int o0 = 0; o0 < tp.nops; o0 += 64) {
             const int o = o0 + lane;
             const bool live = o < tp.nops;
@@ -210,50 +232,52 @@ __global__ __launch_bounds__(kBlock) void k_batch_prep(const CircDev *__restrict
                 }
             }
             const bool rot = form == kRX || form == kRY || form == kRotDiag;
-            double incl = rot ? c : 1.0;
+            Product incl;
+            if (rot) incl = Product{c, unit_residual(c, s / c)};
 #pragma unroll
             for (int d = 1; d < 64; d <<= 1) {
-                const double up = __shfl_up(incl, d, 64);
-                if (lane >= d) incl *= up;
+                const Product up{__shfl_up(incl.v, d, 64), __shfl_up(incl.off, d, 64)};
+                if (lane >= d) incl = incl * up;
             }
-            const double prev = __shfl_up(incl, 1, 64);
+            const Product prev{__shfl_up(incl.v, 1, 64), __shfl_up(incl.off, 1, 64)};
             // the products only shrink: the gates above the floor come first
             // (a NaN is not above it)
-            const bool above = fabs(run * incl) >= kScaleFloor;
+            const bool above = fabs(run.v * incl.v) >= kScaleFloor;
             const uint64_t low = __ballot(!above);
-            const int kept = low ? __ffsll((unsigned long long)low) - 1 : 64;
-            const double last = __shfl(incl, kept ? kept - 1 : 0, 64);
-            const double end = kept ? run * last : run;
+            const int kept = low ? __ffsll((unsigned long long)low) - 1 : 64, from = kept ? kept - 1 : 0;
+            const Product last{__shfl(incl.v, from, 64), __shfl(incl.off, from, 64)};
+            const Product end = kept ? run * last : run;
             const bool unit = rot && lane < kept;
             if (live) {
                 if (form != kFixed) set_gate(f, form, c, s, th, unit);
                 cd.fops[tp.op_begin + o] = f;
                 const int slot = int((f.meta >> 8) & 255u) - 1;
                 if (p >= nf && p < np && slot >= 0) {
-                    const double before = lane <= kept ? (lane ? run * prev : run) : end;
-                    slots[tp.slot_begin + slot] = before * before;
+                    const Product before = lane <= kept ? (lane ? run * prev : run) : end;
+                    slots[tp.slot_begin + slot] = (before * before).rounded();
                 }
             }
             run = end;
         }
-        if (p < np && lane == 0) pend[p] = run;
+        if (p < np && lane == 0) pend[p] = run.rounded();
     }
     __syncthreads();
     for (int p = threadIdx.x; p <= np; p += kBlock) {
         // p == np stands for the observable, after the last forward pass
         const int q = p < np ? p : nf, g0 = q / kScaleGroup * kScaleGroup;
-        double base = 1.0, back = 1.0;
-        for (int r = g0; r < q; ++r) base *= pend[r];
+        Product base, back;
+        for (int r = g0; r < q; ++r) base = base * Product{pend[r], 0.0};
         if (q == g0 && q > 0)
-            for (int r = g0 - kScaleGroup; r < g0; ++r) back *= pend[r];
+            for (int r = g0 - kScaleGroup; r < g0; ++r) back = back * Product{pend[r], 0.0};
         if (p == np) { // its state is read as it lies
-            load[np] = base * base * back * back;
+            load[np] = (base * base * back * back).rounded();
             continue;
         }
-        load[p] = back;
+        load[p] = back.rounded();
         if (p >= nf) {
             const TPass &tp = t->rev[p - nf];
-            for (int s = 0; s < tp.nslots; ++s) slots[tp.slot_begin + s] *= base * base;
+            const double square = (base * base).rounded();
+            for (int s = 0; s < tp.nslots; ++s) slots[tp.slot_begin + s] *= square;
         }
     }
 }
