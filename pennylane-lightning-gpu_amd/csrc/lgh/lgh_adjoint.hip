@@ -484,12 +484,22 @@ template <class R> void zsign(lgh_sv *dst, const void *src, uint64_t zmask, hipS
 // scratch that the sweep fills with Z_j psi (inside its first reverse pass
 // where that pass is fused).
 template <class R>
-void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras, int nobs, const lgh_op *ops, int64_t nops,
+void adjoint_t(const lgh_sv *psi_in, lgh_sv *const *bras_in, int nobs, const lgh_op *ops, int64_t nops,
                const int64_t *tp, int64_t ntp, bool apply_ops, double *jac_host, const uint64_t *zmasks) {
     const int n = psi_in->n;
     StreamCtx *ctx = psi_in->ctx;
-    for (int j = 0; j < nobs; ++j)
-        if (bras[j]->ctx != ctx) bras[j]->ctx->sync();
+    // The observable states may belong to other streams: what those still do is
+    // waited for, and the sweep works on them in psi's stream throughout (the
+    // gates that run on their own too), which it waits for before it returns.
+    std::vector<lgh_sv> views;
+    std::vector<lgh_sv *> bras;
+    views.reserve(size_t(nobs));
+    for (int j = 0; j < nobs; ++j) {
+        if (bras_in[j]->ctx != ctx) bras_in[j]->ctx->sync();
+        views.push_back(*bras_in[j]);
+        views.back().ctx = ctx;
+        bras.push_back(&views.back());
+    }
     const bool fused_path = fusion_enabled() && fused_partials_bytes(n, psi_in->device) > 0 && nobs > 0;
     // Working copies of psi, freed once the stream has been waited for.
     struct Buffers {

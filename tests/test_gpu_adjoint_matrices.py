@@ -77,3 +77,26 @@ def test_more_trainable_gates_than_one_store(nobs):
         N.set_fusion(True)
     # 600 gates of some 8 roundings each on two states
     np.testing.assert_allclose(fused, plain, atol=2 * 8 * 600 * 2.3e-16, rtol=0)
+
+
+@pytest.mark.parametrize("fusion", [True, False])
+@pytest.mark.parametrize("n", [8, 14])
+def test_observable_states_of_another_stream(n, fusion):
+    """States that live on another stream than psi: the gates that run on their own stay in order with the sweep."""
+    ops = circuit(n, n + 1)
+    tp = list(range(sum(1 for o in ops if o[2])))
+    stream = N.C.c_void_p()
+    N.check(N.lib().lgh_stream_create(0, N.C.byref(stream)))
+    N.set_fusion(fusion)
+    try:
+        psi = N.State(n).reset().apply(ops)
+        words = [("X", [0]), ("ZY", [1, n - 1])]
+        same = N.adjoint_jacobian(psi, [N.State(n).set_pauli_word_of(psi, *w) for w in words], ops, tp)
+        for _ in range(5):
+            other = [N.State(n, stream=stream).set_pauli_word_of(psi, *w) for w in words]
+            np.testing.assert_array_equal(N.adjoint_jacobian(psi, other, ops, tp), same)
+        del other
+    finally:
+        N.set_fusion(True)
+    N.check(N.lib().lgh_stream_synchronize(stream))
+    N.check(N.lib().lgh_stream_destroy(stream))
