@@ -2161,13 +2161,14 @@ lgh_status lgh_csr_create(lgh_csr **out, int device, lgh_dtype dtype, int64_t nu
         LGH_REQUIRE(out && indptr && (nnz == 0 || (indices && values)), "null pointer");
         LGH_REQUIRE(num_rows >= 1, "CSR matrix needs at least one row");
         LGH_REQUIRE(indptr[0] == 0 && indptr[num_rows] == nnz, "CSR offsets do not match nnz");
-        int64_t shortest = 0, longest = 0;
-        for (int64_t r = 0; r < num_rows; ++r) {
-            const int64_t len = indptr[r + 1] - indptr[r];
-            shortest = std::min(shortest, len);
-            longest = std::max(longest, len);
-        }
-        LGH_REQUIRE(shortest >= 0, "CSR offsets must not decrease");
+        // the longest row; a negative length is the longest of all, unsigned
+        uint64_t len[4] = {};
+        int64_t r = 0;
+        for (; r + 4 <= num_rows; r += 4)
+            for (int q = 0; q < 4; ++q) len[q] = std::max(len[q], uint64_t(indptr[r + q + 1]) - uint64_t(indptr[r + q]));
+        for (; r < num_rows; ++r) len[0] = std::max(len[0], uint64_t(indptr[r + 1]) - uint64_t(indptr[r]));
+        const uint64_t longest = std::max({len[0], len[1], len[2], len[3]});
+        LGH_REQUIRE(longest <= uint64_t(INT64_MAX), "CSR offsets must not decrease");
         for (int64_t k = 0; k < nnz; ++k)
             LGH_REQUIRE(indices[k] >= 0 && indices[k] < num_rows, "CSR column index out of range");
         auto c = std::make_unique<lgh_csr>();
@@ -2176,7 +2177,7 @@ lgh_status lgh_csr_create(lgh_csr **out, int device, lgh_dtype dtype, int64_t nu
         c->rows = num_rows;
         c->nnz = nnz;
         c->avg_row = double(nnz) / double(num_rows);
-        c->longest_row = longest;
+        c->longest_row = int64_t(longest);
         // 32-bit indices where they fit: a sixth of a complex128 matrix's bytes
         c->idx64 = num_rows >= (int64_t(1) << 31) || nnz >= (int64_t(1) << 31);
         DeviceGuard g(device);
