@@ -624,8 +624,8 @@ __device__ __forceinline__ void fused_adj_body(const AdjArrays &one, const AdjAr
 // Three register bits fit three wavefronts per SIMD in the general kernel
 // (at most 168 VGPRs) and four in the lean ones (103-117 VGPRs; 26 KiB of LDS
 // per workgroup).  The complex128
-// lean kernels are held to 96 VGPRs for five wavefronts per SIMD (a few spills,
-// mostly outside the gate loop; measured 1.3 % faster per pass at level 1 and
+// lean kernels are held to 96 VGPRs for five wavefronts per SIMD (7, 17 and 35 spills at
+// levels 1 to 3, mostly outside the gate loop; measured 1.3 % faster per pass at level 1 and
 // 2.2 % at level 2).
 // Lv: lean level of the pass (0: any fusable gate).
 template <class R, int Lv = 0>
@@ -637,7 +637,7 @@ __global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 5 : 3) void k
                              bra_from_lam);
 }
 // Four register bits: the complex128 lean kernels are held to 168 VGPRs for
-// three wavefronts per SIMD (39 dwords spilled to scratch at level 1; 4.50
+// three wavefronts per SIMD (39, 40 and 76 dwords spilled to scratch at levels 1 to 3; 4.50
 // against 4.88 ms per 28-qubit pass at two wavefronts).
 template <class R, int Lv = 0>
 __global__ __launch_bounds__(kBlock, (Lv >= 1 && sizeof(R) == 8) ? 3 : 1) void k_fused_adj4(
@@ -689,7 +689,7 @@ __global__ __launch_bounds__(kBlock) void k_slot_store(const double *__restrict_
 // host form of FOp before its fields are packed into meta
 struct HOp {
     uint32_t kind = 0, gkind = 0, dneg = 0;
-    uint32_t rot = 0; // 1: matrix [[1, -t], [t, 1]], 2: [[t, -1], [1, t]] (a rotation with a factor taken out)
+    uint32_t rot = 0; // 1: matrix [[1, -t], [t, 1]], 2: [[t, -1], [1, t]], 3: [[1, iu], [iu, 1]] (a factor taken out)
     int loc = 0, slot = -1;
     uint64_t cm_reg = 0, pm_reg = 0; // control / parity bits among the register bits
     FOp f{};

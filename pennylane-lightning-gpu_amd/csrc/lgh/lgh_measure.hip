@@ -233,7 +233,7 @@ __global__ __launch_bounds__(kBlock) void k_expval_reg(const cx<R> *__restrict__
 // FMAs more.  64 KiB of LDS: two workgroups of eight wavefronts per CU.
 // Bound by the state reads, one per launch.  24 qubits, 256 words,
 // complex128: 3712 us in 16 launches with tiles of 2^11 and an LDS read per
-// word and amplitude, 1091 us in 11 launches here.
+// word and amplitude, 1091 us in 13 launches here.
 constexpr int kPTileBits = 12;       // amplitudes per tile: 2^12
 constexpr int kPFixedBits = 3;       // lowest index bits in every tile
 constexpr int kPBlock = 512;
@@ -561,7 +561,7 @@ template <class R> __global__ __launch_bounds__(kBlock) void k_zero(cx<R> *__res
 // workgroup's rows fill about one step.
 // Bound by reading the matrix (70 us of the 89 it takes at the first of these
 // sizes).  <H> of the 21-entry rows of a transverse-field Ising chain on 20
-// qubits, call to call: 150 -> 103 us in complex128 (32-bit indices; with 64
+// qubits, call to call: 150 -> 100 us in complex128 (32-bit indices; with 64
 // the matrix has 528 MB for 440), 119 -> 82 in complex64, against 16 lanes
 // per row, whose loads of x took a cache line per lane and whose second round
 // had 5 of 16 lanes at work.
