@@ -1432,13 +1432,13 @@ void AdjPasses::run_t(const AdjSweep *sweeps, int count, double *partials, void 
         if (it->standalone) {
             close(); // before what the gate uploads
             const int i = it->ops[0];
-            if (pairs_pay(udag_[size_t(i)], n_, dtype_, true)) {
+            if (pairs_pay(udag_[size_t(i)], n_, dtype_, true, slot_col_[size_t(i)] >= 0)) {
                 // a run's partial sums, a row of one double per workgroup for
                 // every trainable gate, fit the partials
                 size_t room = stride;
                 for (auto next = it; next != passes_->rend() && next->standalone; ++next) {
                     const size_t g = size_t(next->ops[0]);
-                    if (!pairs_pay(udag_[g], n_, dtype_, true)) break;
+                    if (!pairs_pay(udag_[g], n_, dtype_, true, slot_col_[g] >= 0)) break;
                     if (slot_col_[g] >= 0) {
                         const unsigned blocks = adj_pairs_blocks(n_, udag_[g]);
                         if (blocks > room || (st.blocks && blocks != st.blocks)) break;

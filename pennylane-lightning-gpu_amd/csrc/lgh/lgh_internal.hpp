@@ -379,11 +379,11 @@ struct KOp {
 //   128 MiB, runs shorter than 128 bytes 1.00-1.05 above;
 //  one pair, adjoint: 0.59-0.93 in complex128, whole lines 0.60-0.94 and both
 //   bits inside a line 0.71-0.98 in complex64, one inside 0.77-0.98 below 32 MiB,
-//   1.05-1.17 from there;
+//   there 0.95-0.98 with a generator and 1.05-1.07 without, 1.08-1.17 above;
 //  two pairs, adjoint: runs of 128 bytes 0.68-1.03, shorter ones 0.67-0.98 below
 //   32 MiB, up to 1.56 from there.
 // Four targets (a double excitation: an eighth of the state) always pay.
-inline bool pairs_pay(const KOp &op, int n, lgh_dtype dtype, bool adjoint) {
+inline bool pairs_pay(const KOp &op, int n, lgh_dtype dtype, bool adjoint, bool trained = false) {
     if (op.npair == 0) return false;
     if (op.k != 2) return true;
     const bool single = dtype == LGH_C64;
@@ -391,7 +391,7 @@ inline bool pairs_pay(const KOp &op, int n, lgh_dtype dtype, bool adjoint) {
     const size_t low = amp << std::min(op.tbits[0], op.tbits[1]), high = amp << std::max(op.tbits[0], op.tbits[1]);
     if (op.npair == 2) return low >= 128 || (adjoint ? state < 32 * MiB : !single || state < 256 * MiB);
     if (low >= 64) return true;
-    if (adjoint) return !single || high < 64 || state < 32 * MiB;
+    if (adjoint) return !single || high < 64 || state < (trained ? 64 : 32) * MiB;
     return single ? state < 64 * MiB : high < 64 || state < 512 * MiB;
 }
 
