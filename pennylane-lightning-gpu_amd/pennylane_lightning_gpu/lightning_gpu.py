@@ -175,34 +175,36 @@ class LightningGPU:
         gates gets them together and applies them in fused passes."""
         sequence = getattr(self._gpu_state, "applySequence", None)
         pending, held = [], 0
-        for o in operations:
-            if o.name == "Identity":
-                continue
-            invert = hasattr(o, "base")
-            name = o.base.name if invert else o.name
-            method = getattr(self._gpu_state, name, None)
-            wires = self.map_wires(o.wires)
-            mat, params = _NO_MATRIX, []
-            if method is None:
-                invert = False
-                mat = np.asarray(o.matrix(), dtype=self.C_DTYPE)  # already holds the adjoint
-                if mat.size == 0:
-                    raise DeviceError("Unsupported operation")
-                mat = mat.ravel(order="C")
-            elif o.parameters:
-                params = [float(p) for p in np.ravel(o.parameters)]
-            if sequence is not None:
-                pending.append((name, wires, invert, params, mat))
-                held += mat.nbytes
-                if len(pending) == _SEQUENCE_MAX or held >= _SEQUENCE_MATRIX_BYTES:
-                    sequence(*zip(*pending))
-                    pending, held = [], 0
-            elif method is None:
-                self._gpu_state.apply(name, wires, False, [], mat)
-            else:
-                method(wires, invert, params)
-        if pending:
-            sequence(*zip(*pending))
+        try:
+            for o in operations:
+                if o.name == "Identity":
+                    continue
+                invert = hasattr(o, "base")
+                name = o.base.name if invert else o.name
+                method = getattr(self._gpu_state, name, None)
+                wires = self.map_wires(o.wires)
+                mat, params = _NO_MATRIX, []
+                if method is None:
+                    invert = False
+                    mat = np.asarray(o.matrix(), dtype=self.C_DTYPE)  # already holds the adjoint
+                    if mat.size == 0:
+                        raise DeviceError("Unsupported operation")
+                    mat = mat.ravel(order="C")
+                elif o.parameters:
+                    params = [float(p) for p in np.ravel(o.parameters)]
+                if sequence is not None:
+                    pending.append((name, wires, invert, params, mat))
+                    held += mat.nbytes
+                    if len(pending) == _SEQUENCE_MAX or held >= _SEQUENCE_MATRIX_BYTES:
+                        ready, pending, held = pending, [], 0
+                        sequence(*zip(*ready))
+                elif method is None:
+                    self._gpu_state.apply(name, wires, False, [], mat)
+                else:
+                    method(wires, invert, params)
+        finally:  # the gates before one that is refused are applied, as one by one
+            if pending:
+                sequence(*zip(*pending))
 
     def apply(self, operations, **kwargs):
         """lightning_gpu.py:557-575."""

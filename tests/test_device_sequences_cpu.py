@@ -37,3 +37,12 @@ def test_matrices_held_at_once_are_bounded(ks):
         assert sum(m.nbytes for m in mats) < lg._SEQUENCE_MATRIX_BYTES + largest
     assert [n for c in seqs for n in c[1]] == [o.name for o in ops]
     assert [p for c in seqs for p in c[4]] == [[float(x) for x in o.parameters] if o.name == "RX" else [] for o in ops]
+
+
+def test_gates_before_a_refused_one_are_applied():
+    dev = lg.LightningGPU(3, _backend=SequenceBackend)
+    bad = qc.Operation("QubitUnitary", [0], [], matrix=np.zeros((0, 0)))
+    with pytest.raises(Exception):
+        dev.apply_cq([qc.Operation("PauliX", [0]), qc.Operation("RY", [1], [0.5]), bad, qc.Operation("PauliZ", [2])])
+    seqs = [c for c in dev._gpu_state.calls if c[0] == "applySequence"]
+    assert [n for c in seqs for n in c[1]] == ["PauliX", "RY"]
